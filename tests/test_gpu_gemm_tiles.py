@@ -1,0 +1,48 @@
+"""The many-token GEMM (tcq_gemm_i8, tcq_gemm_bf16) at the edges of its tiles: sizes that select each tile, with remainders in
+tokens, weight rows and K (whole and partial 128-byte steps, fewer steps than the rings hold)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = 'cuda'
+
+# 64 x 64, 128 x 64, 128 x 128, 256 x 128 and 256 x 256 tiles (the last line of each pair with remainders)
+SIZES = [(65, 64, 16), (129, 1156, 1168), (65, 12800, 128), (80, 16388, 272), (200, 16384, 384), (449, 8196, 144), (400, 16384, 256),
+         (385, 16420, 400), (768, 16384, 512), (801, 16516, 656), (1, 132, 32), (66, 16640, 2048)]
+
+
+def _ints(*shape, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return torch.randint(-127, 128, shape, generator=g, device=DEV, dtype=torch.int8)
+
+
+@pytest.mark.parametrize('M,N,K', SIZES)
+def test_int8_tiles_bitexact(M, N, K):
+    from yanlongvla_amd import kernels as Kn
+    a, w = _ints(M, K, seed=1), _ints(N, K, seed=2)
+    sa = torch.rand(M, device=DEV) + 0.01
+    sw = torch.rand(N, device=DEV) + 0.01
+    want = (a.double() @ w.double().t()).to(torch.int32)                       # exact: |sum| < 2^53
+    pad = torch.full((M, N + 8), 7, dtype=torch.int32, device=DEV)
+    acc = Kn.gemm_i8(a, w, pad[:, :N])
+    assert torch.equal(acc, want) and bool((pad[:, N:] == 7).all())            # a wider row stride, nothing past the columns
+    z = (want.float() * sa[:, None]) * sw[None, :]
+    assert torch.equal(Kn.gemm_i8(a, w, torch.empty(M, N, device=DEV), sa=sa, sw=sw), z)
+    y = torch.full((M, N + 4), 3.0, dtype=torch.bfloat16, device=DEV)
+    assert torch.equal(Kn.gemm_i8(a, w, y[:, :N], sa=sa, sw=sw), z.bfloat16()) and bool((y[:, N:] == 3.0).all())
+
+
+@pytest.mark.parametrize('M,N,K', SIZES)
+def test_bf16_tiles_against_fp64(M, N, K):
+    """Products of BF16 values are exact in FP32; every sum of K of them in FP32, in whatever order, is within K 2^-24 of the
+    sum of their magnitudes."""
+    from yanlongvla_amd import kernels as Kn
+    g = torch.Generator(device=DEV).manual_seed(3)
+    a, w = torch.randn(M, K, generator=g, device=DEV).bfloat16(), _ints(N, K, seed=4).bfloat16()
+    want, mag = a.double() @ w.double().t(), a.double().abs() @ w.double().abs().t()
+    z = Kn.gemm_bf16(a, w, torch.empty(M, N, device=DEV))
+    assert bool(((z.double() - want).abs() <= K * 2.0 ** -24 * mag).all())
+    sw = torch.rand(N, device=DEV) + 0.01
+    assert torch.equal(Kn.gemm_bf16(a, w, torch.empty(M, N, device=DEV), sw=sw), z * sw)
+    assert torch.equal(Kn.gemm_bf16(a, w, torch.empty(M, N, dtype=torch.bfloat16, device=DEV)), z.bfloat16())

@@ -1,38 +1,48 @@
-// GEMM for many tokens, acc[m, n] = sum_k a[m, k] w[n, k], a (M, K) and w (N, K) both row-major with K contiguous, so every
+// GEMM for many tokens, acc[m, n] = sum_k x[m, k] w[n, k], x (M, K) and w (N, K) both row-major with K contiguous, so every
 // MFMA operand is 16 consecutive bytes of one row:
-//   INT8 (W8A8) on v_mfma_i32_32x32x32_i8 (measured on MI355X: 4.05 POPS for back-to-back independent 32 x 32 x 32 products
-//   against 2.7 for 16 x 16 x 64): exact int32 acc, written as int32, as FP32 (float(acc) * sa[m]) * sw[n], or as BF16 of
-//   that;
-//   BF16 (the W2 float path: BF16 rotated activations times the INT8 table values as BF16) on v_mfma_f32_32x32x16_bf16 with
+//   INT8 (W8A8) on v_mfma_i32_16x16x64_i8: exact int32 acc, written as int32 (optionally in K parts), as FP32
+//   (float(acc) * sa[m]) * sw[n], or as BF16 of that;
+//   BF16 (the W2 float path: BF16 rotated activations times the INT8 table values as BF16) on v_mfma_f32_16x16x32_bf16 with
 //   FP32 accumulation, written as FP32 (acc * sa[m]) * sw[n] (either scale may be absent) or as BF16 of that.
-// Both take 64-byte K steps: 64 int8 = two 32-element MFMA halves, or 32 bf16 = two 16-element MFMA steps, with the same
-// 16-byte fragment per lane.
+// 16 x 16 blocks although 32 x 32 ones issue at a higher peak: on random operands the part holds 2.23 GHz through
+// 16x16x64 (3.95 POP/s) but drops to 1.78 GHz through 32x32x32 (3.53 POP/s), and the rest of the loop runs at that clock
+// too (BF16: 1.92 against 1.85 PFLOP/s).
 //
-// Workgroup tile TN weights x TM tokens, WN x WM waves, each (TN / WN) x (TM / WM) in 32 x 32 MFMA blocks. MFMA A = 32
-// token rows (lane (h, r): row r, 16 columns of half h of the 32), B = 32 weight rows, D: register 4 q + e of lane (h, c)
-// holds token 8 q + 4 h + e of weight c, so the 32 lanes of a half store 32 consecutive output columns.
-// K steps of 64 bytes go HBM -> LDS by buffer_load_dwordx4 ... lds (no registers), NS steps in flight: the loads of step
-// kt + NS - 1 are issued right after the barrier that opens step kt. A step holds 1 KiB blocks of 16 rows x 64 bytes; lane
-// p of a load writes position p of its block, which holds row p / 4 and 16-byte granule (p % 4) ^ ((row / 4) % 4), so the
-// 16 rows of a fragment read hit 16 different bank groups. Rows past M / N and columns past K read zeros.
+// Workgroup tile TN weights x TM tokens, WN x WM waves. MFMA A = 16 weight rows, B = 16 token rows, 64 bytes of K each; D:
+// register e of lane (g, c) holds weight 4 g + e of token c, so a lane stores 4 consecutive columns (16 bytes of FP32 /
+// int32) straight from its registers; for BF16 outputs the weight rows of two blocks are interleaved so that it is 8.
+//
+// K goes by in steps of 128 bytes, whole cache lines of both operands (64-byte steps fetch every line twice: 42.3 against
+// 37.1 us at 800 x 2048 x 16384), HBM -> LDS by buffer_load_dwordx4 ... lds without registers, into two rings: NSX steps of
+// activations, NSW of weights. Weights come from HBM and activations from the caches, so the 160 KiB of a 256 x 256 tile
+// hold three steps of weights and two of activations. A load fills 8 rows x 128 bytes; lane p writes position p, which holds
+// row p / 8 and 16-byte granule (p % 8) ^ f(row), f = the row's low three bits with bit 3 folded in, so that the rows of a
+// fragment read (consecutive, or interleaved for BF16 outputs) fall into different banks.
+// A step runs in four quarters (k half x half of the wave's weight blocks); the fragment reads of the next quarter and the
+// loads of later steps are scheduled between the MFMAs of this one. The one barrier of a step stands before its last
+// quarter, whose fragments are in registers by then: it publishes the next step and frees this one, with MFMAs on both sides.
+// Rows past M / N and columns past K read zeros; waves whose tokens are all padding only load.
+// What bounds it (256 x 256, INT8, K long enough): 1.5 us per step, 2.8 POP/s; the MFMAs alone take 1.05 us, the loads and
+// fragment reads alone 0.7 (in cache) to 1.2 us (streaming): LDS cycles (fragment reads 1536 + loads 512 against 2048 MFMA
+// cycles per step) and power. One wave per SIMD with 128 x 128 each (a third fewer fragment reads) measured the same.
 #include "tcq_device.h"
 #include "tcq_launch.h"
 
 namespace {
 
 typedef int int4v __attribute__((ext_vector_type(4)));
-typedef int int16v __attribute__((ext_vector_type(16)));
+typedef float float4v __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-__device__ __forceinline__ int swz(int row, int g) { return row * 64 + 16 * (g ^ ((row >> 2) & 3)); }
-
-// s_waitcnt vmcnt(n) with the other counters left alone (gfx9 encoding: vmcnt bits 3:0 and 15:14)
-template <int n>
-__device__ __forceinline__ void wait_vm() {
-    __builtin_amdgcn_s_waitcnt((n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8));
+// s_waitcnt vmcnt(vm) lgkmcnt(lgkm), expcnt left alone (gfx9 encoding: vmcnt bits 3:0 and 15:14; lgkm 15 = no wait)
+template <int vm, int lgkm>
+__device__ __forceinline__ void wait_cnt() {
+    static_assert(vm <= 63 && lgkm <= 15, "counter range");
+    __builtin_amdgcn_s_waitcnt((vm & 15) | ((vm >> 4) << 14) | (7 << 4) | (lgkm << 8));
 }
 
 // Workgroup barrier without the memory fence of __syncthreads (which waits for every outstanding load, including the LDS
-// loads of later steps): the LDS writes a barrier must publish are the loads waited for just before it (wait_vm), and the
+// loads of later steps): the LDS writes a barrier must publish are the loads waited for just before it (wait_cnt), and the
 // empty asm statements keep the compiler from moving memory accesses across it.
 __device__ __forceinline__ void barrier_nofence() {
     asm volatile("" ::: "memory");
@@ -40,179 +50,255 @@ __device__ __forceinline__ void barrier_nofence() {
     asm volatile("" ::: "memory");
 }
 
-}  // namespace
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float float16v __attribute__((ext_vector_type(16)));
-
 template <int ESZ> struct MfmaOf;
 template <> struct MfmaOf<1> {                 // INT8
-    typedef int16v acc_t;
-    static __device__ __forceinline__ acc_t mma(int4v a, int4v b, acc_t c) { return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0); }
+    typedef int4v acc_t;
+    static __device__ __forceinline__ acc_t mma(int4v a, int4v b, acc_t c) { return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0); }
 };
 template <> struct MfmaOf<2> {                 // BF16
-    typedef float16v acc_t;
+    typedef float4v acc_t;
     static __device__ __forceinline__ acc_t mma(int4v a, int4v b, acc_t c) {
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
     }
 };
 
-// ESZ: element size (1 INT8, 2 BF16); K in elements. WAUX: cache policy of the weight loads, non-temporal (2) when a single
-// tile row of tokens reads every weight once, temporal (0) when several token tiles reread them (measured at M = 800,
-// N = 16384, K = 2048: 40.6 against 46.3 us per launch; the four token tiles of a weight tile run on one XCD and share its L2).
-template <int ESZ, int TN, int TM, int WN, int WM, int NS, int ODT, int WAUX = 2>
-__global__ __launch_bounds__(64 * WN * WM) void k_gemm_i8(const void* a_, const void* w_, const float* sa, const float* sw, void* out,
-                                                          int ldo, int M, int N, int K_) {
+template <int n> struct Num { static constexpr int value = n; };
+struct Full { static constexpr bool value = true; };
+struct Tail { static constexpr bool value = false; };
+
+}  // namespace
+
+// ESZ: element size (1 INT8, 2 BF16); K in elements. parts: K parts (grid.z, int32 outputs): part z sums the steps
+// [z ceil(nk / parts), ...) into out + z M ldo.
+template <int ESZ, int TN, int TM, int WN, int WM, int NSW, int NSX, int ODT>
+__global__ __launch_bounds__(64 * WN * WM) void k_gemm_i8(const void* x_, const void* w_, const float* sa, const float* sw, void* out,
+                                                       int ldo, int M, int N, int K_, int parts) {
     typedef typename MfmaOf<ESZ>::acc_t acc_t;
-    const char* a = (const char*)a_;
-    const char* w = (const char*)w_;
-    const int K = K_ * ESZ;                                              // row length in bytes
     constexpr int NWAVE = WN * WM;
-    constexpr int WBLK = TN / 16, ABLK = TM / 16, BLK = WBLK + ABLK;    // 1 KiB blocks (16 rows x 64 bytes) per step
-    constexpr int PW = BLK / NWAVE;                                      // direct loads per wave per step
-    constexpr int BN = TN / WN / 32, BM = TM / WM / 32;                  // 32 x 32 MFMA blocks per wave
-    static_assert(BLK % NWAVE == 0 && TN % (32 * WN) == 0 && TM % (32 * WM) == 0, "tile shape");
-    __shared__ __attribute__((aligned(1024))) char lds[NS][BLK * 1024];
+    constexpr int WL = TN / 8 / NWAVE, XL = TM / 8 / NWAVE;              // 1 KiB loads (8 rows x 128 bytes) per wave and step
+    constexpr int NB = TN / WN / 16, MB = TM / WM / 16, HB = NB / 2;     // 16 x 16 blocks per wave; weight blocks per quarter
+    static_assert(WL * 8 * NWAVE == TN && XL * 8 * NWAVE == TM && HB * 2 == NB && MB * 16 * WM == TM, "tile shape");
+    const int K = K_ * ESZ;                                              // row length in bytes
+    extern __shared__ __attribute__((aligned(1024))) char lds[];
+    char* ldsw = lds;
+    char* ldsx = lds + NSW * TN * 128;
     const int n0 = blockIdx.x * TN, m0 = blockIdx.y * TM;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int wn = wave % WN, wm = wave / WN;
-    const int l32 = lane & 31, lh = lane >> 5;                           // MFMA operand lane: row l32, k-half lh
-    const rsrc_t RA = make_rsrc(a, (u32)M * (u32)K), RW = make_rsrc(w, (u32)N * (u32)K);
-    const int nk = (K + 63) >> 6;
-    const int prow = lane >> 2, pg = (lane & 3) ^ ((prow >> 2) & 3);  // what this lane loads in a block
+    const int lr = lane & 15, lg = lane >> 4;
+    const rsrc_t RX = make_rsrc(x_, (u32)M * (u32)K), RW = make_rsrc(w_, (u32)N * (u32)K);
+    const int nkall = (K + 127) >> 7, per = (nkall + parts - 1) / parts, kb = blockIdx.z * per;
+    const int nk = min(per, nkall - kb), kend = min(K, 128 * (kb + nk));
 
-    auto issue = [&](int kt) {
-        char* st = lds[kt % NS];
-        const int k = 64 * kt + 16 * pg;
+    // load u of a wave fills block (wave * L + u) of 8 rows: lane p writes position p, which holds row p / 8, slot p % 8
+    const int prow = lane >> 3;
+    u32 offw[WL], offx[XL];
 #pragma unroll
-        for (int u = 0; u < PW; ++u) {
-            const int blk = wave * PW + u;
-            char* dst = st + blk * 1024;
-            if (blk < WBLK) {
-                const int row = n0 + 16 * blk + prow;
-                const u32 off = (row < N && k < K) ? (u32)row * (u32)K + (u32)k : RSRC_OOB;
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(RW, (__attribute__((address_space(3))) void*)dst, 16, off, 0, 0, WAUX);
-            } else {
-                const int row = m0 + 16 * (blk - WBLK) + prow;
-                const u32 off = (row < M && k < K) ? (u32)row * (u32)K + (u32)k : RSRC_OOB;
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(RA, (__attribute__((address_space(3))) void*)dst, 16, off, 0, 0, 0);
+    for (int u = 0; u < WL; ++u) {
+        const int blk = wave * WL + u, row = n0 + 8 * blk + prow, g = (lane & 7) ^ prow ^ ((blk & 1) << 2);
+        offw[u] = row < N ? (u32)row * (u32)K + 16u * g : RSRC_OOB;
+    }
+#pragma unroll
+    for (int u = 0; u < XL; ++u) {
+        const int blk = wave * XL + u, row = m0 + 8 * blk + prow, g = (lane & 7) ^ prow ^ ((blk & 1) << 2);
+        offx[u] = row < M ? (u32)row * (u32)K + 16u * g : RSRC_OOB;
+    }
+    // loads of K step kt: the row offsets stay in registers, the step is the scalar offset; only the last, partial step of K (and
+    // the loads past the end, which read zeros) select per lane
+    const int nfull = (kend - 128 * kb) >> 7;
+    auto issue_w = [&](int kt, auto full) {
+        char* st = ldsw + (kt % NSW) * (TN * 128) + wave * WL * 1024;
+        const int k = 128 * (kb + kt);
+        if constexpr (decltype(full)::value) {
+#pragma unroll
+            for (int u = 0; u < WL; ++u) {
+                char* dst = st + u * 1024;
+                const u32 off = offw[u];
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(RW, (__attribute__((address_space(3))) void*)dst, 16, off, k, 0, 0);
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < WL; ++u) {
+                char* dst = st + u * 1024;
+                const int g = (lane & 7) ^ prow ^ (((wave * WL + u) & 1) << 2);
+                const u32 off = (k + 16 * g < kend) ? offw[u] + (u32)k : RSRC_OOB;
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(RW, (__attribute__((address_space(3))) void*)dst, 16, off, 0, 0, 0);
             }
         }
     };
-    // fragment of 32 rows starting at 16-row block b0, k half kk (columns 32 kk .. 32 kk + 31 of the step)
-    auto frag = [&](const char* st, int b0, int kk) {
-        return *(const int4v*)(st + (b0 + (l32 >> 4)) * 1024 + swz(l32 & 15, 2 * kk + lh));
-    };
-
-    acc_t acc[BN][BM];
+    auto issue_x = [&](int kt, auto full) {
+        char* st = ldsx + (kt % NSX) * (TM * 128) + wave * XL * 1024;
+        const int k = 128 * (kb + kt);
+        if constexpr (decltype(full)::value) {
 #pragma unroll
-    for (int i = 0; i < BN; ++i)
+            for (int u = 0; u < XL; ++u) {
+                char* dst = st + u * 1024;
+                const u32 off = offx[u];
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(RX, (__attribute__((address_space(3))) void*)dst, 16, off, k, 0, 0);
+            }
+        } else {
 #pragma unroll
-        for (int j = 0; j < BM; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0;
-
-#pragma unroll
-    for (int t = 0; t < NS - 1; ++t)
-        if (t < nk) issue(t);
-    for (int kt = 0; kt < nk; ++kt) {
-        if (kt + NS - 2 < nk) wait_vm<(NS - 2) * PW>();                 // this wave's loads of step kt have landed
-        else wait_vm<0>();
-        barrier_nofence();                                               // ... and every other wave's
-        if (kt + NS - 1 < nk) issue(kt + NS - 1);                        // into the buffer of step kt - 1 (all done with it)
-        const char* st = lds[kt % NS];
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-            int4v A[BM], B[BN];
-#pragma unroll
-            for (int j = 0; j < BM; ++j) A[j] = frag(st, WBLK + (wm * BM + j) * 2, kk);
-#pragma unroll
-            for (int i = 0; i < BN; ++i) B[i] = frag(st, (wn * BN + i) * 2, kk);
-#pragma unroll
-            for (int j = 0; j < BM; ++j)
-                // blocks of padding rows only: no MFMA work (with one wave row, where a tile always holds rows, the test is
-                // left out: the branch changed the code of the narrow tiles and slowed them)
-                if (WM == 1 || m0 + (wm * BM + j) * 32 < M)
-#pragma unroll
-                    for (int i = 0; i < BN; ++i) acc[i][j] = MfmaOf<ESZ>::mma(A[j], B[i], acc[i][j]);
+            for (int u = 0; u < XL; ++u) {
+                char* dst = st + u * 1024;
+                const int g = (lane & 7) ^ prow ^ (((wave * XL + u) & 1) << 2);
+                const u32 off = (k + 16 * g < kend) ? offx[u] + (u32)k : RSRC_OOB;
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(RX, (__attribute__((address_space(3))) void*)dst, 16, off, 0, 0, 0);
+            }
         }
+    };
+    constexpr int FLY0 = WL * (NSW - 2) + XL * (NSX - 1), FLY = WL * (NSW - 2) + XL * (NSX - 2);
+    // stages 0 .. NSX - 1 of the activations and 0 .. NSW - 2 of the weights, in the order of the loop's own loads: the waits
+    // count the loads issued after the stage they wait for
+    constexpr int NS = NSX > NSW ? NSX : NSW;
+#pragma unroll
+    for (int t = 1 - NS; t <= 0; ++t) {
+        if (t - 1 + NSX >= 0) issue_x(t - 1 + NSX, Tail{});
+        if (t - 1 + NSW >= 0 && t < 0) issue_w(t - 1 + NSW, Tail{});
     }
 
-    // epilogue: block (i, j), register 4 q + e of lane (lh, l32) = token m0 + (wm BM + j) 32 + 8 q + 4 lh + e, weight
-    // n0 + (wn BN + i) 32 + l32.
-    if constexpr (ODT == TCQ_I32) {
-        // the 32 lanes of a half store 32 consecutive int32 columns: whole 128-byte lines
+    if (m0 + wm * (TM / WM) >= M) {                 // this wave's tokens are padding: only its share of the loads
+        wait_cnt<FLY0, 15>();
+        barrier_nofence();
+        for (int kt = 0; kt < nk; ++kt) {
+            issue_w(kt + NSW - 1, Tail{});
+            wait_cnt<FLY, 15>();
+            barrier_nofence();
+            issue_x(kt + NSX, Tail{});
+        }
+        wait_cnt<0, 15>();                          // no load into the LDS outlives the workgroup
+        return;
+    }
+
+    // weight row of A row r of block i: BF16 outputs pair the blocks so that a lane ends with 8 consecutive columns
+    constexpr bool PAIR = ODT == TCQ_BF16;
+    auto wrow = [&](int i) { return PAIR ? 32 * (i >> 1) + 8 * (lr >> 2) + 4 * (i & 1) + (lr & 3) : 16 * i + lr; };
+    auto slot = [&](int row, int g) { return row * 128 + 16 * (g ^ (row & 7) ^ (((row >> 3) & 1) << 2)); };
+    // rows 32 apart share their slot pattern: two (PAIR) or one base offsets per k half, the rest constants
+    int fw[2][2], fx[2];
 #pragma unroll
-        for (int j = 0; j < BM; ++j) {
-            const int mb = m0 + (wm * BM + j) * 32 + 4 * lh;
+    for (int h = 0; h < 2; ++h) {
+        fw[h][0] = slot(wrow(0), 4 * h + lg);
+        fw[h][1] = slot(wrow(1), 4 * h + lg);
+        fx[h] = slot(lr, 4 * h + lg);
+    }
+    acc_t acc[NB][MB];
 #pragma unroll
-            for (int i = 0; i < BN; ++i) {
-                const int n = n0 + (wn * BN + i) * 32 + l32;
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int j = 0; j < MB; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[i][j][e] = 0;
+    int4v A[2][HB], B[2][MB];
+    auto read_a = [&](int kt, int h, int half, int s) {                  // weight blocks half * HB .. of k half h
+        const char* p = ldsw + (kt % NSW) * (TN * 128) + wn * NB * 2048;
+#pragma unroll
+        for (int i = 0; i < HB; ++i) {
+            const int b = half * HB + i;
+            A[s][i] = *(const int4v*)(p + (b >> 1) * 4096 + fw[h][b & 1]);
+        }
+    };
+    auto read_b = [&](int kt, int h, int s) {
+        const char* p = ldsx + (kt % NSX) * (TM * 128) + wm * MB * 2048 + fx[h];
+#pragma unroll
+        for (int j = 0; j < MB; ++j) B[s][j] = *(const int4v*)(p + j * 2048);
+    };
+    auto mm = [&](int half, int s, int sb) {
+#pragma unroll
+        for (int i = 0; i < HB; ++i)
+#pragma unroll
+            for (int j = 0; j < MB; ++j) acc[half * HB + i][j] = MfmaOf<ESZ>::mma(A[s][i], B[sb][j], acc[half * HB + i][j]);
+    };
+    // the fragment reads and the loads of a quarter step between its MFMAs
+    auto spread = [&](auto reads, auto loads) {
+        constexpr int R = decltype(reads)::value, L = decltype(loads)::value, NM = HB * MB, G = NM / (R + L) > 0 ? NM / (R + L) : 1;
+#pragma unroll
+        for (int q = 0; q < R + L; ++q) {
+            __builtin_amdgcn_sched_group_barrier(0x008, G, 0);
+            if (q < R) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            else __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    wait_cnt<FLY0, 15>();
+    barrier_nofence();
+    read_b(0, 0, 0);
+    read_a(0, 0, 0, 0);
+    auto step = [&](int kt, auto full) {
+        issue_w(kt + NSW - 1, full);
+        read_a(kt, 0, 1, 1);
+        mm(0, 0, 0);
+        spread(Num<HB>{}, Num<WL>{});
+        read_b(kt, 1, 1);
+        read_a(kt, 1, 0, 0);
+        mm(1, 1, 0);
+        spread(Num<HB + MB>{}, Num<0>{});
+        read_a(kt, 1, 1, 1);
+        mm(0, 0, 1);
+        spread(Num<HB>{}, Num<0>{});
+        wait_cnt<FLY, 0>();
+        barrier_nofence();
+        issue_x(kt + NSX, full);
+        read_b(kt + 1, 0, 0);
+        read_a(kt + 1, 0, 0, 0);
+        mm(1, 1, 1);
+        spread(Num<HB + MB>{}, Num<XL>{});
+    };
+    int kt = 0;
+    for (; kt + NS < nfull; ++kt) step(kt, Full{});
+    for (; kt < nk; ++kt) step(kt, Tail{});
+    wait_cnt<0, 0>();                               // no load into the LDS outlives the workgroup
+    // D: register e of lane (g, c) = weight row 4 g + e of the A block, token c of the B block
+    const int z = blockIdx.z;
+#pragma unroll
+    for (int j = 0; j < MB; ++j) {
+        const int m = m0 + (wm * MB + j) * 16 + lr;
+        if (m >= M) continue;
+        const float s = (ODT != TCQ_I32 && sa) ? gptr(sa)[m] : 1.f;
+        if constexpr (PAIR) {
+#pragma unroll
+            for (int i = 0; i < NB; i += 2) {
+                const int n = n0 + wn * NB * 16 + 16 * i + 8 * lg;
                 if (n >= N) continue;
+                float v[8];
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int m = mb + 8 * (r >> 2) + (r & 3);
-                    if (m < M) gptr((int*)out)[(size_t)m * ldo + n] = (int)acc[i][j][r];
-                }
-            }
-        }
-    } else {
-        // FP32 / BF16: each wave stages one 32-token block row of its tile at a time in its own slice of the (now idle) LDS
-        // ring, row-major, and stores it back as 16-byte pieces of whole row segments (2-byte scattered stores of BF16
-        // leave half lines and run at a fraction of the bandwidth).
-        constexpr int OSZ = ODT == TCQ_BF16 ? 2 : 4;
-        constexpr int WTN = TN / WN, RB = WTN * OSZ, GPR = RB / 16, EPG = 16 / OSZ;
-        constexpr int SLICE = NS * BLK * 1024 / NWAVE;
-        static_assert(32 * RB <= SLICE, "epilogue staging slice");
-        __syncthreads();                                                 // every wave is done with the ring
-        char* slice = &lds[0][0] + wave * SLICE;
-        const int nw0 = n0 + wn * WTN;
-        const bool vec = ((size_t)ldo * OSZ) % 16 == 0 && ((uintptr_t)out % 16) == 0;
-        float swv[BN];
+                for (int b = 0; b < 2; ++b) {
+                    float4v r = {1.f, 1.f, 1.f, 1.f};
+                    if (sw && n + 4 * b < N) r = gptr((const float4v*)(sw + n))[b];      // N is a multiple of 4
 #pragma unroll
-        for (int i = 0; i < BN; ++i) {
-            const int n = nw0 + i * 32 + l32;
-            swv[i] = (sw && n < N) ? gptr(sw)[n] : 1.f;
-        }
-#pragma unroll
-        for (int j = 0; j < BM; ++j) {
-            const int mb = m0 + (wm * BM + j) * 32;
-            float sam[16];
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int m = mb + 8 * (r >> 2) + 4 * lh + (r & 3);
-                sam[r] = (sa && m < M) ? gptr(sa)[m] : 1.f;
-            }
-#pragma unroll
-            for (int i = 0; i < BN; ++i)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int tr = 8 * (r >> 2) + 4 * lh + (r & 3);
-                    const float v = ESZ == 1 ? ((float)acc[i][j][r] * sam[r]) * swv[i]
-                                             : (sa ? (float)acc[i][j][r] * sam[r] : (float)acc[i][j][r]) * (sw ? swv[i] : 1.f);
-                    char* dst = slice + tr * RB + (i * 32 + l32) * OSZ;
-                    if (ODT == TCQ_F32) *(float*)dst = v;
-                    else *(u16*)dst = f32_to_bf16(v);
-                }
-            constexpr int NG = (32 * GPR + 63) / 64;                     // 16-byte pieces per lane (a fixed count: unrolled)
-#pragma unroll
-            for (int it = 0; it < NG; ++it) {
-                const int g = lane + 64 * it;
-                const int tr = g / GPR, cg = g - tr * GPR;
-                const int m = mb + tr, n = nw0 + cg * EPG;
-                if (g >= 32 * GPR || m >= M || n >= N) continue;
-                const uint4_t v = *(const uint4_t*)(slice + tr * RB + cg * 16);
-                char* o = (char*)out + ((size_t)m * ldo + n) * OSZ;
-                if (vec && n + EPG <= N) {
-                    *gptr((uint4_t*)o) = v;
-                } else {                                                 // row end or unaligned rows: element stores
-#pragma unroll
-                    for (int e = 0; e < EPG; ++e) {
-                        if (n + e >= N) break;
-                        const u32 word = v[e * OSZ / 4];
-                        if (OSZ == 2) gptr((u16*)o)[e] = (u16)(word >> (16 * (e & 1)));
-                        else gptr((u32*)o)[e] = word;
+                    for (int e = 0; e < 4; ++e) {
+                        float a = (float)acc[i + b][j][e];
+                        if (sa) a = a * s;
+                        v[4 * b + e] = sw ? a * r[e] : a;
                     }
+                }
+                const uint4_t o = {bf16x2(v[0], v[1]), bf16x2(v[2], v[3]), bf16x2(v[4], v[5]), bf16x2(v[6], v[7])};
+                u16* p = (u16*)out + (size_t)m * ldo + n;
+                if (n + 8 <= N && ldo % 8 == 0) *gptr((uint4_t*)p) = o;
+                else {                                                    // N, ldo multiples of 4: 8-byte pieces
+                    *gptr((uint2_t*)p) = uint2_t{o[0], o[1]};
+                    if (n + 8 <= N) *gptr((uint2_t*)(p + 4)) = uint2_t{o[2], o[3]};
+                }
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                const int n = n0 + wn * NB * 16 + 16 * i + 4 * lg;
+                if (n >= N) continue;
+                if constexpr (ODT == TCQ_I32) {
+                    *gptr((acc_t*)((int*)out + ((size_t)z * M + m) * ldo + n)) = acc[i][j];
+                } else {
+                    float4v v;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        v[e] = (float)acc[i][j][e];
+                        if (sa) v[e] = v[e] * s;
+                    }
+                    if (sw) {
+                        const float4v r = gptr((const float4v*)(sw + n))[0];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) v[e] = v[e] * r[e];
+                    }
+                    *gptr((float4v*)((float*)out + ((size_t)z * M + m) * ldo + n)) = v;
                 }
             }
         }
@@ -220,33 +306,46 @@ __global__ __launch_bounds__(64 * WN * WM) void k_gemm_i8(const void* a_, const 
 }
 
 // =========================================================================================================== C ABI
-template <int ESZ, int TN, int TM, int WN, int WM, int NS>
-static void launch_gemm(int odt, hipStream_t st, const void* a, const void* w, const float* sa, const float* sw, void* out, int ldo,
-                        int M, int N, int K) {
-    const dim3 grid((N + TN - 1) / TN, (M + TM - 1) / TM), block(64 * WN * WM);
-    if (grid.y > 1) {                                   // token tiles share each weight tile: keep the weights in L2
-        if (odt == TCQ_I32) launch_k(k_gemm_i8<ESZ, TN, TM, WN, WM, NS, TCQ_I32, 0>, grid, block, 0, st, a, w, sa, sw, out, ldo, M, N, K);
-        else if (odt == TCQ_F32) launch_k(k_gemm_i8<ESZ, TN, TM, WN, WM, NS, TCQ_F32, 0>, grid, block, 0, st, a, w, sa, sw, out, ldo, M, N, K);
-        else launch_k(k_gemm_i8<ESZ, TN, TM, WN, WM, NS, TCQ_BF16, 0>, grid, block, 0, st, a, w, sa, sw, out, ldo, M, N, K);
-        return;
+template <int ESZ, int TN, int TM, int WN, int WM, int NSW, int NSX>
+static void launch_gemm(int odt, hipStream_t st, const void* x, const void* w, const float* sa, const float* sw, void* out, int ldo,
+                        int M, int N, int K, int parts) {
+    const dim3 grid((N + TN - 1) / TN, (M + TM - 1) / TM, parts), block(64 * WN * WM);
+    const size_t lds = (size_t)(NSW * TN + NSX * TM) * 128;
+    if (ESZ == 1 && odt == TCQ_I32) launch_k(k_gemm_i8<ESZ, TN, TM, WN, WM, NSW, NSX, ESZ == 1 ? TCQ_I32 : TCQ_F32>, grid, block, lds, st, x, w, sa, sw, out, ldo, M, N, K, parts);
+    else if (odt == TCQ_F32) launch_k(k_gemm_i8<ESZ, TN, TM, WN, WM, NSW, NSX, TCQ_F32>, grid, block, lds, st, x, w, sa, sw, out, ldo, M, N, K, parts);
+    else launch_k(k_gemm_i8<ESZ, TN, TM, WN, WM, NSW, NSX, TCQ_BF16>, grid, block, lds, st, x, w, sa, sw, out, ldo, M, N, K, parts);
+}
+
+// The tile with the least estimated time. Workgroups run in rounds of 256 (one per CU); c1 is what a step of one round
+// costs, c2 a step of two rounds (the tiles up to 128 x 128 fit two workgroups on a CU, which share its LDS and matrix
+// cores), later rounds as pairs. In units of 1/16 us per 128-byte step, fitted to INT8 runs over M = 80 .. 968 and N = 1024
+// .. 32768 on MI355X (us, K = 2048): 64 x 64 8.0 (256 workgroups) / 10.1 (512), 128 x 64 9.9 / 15.4, 128 x 128 13.4 / 24.6,
+// 256 x 128 19.4 / 44, 256 x 256 33 / 73. The best tile was the chosen one or within 8 % of it at every size measured:
+// 968 x 2560: 13.3 on 128 x 128 against 15.0 and 15.4; 968 x 2048: 10.6 on 64 x 64 against 12.8 on 128 x 128; 768 x 1152 x
+// 4304: 13.5 on 64 x 64 against 25.2 on 128 x 128.
+struct TileCost { int tn, tm, c1, c2; };
+constexpr TileCost TILES[5] = {{64, 64, 4, 6}, {128, 64, 6, 12}, {128, 128, 9, 20}, {256, 128, 16, 38}, {256, 256, 30, 68}};
+static int choose_tile(int M, int N, int parts) {
+    int best = 0;
+    long bc = 0;
+    for (int i = 0; i < 5; ++i) {
+        const long w = (long)((N + TILES[i].tn - 1) / TILES[i].tn) * ((M + TILES[i].tm - 1) / TILES[i].tm) * parts, r = (w + 255) / 256;
+        const long c = r == 1 ? 2 * TILES[i].c1 : r * TILES[i].c2;
+        if (i == 0 || c < bc) { best = i; bc = c; }
     }
-    if (odt == TCQ_I32) launch_k(k_gemm_i8<ESZ, TN, TM, WN, WM, NS, TCQ_I32>, grid, block, 0, st, a, w, sa, sw, out, ldo, M, N, K);
-    else if (odt == TCQ_F32) launch_k(k_gemm_i8<ESZ, TN, TM, WN, WM, NS, TCQ_F32>, grid, block, 0, st, a, w, sa, sw, out, ldo, M, N, K);
-    else launch_k(k_gemm_i8<ESZ, TN, TM, WN, WM, NS, TCQ_BF16>, grid, block, 0, st, a, w, sa, sw, out, ldo, M, N, K);
+    return best;
 }
 
 template <int ESZ>
-static void launch_by_m(int odt, hipStream_t st, const void* a, const void* w, const float* sa, const float* sw, void* out, int ldo,
-                        int M, int N, int K) {
-    // The largest tile (weights x tokens) that still gives one workgroup per CU (256), else the smallest: a narrow product
-    // on 256 x 256 tiles leaves most CUs idle. Measured on MI355X at M = 800 (FP32 out, bit-identical across tiles):
-    // N = 2048, K = 16384: 206.5 us on 256 x 256 (32 workgroups), 84.3 on 128 x 64 (208); N = 2048, K = 2048: 32.3 -> 15.4;
-    // N = 2560: 37.9 -> 16.8; N = 32768 (512 workgroups of 256 x 256): 118.5 against 143-274 on the smaller tiles.
-    auto wgs = [&](int tn, int tm) { return (long)((N + tn - 1) / tn) * ((M + tm - 1) / tm); };
-    if (M > 128 && wgs(256, 256) >= 256) launch_gemm<ESZ, 256, 256, 2, 4, 4>(odt, st, a, w, sa, sw, out, ldo, M, N, K);
-    else if (M > 64 && wgs(256, 128) >= 256) launch_gemm<ESZ, 256, 128, 4, 2, 4>(odt, st, a, w, sa, sw, out, ldo, M, N, K);
-    else if (wgs(256, 64) >= 256) launch_gemm<ESZ, 256, 64, 4, 1, 4>(odt, st, a, w, sa, sw, out, ldo, M, N, K);
-    else launch_gemm<ESZ, 128, 64, 4, 1, 4>(odt, st, a, w, sa, sw, out, ldo, M, N, K);
+static void launch_by_size(int odt, hipStream_t st, const void* x, const void* w, const float* sa, const float* sw, void* out, int ldo,
+                           int M, int N, int K, int parts) {
+    switch (choose_tile(M, N, parts)) {
+        case 0: launch_gemm<ESZ, 64, 64, 2, 2, 4, 4>(odt, st, x, w, sa, sw, out, ldo, M, N, K, parts); break;
+        case 1: launch_gemm<ESZ, 128, 64, 4, 2, 3, 3>(odt, st, x, w, sa, sw, out, ldo, M, N, K, parts); break;
+        case 2: launch_gemm<ESZ, 128, 128, 2, 4, 3, 2>(odt, st, x, w, sa, sw, out, ldo, M, N, K, parts); break;
+        case 3: launch_gemm<ESZ, 256, 128, 4, 2, 3, 3>(odt, st, x, w, sa, sw, out, ldo, M, N, K, parts); break;
+        default: launch_gemm<ESZ, 256, 256, 2, 4, 3, 2>(odt, st, x, w, sa, sw, out, ldo, M, N, K, parts); break;
+    }
 }
 
 extern "C" int tcq_gemm_i8(const int8_t* a, const int8_t* w, const float* sa, const float* sw, void* out, int out_dtype, int ldo,
@@ -262,7 +361,7 @@ extern "C" int tcq_gemm_i8(const int8_t* a, const int8_t* w, const float* sa, co
         if (N % 16 == 0) return tcq_gemm_w8(&seg, 1, a, sa, M, K, out_dtype, ldo, stream);
     }
     if (out_dtype != TCQ_I32 && out_dtype != TCQ_F32 && out_dtype != TCQ_BF16) return TCQ_ERR_DTYPE;
-    launch_by_m<1>(out_dtype, (hipStream_t)stream, a, w, sa, sw, out, ldo, M, N, K);
+    launch_by_size<1>(out_dtype, (hipStream_t)stream, a, w, sa, sw, out, ldo, M, N, K, 1);
     return launch_status();
 }
 
@@ -273,6 +372,6 @@ extern "C" int tcq_gemm_bf16(const void* a, const void* w, const float* sa, cons
     if (K % 16 || N % 4) return TCQ_ERR_SHAPE;
     if ((size_t)M * K * 2 >= ((size_t)1 << 31) || (size_t)N * K * 2 >= ((size_t)1 << 31)) return TCQ_ERR_SHAPE;
     if ((uintptr_t)a % 16 || (uintptr_t)w % 16 || (uintptr_t)out % 16 || (sw && (uintptr_t)sw % 16) || ldo % 4) return TCQ_ERR_ALIGN;
-    launch_by_m<2>(out_dtype, (hipStream_t)stream, a, w, sa, sw, out, ldo, M, N, K);
+    launch_by_size<2>(out_dtype, (hipStream_t)stream, a, w, sa, sw, out, ldo, M, N, K, 1);
     return launch_status();
 }
