@@ -365,6 +365,15 @@ typedef struct tcq_gemm_seg {
     int rows_per_table;  /* row-group tables: rows m / G per table (a multiple of 16); 0 = one table */
 } tcq_gemm_seg;
 
+/* Dense weights of up to TCQ_MAX_SEGS layers of one width n in one launch: segment i's (m, n) rows, row-major and 16-byte
+ * aligned, of out_dtype I8 (the bytes of tcq_decode_i8) or BF16 (the BF16 images of those values, exact; kernels.decode_bf16,
+ * deploy/tcq_kernels/kernels.py:320-337, 683-686), from the tcq_repack words (16-byte aligned) and t8; rows_per_table as in
+ * the descriptor; rs unused. segs: HOST array. The prefill products of a group read them. */
+int tcq_decode_group(const tcq_gemm_seg* segs, int nseg, int n, int out_dtype, tcq_stream_t stream);
+/* count INT8 values -> BF16 (exact); count a multiple of 16, both 16-byte aligned. The float path's weights of a runtime that
+ * holds INT8 ones. No reference counterpart (k_gemmf_w8 converts in registers, kernels.py:443-462). */
+int tcq_i8_to_bf16(const int8_t* in, void* out, int64_t count, tcq_stream_t stream);
+
 /* W2A8 fused decode + product for M <= 64 tokens: acc[t, i] = sum_k q[t, k] * w8[i, k], exact in int32, with w8 = sign *
  * t8[hash(state)] decoded from the words on the fly. out_dtype F32: z = (float(acc) * s[t]) * rs[i]; BF16: its rounding;
  * I32: acc (with TCQ_K_PARTS2 / TCQ_K_PARTS4: its K parts, M <= 64). q (M, K) int8 row-major (or in the token-block

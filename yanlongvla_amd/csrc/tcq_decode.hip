@@ -76,51 +76,100 @@ __global__ void k_decode_i8(const u16* bits, const i8* t8_all, i8* out, int rpt,
     *(uint4_t*)(out + (size_t)row * n + 16 * J) = w;
 }
 
-// Dense INT8 decode from the tcq_repack words: a wave takes one 1 KiB chunk (one tile row, 256 columns); lane (g, r)
-// holds the windows of row r for tiles 16 c + 4 j + g (j = 0..3) in one dwordx4 and writes their 16 weights, so a store
-// writes 64 contiguous bytes of each of the 16 rows. The lookups are those of the fused products (pk_code states, a
-// sign-folded table with 16 copies, lane l reading copy l mod 16), whose 16 bytes per lane and j are the row's weights in
-// column order, so the output equals k_decode_i8's byte for byte.
-constexpr int DW_C = 16, DW_NW = 16;
+// Dense decode from the tcq_repack words of up to TCQ_MAX_SEGS layers in one launch, INT8 or BF16 out. A wave takes 1 KiB
+// chunks (one tile row, 256 columns); lane (g, r) holds the windows of row r for tiles 16 c + 4 j + g (j = 0..3) in one
+// dwordx4 and writes their 16 weights, so a store covers 64 (INT8) or, in two, 128 contiguous bytes of each of the 16 rows.
+// The lookups are those of the fused products (pk_code states, a sign-folded table with C copies, lane l reading copy
+// l mod C), whose results per lane and j are the row's weights in column order, so the INT8 output equals k_decode_i8's byte
+// for byte; BF16 entries are the table values' BF16 images (exact, |t8| <= 127), the sign folded into bit 15.
+// grid (blocks of NW * CPW chunks, layers, row-group tables); a workgroup reads one table.
+// What bounds it: the writes, once the launch and the table fill (global round trip, 4 C KiB of LDS) are paid for: one
+// launch for a layer group pays them once, and CPW chunks per wave keep one round of workgroups. Backbone gate | up (2 x
+// 16384 x 2048, 67 MB out): 20.9 us as two launches of one chunk per wave.
+struct DecSegs {
+    tcq_gemm_seg s[TCQ_MAX_SEGS];
+};
 
-__global__ __launch_bounds__(64 * DW_NW) void k_decode_i8_words(const u32* words, const i8* t8, i8* out, int m, int n) {
-    __shared__ __attribute__((aligned(16))) u32 tab[1024 * DW_C];
+template <int ODT, int NW, int C, int CPW>
+__global__ __launch_bounds__(64 * NW) void k_decode_words(const DecSegs P, int n) {
+    __shared__ __attribute__((aligned(16))) u32 tab[1024 * C];
+    const tcq_gemm_seg S = P.s[blockIdx.y];
+    const int rpt = S.rows_per_table > 0 ? S.rows_per_table : S.m;
     const int nch = (n + 255) >> 8, tiles = n >> 4;
-    const long long chunk = (long long)blockIdx.x * DW_NW + (threadIdx.x >> 6);
+    const int first = blockIdx.z * rpt;                                  // first row of this table's group
+    const int nchunks = (rpt >> 4) * nch, c0 = blockIdx.x * (NW * CPW) + (threadIdx.x >> 6);
+    if (first >= S.m || (int)blockIdx.x * (NW * CPW) >= nchunks) return; // uniform
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    const bool live = chunk < (long long)(m >> 4) * nch;                 // uniform per wave
-    uint4_t wa = uint4_t{0u, 0u, 0u, 0u};
-    if (live) wa = gptr((const uint4_t*)(words + chunk * 256))[lane];
-    for (int e = threadIdx.x; e < 1024; e += blockDim.x) {
-        const int h = e & 511;
-        int v0 = t8[2 * h];
-        const int v1 = t8[2 * h + 1];
-        if (e >> 9) v0 = -v0;
-        const u32 v = (u32)(v0 & 0xff) | ((u32)(v1 & 0xff) << 8);
-        const u32 vv = v | (v << 16);
+    uint4_t wa[CPW];
 #pragma unroll
-        for (int c = 0; c < DW_C; c += 4) *(uint4_t*)(tab + e * DW_C + c) = uint4_t{vv, vv, vv, vv};
+    for (int i = 0; i < CPW; ++i) {
+        wa[i] = uint4_t{0u, 0u, 0u, 0u};
+        if (c0 + i * NW < nchunks) wa[i] = gptr((const uint4_t*)((const u32*)S.w + ((size_t)(first >> 4) * nch + c0 + i * NW) * 256))[lane];
+    }
+    const i8* t8 = S.t8 + 1024 * blockIdx.z;
+    for (int e = threadIdx.x; e < 1024; e += 64 * NW) {
+        const int h = e & 511, v0 = t8[2 * h], v1 = t8[2 * h + 1];
+        u32 v;
+        if (ODT == TCQ_I8) {
+            v = (u32)((e >> 9 ? -v0 : v0) & 0xff) | ((u32)(v1 & 0xff) << 8);
+            v |= v << 16;
+        } else {
+            v = ((__float_as_uint((float)v0) >> 16) ^ ((u32)(e >> 9) << 15)) | (__float_as_uint((float)v1) & 0xffff0000u);
+        }
+#pragma unroll
+        for (int c = 0; c < C; c += 4) *(uint4_t*)(tab + e * C + c) = uint4_t{v, v, v, v};
     }
     __syncthreads();
-    if (!live) return;
-    const int I = (int)(chunk / nch), c = (int)(chunk % nch);
-    const u32 cp4 = (u32)(lane & (DW_C - 1)) << 2;
+    const u32 cp4 = (u32)(lane & (C - 1)) << 2;
+    constexpr int SH = C == 16 ? 6 : 4;                                  // log2 of an entry's bytes
+    static_assert(4 * C == 1 << SH, "copies");
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const u32 hi = wa[j];
-        const u32 hn = (u32)__builtin_amdgcn_mov_dpp((int)hi, 0x12F, 0xf, 0xf, false);
-        u32 e0[4], e1[4];
+    for (int i = 0; i < CPW; ++i) {
+        const int chunk = c0 + i * NW;
+        if (chunk >= nchunks) break;                                     // uniform per wave
+        const int I = chunk / nch, c = chunk - I * nch;
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            const u32 x = pk_code(p == 0 ? hi : __builtin_amdgcn_alignbit(hi, hn, 32 - 4 * p));
-            e0[p] = *(const u16*)((const char*)tab + (((x >> 22) << 6) | cp4));            // pair p
-            e1[p] = *(const u16*)((const char*)tab + ((x & 0xFFC0u) | cp4));                // pair p + 4
+        for (int j = 0; j < 4; ++j) {
+            const u32 hi = wa[i][j];
+            const u32 hn = (u32)__builtin_amdgcn_mov_dpp((int)hi, 0x12F, 0xf, 0xf, false);
+            u32 e0[4], e1[4];
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                const u32 x = pk_code(p == 0 ? hi : __builtin_amdgcn_alignbit(hi, hn, 32 - 4 * p));
+                const char* a0 = (const char*)tab + (((x >> 22) << SH) | cp4);               // pair p
+                const char* a1 = (const char*)tab + ((((x >> 6) & 1023u) << SH) | cp4);      // pair p + 4
+                if (ODT == TCQ_I8) { e0[p] = *(const u16*)a0; e1[p] = *(const u16*)a1; }
+                else { e0[p] = *(const u32*)a0; e1[p] = *(const u32*)a1; }
+            }
+            const int tile = 16 * c + 4 * j + g;
+            if (tile >= tiles) continue;
+            const size_t at = (size_t)(first + 16 * I + r) * n + 16 * tile;
+            if (ODT == TCQ_I8) {
+                *gptr((uint4_t*)((i8*)S.out + at)) =
+                    uint4_t{e0[0] | (e0[1] << 16), e0[2] | (e0[3] << 16), e1[0] | (e1[1] << 16), e1[2] | (e1[3] << 16)};
+            } else {
+                gptr((uint4_t*)((u16*)S.out + at))[0] = uint4_t{e0[0], e0[1], e0[2], e0[3]};
+                gptr((uint4_t*)((u16*)S.out + at))[1] = uint4_t{e1[0], e1[1], e1[2], e1[3]};
+            }
         }
-        const int tile = 16 * c + 4 * j + g;
-        if (tile < tiles)
-            *gptr((uint4_t*)(out + (size_t)(16 * I + r) * n + 16 * tile)) =
-                uint4_t{e0[0] | (e0[1] << 16), e0[2] | (e0[3] << 16), e1[0] | (e1[1] << 16), e1[2] | (e1[3] << 16)};
     }
+}
+
+// INT8 -> BF16 (exact), 16 values per thread
+__global__ void k_i8_to_bf16(const i8* in, u16* out, size_t n16) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n16) return;
+    const uint4_t w = gptr((const uint4_t*)in)[i];
+    u32 v[8];
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const float a = (float)(i8)(w[d] >> (16 * h)), b = (float)(i8)(w[d] >> (16 * h + 8));
+            v[2 * d + h] = __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+        }
+    gptr((uint4_t*)out)[2 * i] = uint4_t{v[0], v[1], v[2], v[3]};
+    gptr((uint4_t*)out)[2 * i + 1] = uint4_t{v[4], v[5], v[6], v[7]};
 }
 
 __global__ void k_decode_f16(const u16* bits, const u16* tlut_all, u16* out, int rpt, int n) {
@@ -192,13 +241,57 @@ extern "C" int tcq_decode_i8_groups(const void* bits, const int8_t* t8, int G, i
     return launch_status();
 }
 
+template <int ODT>
+static void launch_words(const DecSegs& P, int nseg, int tables, long long total, long long most, int n, hipStream_t st) {
+    auto grid = [&](int per) { return dim3((unsigned)((most + per - 1) / per), nseg, tables); };
+    // 512 workgroups of 16 waves fill the chip (64 KiB of table, two per CU); below a quarter of that, smaller workgroups
+    // with a smaller table spread over more CUs
+    if (total < 2048) launch_k(k_decode_words<ODT, 4, 4, 1>, grid(4), dim3(256), 0, st, P, n);
+    else if (total <= 8192) launch_k(k_decode_words<ODT, 16, 16, 1>, grid(16), dim3(1024), 0, st, P, n);
+    else if (total <= 16384) launch_k(k_decode_words<ODT, 16, 16, 2>, grid(32), dim3(1024), 0, st, P, n);
+    else launch_k(k_decode_words<ODT, 16, 16, 4>, grid(64), dim3(1024), 0, st, P, n);
+}
+
+extern "C" int tcq_decode_group(const tcq_gemm_seg* segs, int nseg, int n, int out_dtype, tcq_stream_t stream) {
+    if (!segs || nseg <= 0 || n <= 0) return TCQ_ERR_ARG;
+    if (out_dtype != TCQ_I8 && out_dtype != TCQ_BF16) return TCQ_ERR_DTYPE;
+    if (nseg > TCQ_MAX_SEGS) return TCQ_ERR_UNSUPPORTED;
+    if (n % 16) return TCQ_ERR_SHAPE;
+    DecSegs P = {};
+    const long long nch = (n + 255) / 256;
+    long long total = 0, most = 0;
+    int tables = 1;
+    for (int i = 0; i < nseg; ++i) {
+        const tcq_gemm_seg& g = segs[i];
+        if (!g.w || !g.t8 || !g.out || g.m <= 0) return TCQ_ERR_ARG;
+        if (g.m % 16 || g.rows_per_table < 0 || (g.rows_per_table > 0 && !groups_ok(g.m, g.m / g.rows_per_table))) return TCQ_ERR_SHAPE;
+        if (g.rows_per_table > 0 && g.m % g.rows_per_table) return TCQ_ERR_SHAPE;
+        if ((g.m / 16) * nch >= ((long long)1 << 31)) return TCQ_ERR_SHAPE;
+        if ((uintptr_t)g.out % 16 || (uintptr_t)g.w % 16) return TCQ_ERR_ALIGN;
+        const int rpt = g.rows_per_table > 0 ? g.rows_per_table : g.m;
+        const long long chunks = (rpt / 16) * nch;
+        if (g.m / rpt > tables) tables = g.m / rpt;
+        if (chunks > most) most = chunks;
+        total += chunks * (g.m / rpt);
+        P.s[i] = g;
+    }
+    if (out_dtype == TCQ_I8) launch_words<TCQ_I8>(P, nseg, tables, total, most, n, (hipStream_t)stream);
+    else launch_words<TCQ_BF16>(P, nseg, tables, total, most, n, (hipStream_t)stream);
+    return launch_status();
+}
+
 extern "C" int tcq_decode_i8_words(const void* words, const int8_t* t8, int8_t* out, int m, int n, tcq_stream_t stream) {
-    if (!words || !t8 || !out || m <= 0 || n <= 0) return TCQ_ERR_ARG;
-    if (m % 16 || n % 16) return TCQ_ERR_SHAPE;
-    if ((uintptr_t)out % 16 || (uintptr_t)words % 16) return TCQ_ERR_ALIGN;
-    const long long chunks = (long long)(m / 16) * ((n + 255) / 256);
-    launch_k(k_decode_i8_words, dim3((unsigned)((chunks + DW_NW - 1) / DW_NW)), dim3(64 * DW_NW), 0, (hipStream_t)stream,
-             (const u32*)words, (const i8*)t8, (i8*)out, m, n);
+    if (m <= 0) return TCQ_ERR_ARG;
+    const tcq_gemm_seg seg = {words, t8, nullptr, out, m, 0};
+    return tcq_decode_group(&seg, 1, n, TCQ_I8, stream);
+}
+
+extern "C" int tcq_i8_to_bf16(const int8_t* in, void* out, int64_t count, tcq_stream_t stream) {
+    if (!in || !out || count <= 0) return TCQ_ERR_ARG;
+    if (count % 16 || count / 16 > ((int64_t)1 << 31) * 64) return TCQ_ERR_SHAPE;
+    if ((uintptr_t)in % 16 || (uintptr_t)out % 16) return TCQ_ERR_ALIGN;
+    const size_t n16 = (size_t)count / 16;
+    launch_k(k_i8_to_bf16, dim3((unsigned)((n16 + 255) / 256)), dim3(256), 0, (hipStream_t)stream, (const i8*)in, (u16*)out, n16);
     return launch_status();
 }
 

@@ -69,10 +69,10 @@ struct Tail { static constexpr bool value = false; };
 }  // namespace
 
 // ESZ: element size (1 INT8, 2 BF16); K in elements. parts: K parts (grid.z, int32 outputs): part z sums the steps
-// [z ceil(nk / parts), ...) into out + z M ldo.
+// [z ceil(nk / parts), ...) into out + z M ldo. flush: steps per first-level sum (BF16).
 template <int ESZ, int TN, int TM, int WN, int WM, int NSW, int NSX, int ODT>
 __global__ __launch_bounds__(64 * WN * WM) void k_gemm_i8(const void* x_, const void* w_, const float* sa, const float* sw, void* out,
-                                                       int ldo, int M, int N, int K_, int parts) {
+                                                       int ldo, int M, int N, int K_, int parts, int flush) {
     typedef typename MfmaOf<ESZ>::acc_t acc_t;
     constexpr int NWAVE = WN * WM;
     constexpr int WL = TN / 8 / NWAVE, XL = TM / 8 / NWAVE;              // 1 KiB loads (8 rows x 128 bytes) per wave and step
@@ -243,9 +243,36 @@ __global__ __launch_bounds__(64 * WN * WM) void k_gemm_i8(const void* x_, const 
         mm(1, 1, 1);
         spread(Num<HB + MB>{}, Num<XL>{});
     };
-    int kt = 0;
-    for (; kt + NS < nfull; ++kt) step(kt, Full{});
-    for (; kt < nk; ++kt) step(kt, Tail{});
+    if constexpr (ESZ == 1) {
+        int kt = 0;
+        for (; kt + NS < nfull; ++kt) step(kt, Full{});
+        for (; kt < nk; ++kt) step(kt, Tail{});
+    } else {
+        // FP32 sums in two levels, `flush` steps (two MFMAs each) in a row, then the sums of those: the rounding error of one
+        // chain over all of K grows with its length (relative error of the float path's layers against 64 bits, K = 16384:
+        // 4.3e-4 with two levels, as the few-token products' partial sums give; 4.6e-4 with one chain)
+        acc_t sum[NB][MB];
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int j = 0; j < MB; ++j) sum[i][j] = acc[i][j];
+        for (int kt = 0; kt < nk;) {
+            const int end = min(nk, kt + flush);
+            for (; kt < end && kt + NS < nfull; ++kt) step(kt, Full{});
+            for (; kt < end; ++kt) step(kt, Tail{});
+#pragma unroll
+            for (int i = 0; i < NB; ++i)
+#pragma unroll
+                for (int j = 0; j < MB; ++j) {
+                    sum[i][j] += acc[i][j];
+                    acc[i][j] = acc_t{0, 0, 0, 0};
+                }
+        }
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int j = 0; j < MB; ++j) acc[i][j] = sum[i][j];
+    }
     wait_cnt<0, 0>();                               // no load into the LDS outlives the workgroup
     // D: register e of lane (g, c) = weight row 4 g + e of the A block, token c of the B block
     const int z = blockIdx.z;
@@ -311,9 +338,11 @@ static void launch_gemm(int odt, hipStream_t st, const void* x, const void* w, c
                         int M, int N, int K, int parts) {
     const dim3 grid((N + TN - 1) / TN, (M + TM - 1) / TM, parts), block(64 * WN * WM);
     const size_t lds = (size_t)(NSW * TN + NSX * TM) * 128;
-    if (ESZ == 1 && odt == TCQ_I32) launch_k(k_gemm_i8<ESZ, TN, TM, WN, WM, NSW, NSX, ESZ == 1 ? TCQ_I32 : TCQ_F32>, grid, block, lds, st, x, w, sa, sw, out, ldo, M, N, K, parts);
-    else if (odt == TCQ_F32) launch_k(k_gemm_i8<ESZ, TN, TM, WN, WM, NSW, NSX, TCQ_F32>, grid, block, lds, st, x, w, sa, sw, out, ldo, M, N, K, parts);
-    else launch_k(k_gemm_i8<ESZ, TN, TM, WN, WM, NSW, NSX, TCQ_BF16>, grid, block, lds, st, x, w, sa, sw, out, ldo, M, N, K, parts);
+    int flush = 1;                                      // sqrt(steps / 2): chains of 2 flush and steps / flush are equally long
+    while (2 * flush * flush < (K * ESZ + 127) / 128) ++flush;
+    if (ESZ == 1 && odt == TCQ_I32) launch_k(k_gemm_i8<ESZ, TN, TM, WN, WM, NSW, NSX, ESZ == 1 ? TCQ_I32 : TCQ_F32>, grid, block, lds, st, x, w, sa, sw, out, ldo, M, N, K, parts, flush);
+    else if (odt == TCQ_F32) launch_k(k_gemm_i8<ESZ, TN, TM, WN, WM, NSW, NSX, TCQ_F32>, grid, block, lds, st, x, w, sa, sw, out, ldo, M, N, K, parts, flush);
+    else launch_k(k_gemm_i8<ESZ, TN, TM, WN, WM, NSW, NSX, TCQ_BF16>, grid, block, lds, st, x, w, sa, sw, out, ldo, M, N, K, parts, flush);
 }
 
 // The tile with the least estimated time. Workgroups run in rounds of 256 (one per CU); c1 is what a step of one round
@@ -324,11 +353,11 @@ static void launch_gemm(int odt, hipStream_t st, const void* x, const void* w, c
 // 968 x 2560: 13.3 on 128 x 128 against 15.0 and 15.4; 968 x 2048: 10.6 on 64 x 64 against 12.8 on 128 x 128; 768 x 1152 x
 // 4304: 13.5 on 64 x 64 against 25.2 on 128 x 128.
 struct TileCost { int tn, tm, c1, c2; };
-constexpr TileCost TILES[5] = {{64, 64, 4, 6}, {128, 64, 6, 12}, {128, 128, 9, 20}, {256, 128, 16, 38}, {256, 256, 30, 68}};
-static int choose_tile(int M, int N, int parts) {
+constexpr TileCost TILES[5] = {{64, 64, 4, 7}, {128, 64, 6, 12}, {128, 128, 9, 20}, {256, 128, 16, 38}, {256, 256, 30, 68}};
+static int choose_tile(int M, int N, int parts, int tiles) {
     int best = 0;
     long bc = 0;
-    for (int i = 0; i < 5; ++i) {
+    for (int i = 0; i < tiles; ++i) {
         const long w = (long)((N + TILES[i].tn - 1) / TILES[i].tn) * ((M + TILES[i].tm - 1) / TILES[i].tm) * parts, r = (w + 255) / 256;
         const long c = r == 1 ? 2 * TILES[i].c1 : r * TILES[i].c2;
         if (i == 0 || c < bc) { best = i; bc = c; }
@@ -339,12 +368,13 @@ static int choose_tile(int M, int N, int parts) {
 template <int ESZ>
 static void launch_by_size(int odt, hipStream_t st, const void* x, const void* w, const float* sa, const float* sw, void* out, int ldo,
                            int M, int N, int K, int parts) {
-    switch (choose_tile(M, N, parts)) {
+    switch (choose_tile(M, N, parts, ESZ == 1 ? 5 : 4)) {       // BF16 keeps two levels of sums: no registers for 256 x 256
         case 0: launch_gemm<ESZ, 64, 64, 2, 2, 4, 4>(odt, st, x, w, sa, sw, out, ldo, M, N, K, parts); break;
         case 1: launch_gemm<ESZ, 128, 64, 4, 2, 3, 3>(odt, st, x, w, sa, sw, out, ldo, M, N, K, parts); break;
         case 2: launch_gemm<ESZ, 128, 128, 2, 4, 3, 2>(odt, st, x, w, sa, sw, out, ldo, M, N, K, parts); break;
         case 3: launch_gemm<ESZ, 256, 128, 4, 2, 3, 3>(odt, st, x, w, sa, sw, out, ldo, M, N, K, parts); break;
-        default: launch_gemm<ESZ, 256, 256, 2, 4, 3, 2>(odt, st, x, w, sa, sw, out, ldo, M, N, K, parts); break;
+        default:
+            if constexpr (ESZ == 1) launch_gemm<ESZ, 256, 256, 2, 4, 3, 2>(odt, st, x, w, sa, sw, out, ldo, M, N, K, parts);
     }
 }
 

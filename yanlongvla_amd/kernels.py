@@ -93,6 +93,33 @@ def decode_words(words, t8, out):
     call('tcq_decode_i8_words', ptr(words), ptr(t8), ptr(out), m, n, stream())
 
 
+def decode_group(segs, n):
+    """Dense weights of 1..4 layers of width n in one launch: segs [(words, t8, out), ...], words of repack, t8 (512, 2) or
+    (G, 512, 2), out contiguous (m, n) int8 (the bytes of decode) or bfloat16 (the same values)."""
+    if not 1 <= len(segs) <= _lib.MAX_SEGS:
+        raise ValueError(f'1 to {_lib.MAX_SEGS} segments')
+    arr = (_lib.GemmSeg * len(segs))()
+    kind = segs[0][2].dtype
+    if kind not in (torch.int8, torch.bfloat16):
+        raise TypeError('decode_group: int8 or bfloat16 outputs')
+    for i, (words, t8, out) in enumerate(segs):
+        _contig(words, t8, out)
+        m, G = out.shape[0], _groups(t8)
+        if out.dtype != kind or out.shape[1] != n or words.numel() != repack_words(m, n):
+            raise ValueError(f'segment {i}: words / output {tuple(out.shape)} {out.dtype} do not fit')
+        arr[i] = _lib.GemmSeg(ptr(words), ptr(t8), None, ptr(out), m, 0 if G == 1 else m // G)
+    call('tcq_decode_group', arr, len(segs), n, 1 if kind == torch.bfloat16 else 4, stream())
+
+
+def i8_to_bf16(w, out):
+    """INT8 weights as BF16 (exact), the same shape, contiguous."""
+    _contig(w, out)
+    if w.dtype != torch.int8 or out.dtype != torch.bfloat16 or w.shape != out.shape:
+        raise ValueError('i8_to_bf16: int8 -> bfloat16 of the same shape')
+    call('tcq_i8_to_bf16', ptr(w), ptr(out), w.numel(), stream())
+    return out
+
+
 def decode_f16(bits, tlut, out):
     """Dense decode through the FP16 table, out (m, n) float16 (exact lookup(states, tlut))."""
     m, n = out.shape

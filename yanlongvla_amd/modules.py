@@ -176,12 +176,12 @@ class Group:
     def decode(self, W=None):
         """The group's dense INT8 weight rows into W (default: the resident W)."""
         W = self.W if W is None else W
-        for L, seg in zip(self.layers, self.segments):
-            rows = W[seg.col0:seg.col0 + seg.width]
-            if L.t8.dim() == 2 and L._words is not None:
-                kernels.decode_words(L._words, L.t8, rows)          # the words the fused products keep
-            else:
-                kernels.decode(L.bits, L.t8, rows)
+        rows = [W[s.col0:s.col0 + s.width] for s in self.segments]
+        if all(L._words is not None for L in self.layers):              # the words the fused products keep: one launch
+            kernels.decode_group([(L._words, L.t8, r) for L, r in zip(self.layers, rows)], self.K)
+        else:
+            for L, r in zip(self.layers, rows):
+                kernels.decode(L.bits, L.t8, r)
         return W
 
     # -------------------------------------------------------------------------------------------- activations
@@ -359,12 +359,22 @@ class Group:
 
     def run_float(self, x2, shape):
         """W2: BF16 rotated activations (kernels.rht = the reference's pre_h), the INT8 table values as BF16 weights, FP32
-        sums, on the fused products (kernels.gemmf_segments: the packed words decoded on the fly, or the resident INT8
-        weights; no dense BF16 copy). Expert: z = acc * rs in FP32; prefill: the product rounded to BF16, scaled by rs in
-        the epilogue (modules.py:117-144)."""
+        sums. Few tokens on the fused products (kernels.gemmf_segments: the packed words decoded on the fly, or the resident
+        INT8 weights); many tokens on the BF16 MFMA GEMM over dense BF16 weights made for the call, as the reference's
+        prefill does (modules.py:117-130): the fused products decode every weight again per 64 tokens (backbone gate | up at
+        968 tokens: 1252 us against 30 for the weights and 125 for the GEMM). Expert: z = acc * rs in FP32; prefill: the
+        product rounded to BF16, scaled by rs in the epilogue (modules.py:117-144)."""
         M, dev = x2.shape[0], x2.device
         h = kernels.rht(x2, self.su, torch.empty(M, self.K, dtype=torch.bfloat16, device=dev))
         acc = torch.empty(M, self.Ntot, dtype=torch.float32 if self.small else torch.bfloat16, device=dev)
+        if M > SMALL_M and self.Ntot * self.K < 1 << 30:             # (the GEMM takes weights below 2 GiB)
+            w = torch.empty(self.Ntot, self.K, dtype=torch.bfloat16, device=dev)
+            if self.W is not None:
+                kernels.i8_to_bf16(self.W, w)
+            else:
+                self.decode(w)
+            kernels.gemm_bf16(h, w, acc, sw=self.rs if self.small else None)
+            return self.posts(acc, None, shape)
         if self.W is not None:
             segs = [(self.W[s.col0:s.col0 + s.width], None, s.rs, acc[:, s.col0:]) for s in self.segments]
         else:
