@@ -4,6 +4,7 @@
 //
 // A row moves HBM -> LDS -> HBM in 16-byte vectors (8 elements per thread-step) whenever the row length is a multiple of 8
 // and the rows are 16-byte aligned, else element by element; the Walsh passes run in LDS between the two.
+#include "tcq_blocks.h"
 #include "tcq_device.h"
 #include "tcq_launch.h"
 #include "tcq_rows.h"
@@ -880,6 +881,45 @@ __global__ void k_postg_tw(SEGS segs, const float* s, const u16* gelu_lut, int m
     store_post_row<YDT>(lds, S.y, (size_t)tok * N, S.sv, S.bias, gl, N, vec);
 }
 
+// The same for groups of segments 2^L wide only (8192, 16384; 32 values per thread, 16-byte aligned, checked by the host).
+// Two BF16 rows of 16384 at 968 tokens: 59 us through the LDS engine.
+template <int ADT, int YDT, int L>
+__global__ __launch_bounds__(1 << (L - 5)) void k_postg_tw5(PostPack segs, const float* s, const u16* gelu_lut) {
+    extern __shared__ float lds[];
+    const tcq_post_seg S = segs[blockIdx.y];
+    const int tok = blockIdx.x, i0 = 32 * threadIdx.x;
+    const float st = ADT == TCQ_I32 ? s[tok] : 1.f;
+    float v[32];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+        acc_chunk<ADT>(S.acc, (size_t)tok * S.lda + S.col0 + i0 + 16 * h, st, S.rs ? S.rs + i0 + 16 * h : nullptr, part16(v, h));
+    const Raw16<1> sv[2] = {raw16<1>(S.sv + i0, true), raw16<1>(S.sv + i0 + 16, true)};
+    tw_walsh<L, 5>(v, lds);
+    const float c = (float)(1.0 / __builtin_sqrt((double)(1 << L)));
+#pragma unroll
+    for (int k = 0; k < 32; ++k) v[k] = v[k] * c;
+    tw_to_natural<L, 5>(v, lds);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        float sg[16], b[16];
+        cv16(sv[h], sg);
+        if (S.bias) cv16(raw16<4>(S.bias + i0 + 16 * h, true), b);
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            float& x = v[16 * h + k];
+            x = x * sg[k];
+            if (S.bias) x = x + b[k];
+            if (YDT == TCQ_BF16 && S.gelu) x = bf16_to_f32(gptr(gelu_lut)[f32_to_bf16(x)]);
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            float a[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) a[k] = v[16 * h + 8 * j + k];
+            Elem<YDT>::st8(S.y, ((size_t)tok << L) + i0 + 16 * h + 8 * j, a);
+        }
+    }
+}
 
 // k_mid2 on the register + transpose engine for N = 2^L (2^LE values per thread, 2^(L - LE) threads, aligned): the gate half
 // is loaded at entry and the up half during the gate's transform, each transform returns to the natural layout through LDS,
@@ -1361,6 +1401,8 @@ extern "C" int tcq_rht(const void* x, int x_dtype, int ldx, const int8_t* su, vo
 #undef RHT_Y
         return launch_status();
     }
+    // rows of several blocks, and narrow ones: in the registers of a wave or four (16-bit rows 8-byte aligned, n a multiple of 4)
+    if (blocks_rht(x, x_dtype, ldx, (const i8*)su, y, y_dtype, ldy, M, n, st)) return launch_status();
 #define RHT_Y(XD, YD) launch_k(k_rht<XD, YD>, grid, block, sh, st, x, ldx, (const i8*)su, y, ldy, n, vec)
 #define RHT_X(XD, _)                                          \
     switch (y_dtype) {                                        \
@@ -1422,6 +1464,8 @@ extern "C" int tcq_pre_cs(const void* x, int x_dtype, const int8_t* su, const vo
 #undef PRE_TW
         return launch_status();
     }
+    // rows of several blocks, narrow ones, and column scales
+    if (blocks_pre(x, x_dtype, (const i8*)su, cs, (i8*)q, (int*)q4, ldq, scale, M, K, st)) return launch_status();
 #define PRE(XD, _) launch_k(k_pre<XD>, grid, block, sh, st, x, (const i8*)su, (i8*)q, (int*)q4, ldq, scale, K, vec, cs)
     DISPATCH_X(x_dtype, PRE, 0)
 #undef PRE
@@ -1544,11 +1588,13 @@ extern "C" int tcq_post(const void* acc, int acc_dtype, int lda, int col0, const
 #undef POSTW_K
         return launch_status();
     }
+    hipStream_t st = (hipStream_t)stream;
+    const tcq_post_seg one = {acc, rs, (const i8*)sv, bias, y, lda, col0, N, 0};
+    if (blocks_post(&one, 1, acc_dtype, s, nullptr, y_dtype, M, st)) return launch_status();
     const dim3 grid(M), block(row_threads(M, N));
     const size_t sh = row_lds(N);
     const int vec = N % 8 == 0 && al16(acc) && ((size_t)lda * asz) % 16 == 0 && ((size_t)col0 * asz) % 16 == 0 && al16(y) &&
                     ((size_t)N * dsize(y_dtype)) % 16 == 0 && al8(sv) && (!rs || al16(rs)) && (!bias || al16(bias));
-    hipStream_t st = (hipStream_t)stream;
 #define POST_Y(AD, YD) launch_k(k_post<AD, YD>, grid, block, sh, st, acc, lda, col0, s, rs, (const i8*)sv, bias, y, N, vec)
 #define POST_A(AD)                                           \
     switch (y_dtype) {                                       \
@@ -1690,6 +1736,7 @@ extern "C" int tcq_mid1(const void* acc, int acc_dtype, int lda, const float* s,
     const int svec = al16(sv) && al16(su) && (!bias || al16(bias));
     hipStream_t st = (hipStream_t)stream;
     const i8 *svp = (const i8*)sv, *sup = (const i8*)su;
+    if (blocks_mid1(acc, acc_dtype, lda, s, rs, svp, bias, (const u16*)gelu_lut, sup, (i8*)q, (int*)q4, ldq, scale, M, N, st)) return launch_status();
     switch (acc_dtype) {
         case TCQ_I32: launch_k(k_mid1<TCQ_I32>, grid, block, sh, st, acc, lda, s, rs, svp, bias, gelu_lut, sup, (i8*)q, (int*)q4, ldq, scale, N, vec, svec); break;
         case TCQ_F32: launch_k(k_mid1<TCQ_F32>, grid, block, sh, st, acc, lda, s, rs, svp, bias, gelu_lut, sup, (i8*)q, (int*)q4, ldq, scale, N, vec, svec); break;
@@ -1739,6 +1786,37 @@ extern "C" int tcq_post_group(const tcq_post_seg* segs, int nseg, int acc_dtype,
         wv = wv && (g.N == 256 || g.N == 2048) && al16(g.acc) && ((size_t)g.lda * esz) % 16 == 0 && ((size_t)g.col0 * esz) % 16 == 0 &&
              al16(g.y) && al16(g.sv) && (!g.rs || al16(g.rs)) && (!g.bias || al16(g.bias)) && ysz >= 2;
     }
+    bool tw5 = maxN == 8192 || maxN == 16384;
+    for (int i = 0; i < nseg; ++i) {
+        const tcq_post_seg& g = segs[i];
+        tw5 = tw5 && g.N == maxN && al16(g.acc) && ((size_t)g.lda * esz) % 16 == 0 && ((size_t)g.col0 * esz) % 16 == 0 && al16(g.y) &&
+              al16(g.sv) && (!g.rs || al16(g.rs)) && (!g.bias || al16(g.bias));
+    }
+    if (tw5) {
+        const dim3 g5(M, nseg);
+        const hipStream_t st5 = (hipStream_t)stream;
+#define POST5_Y(AD, YD)                                                                                                    \
+    if (maxN == 8192) launch_k(k_postg_tw5<AD, YD, 13>, g5, dim3(256), row_lds(8192), st5, pk, s, (const u16*)gelu_lut);   \
+    else launch_k(k_postg_tw5<AD, YD, 14>, g5, dim3(512), row_lds(16384), st5, pk, s, (const u16*)gelu_lut)
+#define POST5_A(AD)                                          \
+    switch (y_dtype) {                                       \
+        case TCQ_F32: POST5_Y(AD, TCQ_F32); break;           \
+        case TCQ_BF16: POST5_Y(AD, TCQ_BF16); break;         \
+        case TCQ_F16: POST5_Y(AD, TCQ_F16); break;           \
+        default: return TCQ_ERR_DTYPE;                       \
+    }
+        switch (acc_dtype) {
+            case TCQ_I32: POST5_A(TCQ_I32); break;
+            case TCQ_F32: POST5_A(TCQ_F32); break;
+            case TCQ_BF16: POST5_A(TCQ_BF16); break;
+            default: return TCQ_ERR_DTYPE;
+        }
+#undef POST5_A
+#undef POST5_Y
+        return launch_status();
+    }
+    // segments of several blocks: rows in the registers of a wave or four
+    if (!wv && !tw && blocks_post(segs, nseg, acc_dtype, s, (const u16*)gelu_lut, y_dtype, M, (hipStream_t)stream)) return launch_status();
     const dim3 grid(M, nseg), block(wv ? 512 : tw ? maxN / 16 : row_threads(M * nseg, maxN));
     // no dynamic LDS for k_postg_wv here: its own checks equal the ones above, so it never takes its LDS fallback
     const size_t sh = wv ? 0 : row_lds(maxN);
