@@ -17,6 +17,10 @@
 namespace {
 
 constexpr int AT = 256;          // threads of k_attn_part
+// Causal tokens from which k_attn_rows runs: where its launch of the rotate + quantize, which the combine has fused, is paid
+// back, for both kinds of call so that they round the same outputs. Outputs only, us before / after: 256 tokens 13.4 / 10.4,
+// 968: 53.2 / 33.0. Quantized: 130 tokens 11.9 / 13.6, 256: 15.0 / 14.9, 400: 20.9 / 18.5, 968: 53.9 / 37.6.
+constexpr int ATTN_ROWS_M = 256;
 
 __device__ __forceinline__ const u16* key_row(const u16* cache, const u16* fresh, int P, int j) {
     return j < P ? cache + (size_t)j * AD : fresh + (size_t)(j - P) * AD;
@@ -478,6 +482,191 @@ __global__ __launch_bounds__(128) void k_attn_combine_reg(const float* part, int
     reg_rotate_quantize(v, K, xs, red, q8, q4, ldq, scale, t);
 }
 
+// Many causal tokens. grid ceil(M / 2), 4 waves; a workgroup takes 2 tokens x 8 heads = 16 query rows against all keys that
+// they see, each wave all 16 rows against every fourth 32-key block, with the running maximum, sum and unnormalised outputs of
+// its blocks in registers (rescaled when the maximum grows). The four waves' results merge at the end, weights
+// exp(m_w - max m_w). The last groups see all keys and the first few, so the longest go first.
+// Everything is transposed so that no probability crosses lanes: S^T = K Q^T (A = 16 keys, B = 16 query rows), whose D
+// layout (lane (g, c): keys 4 g .. 4 g + 3 of query c) is the B operand of O^T = V^T P^T once the keys of a 32-key block
+// take the order "4 g .. 4 g + 3 of both 16-key tiles" in lane group g. Keys go from memory straight into the A
+// fragments; values are transposed 8 x 8 in registers and pass through a wave-private LDS tile (dim row (i, dg) = dim 8 dg + i
+// at i VTI + 80 dg, 16 bytes per lane group in one of five slots turned by i: writes and reads spread over all banks), so the
+// loop has no barrier. Scores, exponentials, sums and outputs in FP32, the probabilities rounded to BF16 for the second
+// product, as in k_attn_part.
+// What bounds it: instruction issue; a block of 32 keys is 32 MFMAs in some 500 instructions a wave (without its loads it
+// still takes four fifths of the time), so two workgroups per CU (256 registers, 80 KiB of LDS each) hide each other's
+// waits: groups of 4 tokens need all 512 registers, one workgroup per CU, and measured 33 / 29 / 20 us at 968 / 800 / 400
+// causal tokens against 33 / 26 / 14 here. k_attn_part, which writes and reads back 66 MB of chunk partials at 968 tokens,
+// took 53 / 41 / 19 with its combine. Error against 64 bits (968 tokens, normal inputs): 1.96e-3 against 1.98e-3.
+constexpr int VTI = 32 * 80, VTW = 8 * VTI;                   // bytes between dims i, i + 1 of a group; a wave's tile
+
+__global__ __launch_bounds__(256, 2) void k_attn_rows(const u16* q, const u16* kc, const u16* vc, int P, const u16* kn, const u16* vn,
+                                                      int M, int H, int causal, u16* o) {
+    extern __shared__ __attribute__((aligned(16))) char tiles[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lg = lane >> 4;
+    const int t0 = 2 * ((int)gridDim.x - 1 - (int)blockIdx.x), T = P + M;   // the longest groups first
+    auto visible_end = [&](int t) { return min(T, causal >= 0 ? causal + t + 1 : T); };
+    const int jend = visible_end(min(t0 + 2, M) - 1);
+    char* vt = tiles + wave * VTW;
+    const char* vr = vt + (lr & 7) * VTI + 16 * ((lg + (lr & 7)) % 5);     // this lane's pieces of the values
+    const int t = t0 + (lr >> 3), h = lr & 7;                        // this lane's query row
+    const int vend = t < M ? visible_end(t) : 0;
+    uint4_t Q[8];                                                    // B fragments
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks)
+        Q[ks] = t < M && h < H ? gptr((const uint4_t*)(q + ((size_t)t * H + h) * AD + 32 * ks + 8 * lg))[0] : uint4_t{0, 0, 0, 0};
+    // Rows through buffer resources that end where the group's view does (rows past it read zeros): cache rows below
+    // min(P, jend), this call's rows below jend. The lane offsets are constant; a block is a scalar offset. A block across
+    // row P reads both and joins them (the rows of the other resource are zeros: below it the offset wraps past its end).
+    const int nc = min(P, jend), nn = max(jend - P, 0);
+    const rsrc_t KC_ = make_rsrc(nc ? kc : q, (u32)nc * (AD * 2)), VC_ = make_rsrc(nc ? vc : q, (u32)nc * (AD * 2));
+    const rsrc_t KN_ = make_rsrc(kn, (u32)nn * (AD * 2)), VN_ = make_rsrc(vn, (u32)nn * (AD * 2));
+    const u32 ko = (u32)lr * (AD * 2) + 16u * lg, vo = (u32)(4 * (lane >> 5)) * (AD * 2) + 16u * (lane & 31);
+    uint4_t K[2][8], V[2][8];
+    // block at key j: A fragments (key row lr of tile kt) and the lane's two 8 key x 8 dim pieces (dims 8 (lane % 32) ..,
+    // lane group gv = lane / 32 + 2 b's keys 16 (i / 4) + 4 gv + i % 4)
+    // (fresh: the offset as one register, so that its wrap below zero is the register's)
+    auto fresh = [](u32 off) { asm("" : "+v"(off)); return off; };
+    auto ld = [](rsrc_t r, u32 off) { return __builtin_bit_cast(uint4_t, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0)); };
+    auto kof = [&](int kt, int ks, u32 base) { return base + ko + (u32)(kt * 16 * AD * 2 + ks * 64); };
+    auto vof = [&](int b, int i, u32 base) { return base + vo + (u32)((16 * (i >> 2) + (i & 3) + 8 * b) * AD * 2); };
+    auto load_k = [&](int j) {
+        const bool c = j < P, n = j + 32 > P;                        // uniform
+        const rsrc_t R = c ? KC_ : KN_;
+        const u32 b0 = (u32)(c ? j : j - P) * (AD * 2);
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int ks = 0; ks < 8; ++ks) K[kt][ks] = ld(R, kof(kt, ks, b0));
+        if (c && n)
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                for (int ks = 0; ks < 8; ++ks) K[kt][ks] |= ld(KN_, fresh(kof(kt, ks, (u32)(j - P) * (AD * 2))));
+    };
+    auto load_v = [&](int j) {
+        const bool c = j < P, n = j + 32 > P;
+        const rsrc_t R = c ? VC_ : VN_;
+        const u32 b0 = (u32)(c ? j : j - P) * (AD * 2);
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) V[b][i] = ld(R, vof(b, i, b0));
+        if (c && n)
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) V[b][i] |= ld(VN_, fresh(vof(b, i, (u32)(j - P) * (AD * 2))));
+    };
+    float4_t O[16];
+    float m = -__builtin_inff(), l = 0.f;
+#pragma unroll
+    for (int tl = 0; tl < 16; ++tl) O[tl] = float4_t{0.f, 0.f, 0.f, 0.f};
+    const int all_see = visible_end(t0);                             // keys below it are visible to the whole group
+    constexpr float L2E = 1.44269504088896341f;
+    int j = 32 * wave;
+    if (j < jend) {
+        load_k(j);
+        load_v(j);
+    }
+    for (; j < jend; j += 128) {
+        // values: 8 keys of dim 8 (lane % 32) + i in one 16-byte piece
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const int gv = (lane >> 5) + 2 * b;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                uint4_t w;
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    w[k] = __builtin_amdgcn_perm(V[b][2 * k + 1][i >> 1], V[b][2 * k][i >> 1], (i & 1) ? 0x07060302u : 0x05040100u);
+                *(uint4_t*)(vt + i * VTI + (lane & 31) * 80 + 16 * ((gv + i) % 5)) = w;
+            }
+        }
+        if (j + 128 < jend) load_v(j + 128);
+        float4_t S[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks)
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) S[kt] = mma_bf16(K[kt][ks], Q[ks], S[kt]);
+        if (j + 128 < jend) load_k(j + 128);
+        const bool edge = j + 32 > all_see || t0 + 2 > M;            // uniform: some key of the block is hidden from some row
+        float s[8], p[8], mx = -__builtin_inff();
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s[e] = S[e >> 2][e & 3] * (1.f / 16.f);
+        if (edge)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) s[e] = j + 16 * (e >> 2) + 4 * lg + (e & 3) < vend ? s[e] : -__builtin_inff();
+#pragma unroll
+        for (int e = 0; e < 8; ++e) mx = fmaxf(mx, s[e]);
+        mx = fmaxf(mx, lane_xor(mx, 16, lane));
+        mx = fmaxf(mx, lane_xor(mx, 32, lane));
+        const float mn = fmaxf(m, mx), mz = mn == -__builtin_inff() ? 0.f : mn;
+        if (__builtin_amdgcn_ballot_w64(mn > m)) {                   // uniform: some row's maximum grew
+            const float a = expf(m - mz);                            // 0 for a row without visible keys so far
+            l *= a;
+#pragma unroll
+            for (int tl = 0; tl < 16; ++tl)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) O[tl][e] *= a;
+            m = mn;
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            p[e] = __builtin_amdgcn_exp2f((s[e] - mz) * L2E);
+            l += p[e];
+        }
+        const uint4_t Pb = {bf16_cvt2(p[0], p[1]), bf16_cvt2(p[2], p[3]), bf16_cvt2(p[4], p[5]), bf16_cvt2(p[6], p[7])};
+        // every lane's pieces of the tile are written: the wave's own LDS order, no other wave reads it
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int tl = 0; tl < 16; ++tl) {
+            const uint4_t A = *(const uint4_t*)(vr + (2 * tl + (lr >> 3)) * 80);
+            O[tl] = mma_bf16(A, Pb, O[tl]);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();                             // the next block's values go into the tile after these reads
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    // merge through the tiles' space: the rows' statistics and the waves' outputs, wave w summing dims 64 w .. 64 w + 63
+    __syncthreads();
+    float4_t* x = (float4_t*)tiles;
+    float *sm = (float*)(tiles + 65536), *sl = sm + 64;
+    l += lane_xor(l, 16, lane);
+    l += lane_xor(l, 32, lane);
+    if (lg == 0) {
+        sm[16 * wave + lr] = m;
+        sl[16 * wave + lr] = l;
+    }
+#pragma unroll
+    for (int tl = 0; tl < 16; ++tl) x[(wave * 16 + tl) * 64 + lane] = O[tl];
+    __syncthreads();
+    float mx = -__builtin_inff(), L = 0.f, wt[4];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) mx = fmaxf(mx, sm[16 * w + lr]);
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        const float mw = sm[16 * w + lr];
+        wt[w] = mw == -__builtin_inff() ? 0.f : expf(mw - mx);
+        L = __builtin_fmaf(wt[w], sl[16 * w + lr], L);
+    }
+    if (t >= M || h >= H) return;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int tl = 4 * wave + k;
+        float a[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const float4_t v = x[(w * 16 + tl) * 64 + lane];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a[e] = __builtin_fmaf(wt[w], v[e], a[e]);
+        }
+        *gptr((uint2_t*)(o + ((size_t)t * H + h) * AD + 16 * tl + 4 * lg)) = uint2_t{bf16x2(a[0] / L, a[1] / L), bf16x2(a[2] / L, a[3] / L)};
+    }
+}
+
 extern "C" int tcq_attend_chunks(int P, int M) { return (P + M + KC - 1) / KC; }
 
 extern "C" int tcq_attend_q4(const void* q, const void* k_cache, const void* v_cache, int P, const void* k_new, const void* v_new,
@@ -494,6 +683,15 @@ extern "C" int tcq_attend_q4(const void* q, const void* k_cache, const void* v_c
     const int NC = tcq_attend_chunks(P, M);
     if (NC > MAXC) return TCQ_ERR_UNSUPPORTED;
     hipStream_t st = (hipStream_t)stream;
+    // many causal tokens: no partials; the BF16 rows (into the workspace when the caller wants only their quantized form), then
+    // the rotate + quantize of the row kernels
+    if (M >= ATTN_ROWS_M && causal_offset >= 0 && (!o || (uintptr_t)o % 8 == 0)) {
+        u16* rows = o ? (u16*)o : (u16*)part;
+        launch_k(k_attn_rows, dim3((M + 1) / 2), dim3(256), (size_t)4 * VTW, st, (const u16*)q, (const u16*)k_cache,
+                 (const u16*)v_cache, P, (const u16*)k_new, (const u16*)v_new, M, H, causal_offset, rows);
+        const int e = launch_status();
+        return e || !su ? e : tcq_pre(rows, TCQ_BF16, su, q8, q4, ldq, scale, M, H * AD, stream);
+    }
     // token pairs (16 MFMA rows): measured on MI355X at 50 tokens x 850 keys, 2 tokens per group run 12.5 us, 4 run 13.6 us
     // and 8 run 20 us (fewer, longer groups); single tokens (8 rows, half the MFMA rows empty) match pairs
     launch_k(k_attn_part<2>, dim3((M + 1) / 2, NC), dim3(AT), 0, st, (const u16*)q, (const u16*)k_cache, (const u16*)v_cache, P,
