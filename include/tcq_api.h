@@ -449,6 +449,12 @@ int tcq_gemm_tcq_q4(const void* bits, const int8_t* t8, const int32_t* q4, int l
 int tcq_gemm_i8(const int8_t* a, const int8_t* w, const float* sa, const float* sw, void* out, int out_dtype, int ldo, int M, int N,
                 int K, tcq_stream_t stream);
 
+/* The int32 sums of tcq_gemm_i8 on the tiled GEMM in `parts` = 1, 2 or 4 K parts, part p (consecutive 128-column K steps) at out
+ * + p * M * ldo: for tcq_post_add_norm_pre, which adds them. More than one part needs K >= 2048. No reference counterpart. */
+int tcq_gemm_i8_parts(const int8_t* a, const int8_t* w, int32_t* out, int ldo, int M, int N, int K, int parts, tcq_stream_t stream);
+/* The parts (1, 2 or 4) with the least estimated time of that product and its epilogue, for more than 64 tokens (else 1). */
+int tcq_gemm_i8_best_parts(int M, int N, int K);
+
 /* BF16 GEMM on dense BF16 weights: acc = sum_k a[m, k] w[n, k] with FP32 accumulation, a (M, K) BF16, w (N, K) BF16 (e.g.
  * the INT8 table values as BF16 from tcq_decode_f16 with the BF16 table); out = (acc * sa[m]) * sw[n] as FP32 or BF16
  * (sa / sw may be NULL: factor 1). K % 16 == 0, N % 4 == 0; a, w, out 16-byte aligned. Replaces the prefill product of the

@@ -46,3 +46,21 @@ def test_bf16_tiles_against_fp64(M, N, K):
     sw = torch.rand(N, device=DEV) + 0.01
     assert torch.equal(Kn.gemm_bf16(a, w, torch.empty(M, N, device=DEV), sw=sw), z * sw)
     assert torch.equal(Kn.gemm_bf16(a, w, torch.empty(M, N, dtype=torch.bfloat16, device=DEV)), z.bfloat16())
+
+
+@pytest.mark.parametrize('M,N,K', [(65, 64, 2048), (129, 132, 2064), (300, 1156, 4304), (968, 2048, 16384)])
+@pytest.mark.parametrize('parts', [1, 2, 4])
+def test_k_parts_bitexact(M, N, K, parts):
+    """The parts add to the exact product: parts with a partial last K step, uneven and equal ones."""
+    from yanlongvla_amd import kernels as Kn
+    a, w = _ints(M, K, seed=5), _ints(N, K, seed=6)
+    acc = Kn.gemm_i8_parts(a, w, parts)
+    assert acc.shape == (parts, M, N)
+    assert torch.equal(acc.sum(0), (a.double() @ w.double().t()).to(torch.int64))
+
+
+def test_k_parts_refused():
+    from yanlongvla_amd import _lib, kernels as Kn
+    for K, parts in ((2032, 2), (4096, 3)):
+        with pytest.raises(_lib.TcqError):
+            Kn.gemm_i8_parts(_ints(80, K, seed=7), _ints(64, K, seed=8), parts)

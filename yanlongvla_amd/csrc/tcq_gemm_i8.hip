@@ -354,7 +354,7 @@ static void launch_gemm(int odt, hipStream_t st, const void* x, const void* w, c
 // 4304: 13.5 on 64 x 64 against 25.2 on 128 x 128.
 struct TileCost { int tn, tm, c1, c2; };
 constexpr TileCost TILES[5] = {{64, 64, 4, 7}, {128, 64, 6, 12}, {128, 128, 9, 20}, {256, 128, 16, 38}, {256, 256, 30, 68}};
-static int choose_tile(int M, int N, int parts, int tiles) {
+static int choose_tile(int M, int N, int parts, int tiles, long* cost = nullptr) {
     int best = 0;
     long bc = 0;
     for (int i = 0; i < tiles; ++i) {
@@ -362,6 +362,7 @@ static int choose_tile(int M, int N, int parts, int tiles) {
         const long c = r == 1 ? 2 * TILES[i].c1 : r * TILES[i].c2;
         if (i == 0 || c < bc) { best = i; bc = c; }
     }
+    if (cost) *cost = bc;                               // a step's time in units of 1/32 us
     return best;
 }
 
@@ -393,6 +394,36 @@ extern "C" int tcq_gemm_i8(const int8_t* a, const int8_t* w, const float* sa, co
     if (out_dtype != TCQ_I32 && out_dtype != TCQ_F32 && out_dtype != TCQ_BF16) return TCQ_ERR_DTYPE;
     launch_by_size<1>(out_dtype, (hipStream_t)stream, a, w, sa, sw, out, ldo, M, N, K, 1);
     return launch_status();
+}
+
+extern "C" int tcq_gemm_i8_parts(const int8_t* a, const int8_t* w, int32_t* out, int ldo, int M, int N, int K, int parts,
+                                 tcq_stream_t stream) {
+    if (!a || !w || !out || M <= 0 || N <= 0 || K <= 0 || ldo < N || (parts != 1 && parts != 2 && parts != 4)) return TCQ_ERR_ARG;
+    if (K % 16 || N % 4 || (parts > 1 && K < 128 * 16)) return TCQ_ERR_SHAPE;            // every part has steps of its own
+    if ((size_t)M * K >= ((size_t)1 << 31) || (size_t)N * K >= ((size_t)1 << 31)) return TCQ_ERR_SHAPE;
+    if ((uintptr_t)a % 16 || (uintptr_t)w % 16 || (uintptr_t)out % 16 || ldo % 4) return TCQ_ERR_ALIGN;
+    launch_by_size<1>(TCQ_I32, (hipStream_t)stream, a, w, nullptr, nullptr, out, ldo, M, N, K, parts);
+    return launch_status();
+}
+
+// The K parts with the least estimated time: steps at choose_tile's cost, and for each part past the first its write and the
+// epilogue's read at 3 TB/s. A long K over few tiles leaves the large tiles too few workgroups and the small ones bound by
+// their loads into LDS; parts give the larger tiles the whole chip. MI355X, us with the epilogue in 1 / 2 / 4 parts, the
+// chosen one first: 968 x 2048 x 16384 49 (2) against 61 / 48.7, 800: 45.7 (2) against 56 / 44.4, 200: 23.5 (4) against 40 / 26;
+// 400 x 1024 x 4096 14.5 (2) against 17.5 / 15.8, 968 x 1024 x 4096 19.3 (1) against 18.8 / 20.9; 968 x 2048 x 2048 22.4 (1)
+// against 24.5 / 26.6.
+extern "C" int tcq_gemm_i8_best_parts(int M, int N, int K) {
+    if (M <= 64 || N <= 0 || K < 128 * 16) return 1;
+    int best = 1;
+    double bt = 0;
+    for (int parts = 1; parts <= 4; parts *= 2) {
+        long c = 0;
+        choose_tile(M, N, parts, 5, &c);
+        const int steps = (K + 127) / 128;
+        const double t = (steps + parts - 1) / parts * (c / 32.0) + (parts - 1) * (8.0 * M * N) / 3e6;
+        if (parts == 1 || (t < bt && (size_t)parts * M * N < ((size_t)1 << 31))) { best = parts; bt = t; }
+    }
+    return best;
 }
 
 extern "C" int tcq_gemm_bf16(const void* a, const void* w, const float* sa, const float* sw, void* out, int out_dtype, int ldo, int M,

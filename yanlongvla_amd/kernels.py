@@ -743,6 +743,11 @@ def gemm_tcq(bits, t8, q4, s, rs, z, K, bounds=(1 << 30, 1 << 30)):
          int(bounds[1]), stream())
 
 
+def gemm_i8_best_parts(M, N, K):
+    """The K parts (1, 2 or 4) of gemm_i8_parts with the least estimated time, epilogue included (1 for at most 64 tokens)."""
+    return int(_lib.lib().tcq_gemm_i8_best_parts(M, N, K))
+
+
 def gemm_bf16(a, w, out, sa=None, sw=None):
     """acc = a w^T with FP32 accumulation, a (M, K) / w (N, K) BF16; out (M, ldo) FP32 or BF16 of (acc * sa) * sw (either
     scale may be None). The W2 float path's product (Group.run_float, deploy/tcq_kernels/modules.py:117-144)."""
@@ -846,4 +851,16 @@ def gemm_i8(a, w, out, sa=None, sw=None):
         raise ValueError('gemm_i8: shapes do not match')
     call('tcq_gemm_i8', ptr(a), ptr(w), ptr(sa), ptr(sw), ptr(out), _dt(out, (0, 1, 3), 'gemm_i8 out'), out.stride(0), M, N, K,
          stream())
+    return out
+
+
+def gemm_i8_parts(a, w, parts):
+    """The exact int32 product a w^T in K parts: (parts, M, N), for post_add_norm_pre. a (M, K), w (N, K) int8."""
+    M, K = a.shape
+    N = w.shape[0]
+    _contig(a, w)
+    if w.shape[1] != K:
+        raise ValueError('gemm_i8_parts: shapes do not match')
+    out = torch.empty(parts, M, N, dtype=torch.int32, device=a.device)
+    call('tcq_gemm_i8_parts', ptr(a), ptr(w), ptr(out), N, M, N, K, parts, stream())
     return out

@@ -184,6 +184,10 @@ class Group:
                 kernels.decode(L.bits, L.t8, r)
         return W
 
+    def dense(self):
+        """The dense INT8 weight rows: the resident ones, else decoded into a workspace of this call."""
+        return self.W if self.W is not None else self.decode(torch.empty(self.Ntot, self.K, dtype=torch.int8, device=self.rs.device))
+
     # -------------------------------------------------------------------------------------------- activations
     def prep(self, x):
         """The (M, K) contiguous view of x in a dtype the rotation kernels read."""
@@ -222,11 +226,25 @@ class Group:
             parts *= 2
         return parts
 
+    def epilogue_parts(self, M, *vectors):
+        """K parts for a product whose epilogue is post_add_norm_pre with these side vectors (None: absent): k_parts' for few
+        tokens; for many, the GEMM's own estimate where the epilogue adds parts (the widths of k_parts, every vector 16-byte
+        aligned). MI355X, product + epilogue in one part / the chosen parts: 968 x 2048 x 16384 61 / 49 us, 200 tokens 40 / 24;
+        200 x 1024 x 4096 17.1 / 12.5."""
+        w = self.Ntot
+        if M <= SMALL_M:
+            return self.k_parts(M)
+        if (not FUSE['k_parts'] or w & (w - 1) or not 1024 <= w <= 16384
+                or any(t is not None and t.data_ptr() % 16 for t in (self.rs, self.sv, self.bias) + vectors)):
+            return 1
+        return kernels.gemm_i8_best_parts(M, w, self.K)
+
     def product(self, b, parts=1, pro=None):
         """INT8 activations -> FP32 z = (float(acc) * s) * rs (M, Ntot) of the exact int32 product acc: few tokens on the
         fused decode products, many tokens on the INT8 MFMA GEMM with the scaling in its epilogue (the order of tcq_post).
-        parts 2 / 4 (few tokens): the int32 K parts of acc instead, (parts, M, Ntot), for post_add_norm_pre. pro: one token
-        whose activations the decoder-layer prologue computes inside the product's launch (kernels.prologue; b unused)."""
+        parts 2 / 4 (few tokens, or epilogue_parts' choice): the int32 K parts of acc instead, (parts, M, Ntot), for
+        post_add_norm_pre. pro: one token whose activations the decoder-layer prologue computes inside the product's launch
+        (kernels.prologue; b unused)."""
         if pro is not None:                       # FP32 z after the layer prologue, int32 sums after the rotate + quantize one
             dev = self.rs.device
             layer = pro[0].acc is not None
@@ -243,7 +261,9 @@ class Group:
         M, dev = b['scale'].numel(), q.device
         if parts > 1:
             if M > SMALL_M:
-                raise ValueError(f'K parts are for at most {SMALL_M} tokens')
+                if parts != self.epilogue_parts(M):
+                    raise ValueError(f'{parts} K parts are for at most {SMALL_M} tokens')
+                return kernels.gemm_i8_parts(q, self.dense(), parts)
             acc = torch.empty(parts, M, self.Ntot, dtype=torch.int32, device=dev)
             if self.W is not None:
                 segs = [(self.W[s.col0:s.col0 + s.width], None, s.rs, acc[0, :, s.col0:]) for s in self.segments]
@@ -254,8 +274,7 @@ class Group:
             return acc
         z = torch.empty(M, self.Ntot, dtype=torch.float32, device=dev)
         if M > SMALL_M:
-            W = self.W if self.W is not None else self.decode(torch.empty(self.Ntot, self.K, dtype=torch.int8, device=dev))
-            return kernels.gemm_i8(q, W, z, sa=b['scale'], sw=self.rs)
+            return kernels.gemm_i8(q, self.dense(), z, sa=b['scale'], sw=self.rs)
         if self.W is not None:
             segs = [(self.W[s.col0:s.col0 + s.width], None, s.rs, z[:, s.col0:]) for s in self.segments]
             kernels.gemm_w8_segments(segs, q, b['scale'], self.Ntot)
@@ -648,7 +667,7 @@ class KDecoderLayer(torch.nn.Module):
                                                   q4=b2['q4'])
                 else:
                     b2 = og.quantize(og.prep(self.self_attn.core(q, k, v, cache_k, cache_v, causal_offset)))
-                z = og.product(b2, og.k_parts(M))
+                z = og.product(b2, og.epilogue_parts(M, x2, n2.weight, gu.su))
         x3 = torch.empty_like(x2)
         if self._prologue_fits(z, og, gu):
             # one token: the o epilogue + residual + norm2 + rotate + quantize run inside the gate | up product's launch
@@ -659,7 +678,8 @@ class KDecoderLayer(torch.nn.Module):
             b3 = gu.buffers(M, dev)
             kernels.post_add_norm_pre(z, *self._unscaled(z, b2, og), og.sv, og.bias, x2, x3, n2.weight, n2.eps, gu.su, q=b3['q'],
                                       q4=b3['q4'], scale=b3['scale'])
-            z4, b4 = gu.gated_down(b3, dn, dn.k_parts(M))
+            side = (self._next[0].input_layernorm.weight, self._next[0].groups[0].su) if (self._next and FUSE['chain']) else ()
+            z4, b4 = gu.gated_down(b3, dn, dn.epilogue_parts(M, *side))
         x4 = torch.empty_like(x2)
         nxt = self._next[0] if (self._next and FUSE['chain']) else None
         if nxt is None:
