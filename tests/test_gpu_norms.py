@@ -60,6 +60,33 @@ def test_norm_pre_bitexact(M, K):
     assert np.array_equal(q.cpu().numpy(), qr) and np.array_equal(s.cpu().numpy(), sr[:, 0])
 
 
+@pytest.mark.parametrize('M,K', [(1, 16), (7, 1040), (968, 1024), (65, 2048), (3, 4096), (2, 8192)])
+@pytest.mark.parametrize('off', [0, 1])
+def test_norms_in_registers_match_lds(M, K, off):
+    """Rows in registers (16-byte aligned; off = 0) and on the LDS path (off = 1 element) give the oracle's bits: rmsnorm at
+    partial waves, norm_pre at each register width and beyond, with q, token blocks and words."""
+    from yanlongvla_amd import kernels as Kn
+    rng = np.random.default_rng(M + 2 * K)
+    x = O.bf16_bits(rng.standard_normal((M, K)).astype(np.float32))
+    w = O.bf16_bits(rng.standard_normal(K).astype(np.float32) * 0.2)
+    su = signs(rng, K)
+    xb = torch.zeros(M * K + 8, dtype=torch.bfloat16, device=DEV)[off:off + M * K].view(M, K)
+    xb.copy_(bf16_dev(x))
+    y = torch.empty(M, K, dtype=torch.bfloat16, device=DEV)
+    Kn.rmsnorm(xb, bf16_dev(w), 1e-6, y)
+    n = O.rmsnorm_bf16(O.bf16_to_f32(x), w, 1e-6)
+    assert np.array_equal(bits_of(y), n)
+    qr, sr = O.quantize_tokens(O.fwht(O.bf16_to_f32(n) * su.astype(np.float32)))
+    s = torch.empty(M, dtype=torch.float32, device=DEV)
+    q = torch.empty(M, K, dtype=torch.int8, device=DEV)
+    blocks, words = Kn.token_blocks(M, K, DEV), torch.empty(K // 4, M, dtype=torch.int32, device=DEV)
+    Kn.norm_pre(xb, bf16_dev(w), 1e-6, T(su), q=q, q4=blocks, scale=s)
+    assert np.array_equal(q.cpu().numpy(), qr) and np.array_equal(s.cpu().numpy(), sr[:, 0])
+    assert torch.equal(Kn.rows_of_token_blocks(blocks, M), q)
+    Kn.norm_pre(xb, bf16_dev(w), 1e-6, T(su), q4=words, scale=s)
+    assert np.array_equal(words.cpu().numpy().T.copy().view(np.int8).reshape(M, K), qr)
+
+
 @pytest.mark.parametrize('M,N,parts', [(1, 2048, 2), (50, 1024, 4), (3, 4096, 2), (2, 8192, 4), (1, 16384, 2)])
 def test_post_add_norm_pre_k_parts(M, N, parts):
     """int32 K parts in: the same outputs as their int32 sum in one accumulator (register + transpose engine up to 4096,
