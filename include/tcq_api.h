@@ -387,6 +387,15 @@ int tcq_gemm_tcq(const tcq_gemm_seg* segs, int nseg, const int8_t* q, const floa
  * k_gemm_w8 / k_gemm_w8d (deploy/tcq_kernels/kernels.py:365-399, 662-668). */
 int tcq_gemm_w8(const tcq_gemm_seg* segs, int nseg, const int8_t* q, const float* s, int M, int K, int out_dtype, int ldo,
                 tcq_stream_t stream);
+/* These products with the epilogue of one-sided layers (tcq_post with sv NULL): segment i's (M, m) contiguous BF16 output is the
+ * BF16 rounding of (float(acc) * s) * rs, plus bias[i] where that is not NULL. bias: HOST array of nseg pointers to (m,) FP32,
+ * 16-byte aligned. flags: 0, TCQ_Q_TOKEN_BLOCKS, TCQ_DOT4. No reference counterpart: the product and its epilogue in one launch. */
+int tcq_gemm_tcq_bias(const tcq_gemm_seg* segs, int nseg, const float* const* bias, const int8_t* q, const float* s, int M, int K,
+                      int flags, tcq_stream_t stream);
+int tcq_gemm_w8_bias(const tcq_gemm_seg* segs, int nseg, const float* const* bias, const int8_t* q, const float* s, int M, int K,
+                     int flags, tcq_stream_t stream);
+/* tcq_post with sv NULL for up to TCQ_MAX_SEGS layers side by side in one launch (segs: HOST array, sv and gelu unused). */
+int tcq_post_plain_group(const tcq_post_seg* segs, int nseg, int acc_dtype, const float* s, int y_dtype, int M, tcq_stream_t stream);
 
 /* Prologue of a one-token product, three forms. With acc: the arguments of tcq_post_add_norm_pre for M = 1 with the norm
  * (acc the previous product's int32 sums, acc_dtype TCQ_I32, optionally | TCQ_K_PARTS2 / TCQ_K_PARTS4 with part p at

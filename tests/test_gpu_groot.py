@@ -114,3 +114,56 @@ def test_groot_fit_records_load_and_run(one_sided, tmp_path):
         y = mod(inputs[key])
         want = O.reference_linear(inputs[key].float().cpu().numpy(), oracle[name])
         assert np.array_equal(y.view(torch.int16).cpu().numpy().view(np.uint16), want), name
+
+
+@pytest.mark.parametrize('M', [1, 16, 17, 50, 64])
+@pytest.mark.parametrize('widths,K', [((1536, 1536, 1536), 1536), ((6144,), 1536), ((1536,), 6144), ((32, 2048), 272), ((16,), 16384)])
+def test_bias_product_matches_product_then_plain_epilogue(widths, K, M):
+    """(acc * s) * rs + bias -> BF16 in the product's epilogue, resident and decoded on the fly, rows and token blocks, on every
+    plan: the bits of the FP32 product, torch's FP32 add and its BF16 rounding; tcq_post_plain_group the same."""
+    from yanlongvla_amd import kernels as Kn
+    g = torch.Generator(device='cuda').manual_seed(M + K + sum(widths))
+    r = lambda *s: torch.rand(*s, generator=g, device='cuda')
+    i8 = lambda *s: torch.randint(-127, 128, s, generator=g, device='cuda', dtype=torch.int8)
+    q, s = i8(M, K), r(M) + 0.01
+    blocks = Kn.token_blocks(M, K, 'cuda')
+    pad = torch.zeros(16 * blocks.shape[0], K, dtype=torch.int8, device='cuda')
+    pad[:M] = q
+    blocks.copy_(pad.view(-1, 16, K // 16, 16).permute(0, 2, 1, 3))
+    ws, rss = [i8(n, K) for n in widths], [r(n) + 0.01 for n in widths]
+    bias = [None if i == 1 else r(n) - 0.5 for i, n in enumerate(widths)]
+    fly = []
+    for n in widths:
+        bits = torch.randint(-32768, 32768, (n // 16, K // 16, 32), generator=g, device='cuda', dtype=torch.int16)
+        fly.append((Kn.repack(bits, n, K), i8(512, 2)))
+    z = torch.empty(M, sum(widths), device='cuda')
+    for resident in (True, False):
+        c = [sum(widths[:i]) for i in range(len(widths))]
+        w = [(a, None) for a in ws] if resident else fly
+        (Kn.gemm_w8_segments if resident else Kn.gemm_tcq_segments)([(*a, rs, z[:, c0:]) for a, rs, c0 in zip(w, rss, c)], q, s, z.shape[1])
+        want = [(z[:, c0:c0 + n] if b is None else z[:, c0:c0 + n] + b).bfloat16() for c0, n, b in zip(c, widths, bias)]
+        for act in (q, blocks):
+            ys = [torch.empty(M, n, dtype=torch.bfloat16, device='cuda') for n in widths]
+            Kn.gemm_bias_segments([(*a, rs, b, y) for a, rs, b, y in zip(w, rss, bias, ys)], act, s, resident=resident)
+            assert all(torch.equal(y, v) for y, v in zip(ys, want))
+        ys = [torch.empty(M, n, dtype=torch.bfloat16, device='cuda') for n in widths]
+        Kn.post_plain_group([(z, c0, None, b, y) for c0, b, y in zip(c, bias, ys)], torch.float32, torch.bfloat16, None, M)
+        assert all(torch.equal(y, v) for y, v in zip(ys, want))
+
+
+@pytest.mark.parametrize('adt', [torch.int32, torch.float32, torch.bfloat16])
+@pytest.mark.parametrize('ydt', [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('M,N,col0', [(3, 1024, 4), (70, 1028, 8), (5, 1030, 3), (2, 1, 0)])
+def test_plain_epilogue_bitexact(adt, ydt, M, N, col0):
+    """One-sided epilogues in wide accesses and, where columns or widths are not multiples of four, element by element."""
+    from yanlongvla_amd import kernels as Kn
+    g = torch.Generator(device='cuda').manual_seed(M + N)
+    lda = N + 8 + (0 if N % 4 == 0 else 1)
+    acc = torch.randint(-2 ** 20, 2 ** 20, (M, lda), generator=g, device='cuda', dtype=torch.int32)
+    acc = acc if adt == torch.int32 else (acc.float() * 1e-4).to(adt)
+    s, rs, bias = (torch.rand(n, generator=g, device='cuda') * 1e-3 for n in (M, N, N))
+    y = torch.empty(M, N, dtype=ydt, device='cuda')
+    Kn.post(acc, s if adt == torch.int32 else None, None if adt == torch.float32 else rs, None, bias, y, col0=col0)
+    z = acc[:, col0:col0 + N].float()
+    z = (z * s[:, None]) * rs if adt == torch.int32 else z if adt == torch.float32 else z * rs
+    assert torch.equal(y, (z + bias).to(ydt))

@@ -62,8 +62,10 @@ __device__ __forceinline__ int4v dot_to_mfma_layout(int v, int lane) {
 
 }  // namespace
 
+// bias: FP32 bias of each segment's rows or NULL (BF16 outputs)
 struct SegPack {
     tcq_gemm_seg s[TCQ_MAX_SEGS];
+    const float* bias[TCQ_MAX_SEGS];
 };
 
 // The segments plus the arguments of a one-token prologue (tcq_gemm_tcq_pro / tcq_gemm_w8_pro).
@@ -143,7 +145,7 @@ enum { QL_ROWS = 0, QL_BLOCKS = 1, QL_WORDS = 2 };
 // grid (tile-row groups of the largest segment, segments), NW = blockDim.x / 64 waves; a workgroup takes TR consecutive tile
 // rows (the activation fragments of its chunks, the bulk of the loads, then serve TR rows). MODE 0: decode from tcq_repack
 // words (RB: from the reference word layout, 64 bytes per tile, tiles row-major); MODE 1: resident INT8 weights. ODT: output
-// dtype (F32 scaled, BF16 scaled, I32 accumulators). QL: activation layout (ldq only for QL_WORDS).
+// dtype (F32 scaled; BF16 scaled, plus the segment's bias, with rows ldz apart or, for ldz 0, contiguous; I32 accumulators). QL: activation layout (ldq only for QL_WORDS).
 // KS > 1 (I32 only): K parts, blockIdx.z = part p takes chunks [p * ceil(nch / KS), ...) and writes at out + p * M * ldz.
 // DOT (M == 1): the product on v_dot4c_i32_i8 (dot_product) instead of the MFMA; the epilogues are shared.
 // PL > 0 (M == 1, K = 2^PL): the activations come from the prologue run by every workgroup (run_prologue, ProShape)
@@ -256,7 +258,11 @@ __global__ __launch_bounds__(TR == 1 ? 1024 : 512) void k_gemm_small(const typen
     if (!PL && c0 + wave < nch) load(c0 + wave);
     if (OVS && pw >= 0 && c0 + pw < nch) load(c0 + pw);
     // epilogue scales, loaded with the operands (wave 0 stores; OVS: wave 8)
-    float4_t rsv[TR];
+    constexpr bool BIAS = ODT == TCQ_BF16 && !PL;
+    const float* bias = nullptr;
+    if constexpr (BIAS) bias = P.bias[blockIdx.y];
+    const int ld = BIAS && !ldz ? S.m : ldz;
+    float4_t rsv[TR], bv[BIAS ? TR : 1];
     float sv[NB];
 #pragma unroll
     for (int r = 0; r < TR; ++r) rsv[r] = float4_t{0.f, 0.f, 0.f, 0.f};
@@ -265,6 +271,11 @@ __global__ __launch_bounds__(TR == 1 ? 1024 : 512) void k_gemm_small(const typen
     if (ODT != TCQ_I32 && pw == 0) {
 #pragma unroll
         for (int r = 0; r < TR; ++r) rsv[r] = gptr((const float4_t*)(S.rs + 16 * min(I0 + r, tiles_m - 1) + 4 * lg))[0];
+        if constexpr (BIAS) {
+#pragma unroll
+            for (int r = 0; r < TR; ++r)
+                if (bias) bv[r] = gptr((const float4_t*)(bias + 16 * min(I0 + r, tiles_m - 1) + 4 * lg))[0];
+        }
         if constexpr (!PL) {
 #pragma unroll
             for (int b = 0; b < NB; ++b) sv[b] = gptr(s)[min(16 * b + lr, M - 1)];
@@ -394,7 +405,7 @@ __global__ __launch_bounds__(TR == 1 ? 1024 : 512) void k_gemm_small(const typen
         for (int b = 0; b < NB; ++b) {
             const int t = 16 * b + lr;
             if (t < M) {
-                const size_t o = (size_t)t * ldz + 16 * I + 4 * lg;
+                const size_t o = (size_t)t * ld + 16 * I + 4 * lg;
                 if (ODT == TCQ_I32) {
                     *gptr((int4v*)((int*)S.out + (KS > 1 ? (size_t)blockIdx.z * M * ldz : 0) + o)) = acc[r][b];
                 } else {
@@ -405,6 +416,9 @@ __global__ __launch_bounds__(TR == 1 ? 1024 : 512) void k_gemm_small(const typen
                     if (ODT == TCQ_F32) {
                         *gptr((float4_t*)((float*)S.out + o)) = float4_t{v[0], v[1], v[2], v[3]};
                     } else {
+                        if (BIAS && bias)
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) v[e] = v[e] + bv[BIAS ? r : 0][e];
                         const u32 lo = bf16x2(v[0], v[1]);
                         const u32 hi = bf16x2(v[2], v[3]);
                         *gptr((u64*)((u16*)S.out + o)) = (u64)lo | ((u64)hi << 32);
@@ -494,10 +508,14 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_tcq(const typename PackOf<PL>:
     };
     int4v Bf[2][4];                                                        // activation fragments, two chunks in turn
     if constexpr (!PL) loadB(c0 + part, Bf[0]);
-    float4_t rsv = float4_t{0.f, 0.f, 0.f, 0.f};
+    constexpr bool BIAS = ODT == TCQ_BF16 && !PL;
+    const float* bias = nullptr;
+    if constexpr (BIAS) bias = P.bias[blockIdx.y];
+    float4_t rsv = float4_t{0.f, 0.f, 0.f, 0.f}, bv = rsv;
     float sv = 0.f;
     if (ODT != TCQ_I32 && part == 0) {
         rsv = gptr((const float4_t*)(S.rs + 16 * I + 4 * lg))[0];
+        if (BIAS && bias) bv = gptr((const float4_t*)(bias + 16 * I + 4 * lg))[0];
         if constexpr (!PL) sv = gptr(s)[min(lr, M - 1)];
     }
     // the table, filled by threads from t0 on (OV: the decode waves alone; the prologue waves start at once)
@@ -649,7 +667,7 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_tcq(const typename PackOf<PL>:
     if (I0 + slot >= tiles_m) return;
     const int t = lr;
     if (t >= M) return;
-    const size_t o = (size_t)t * ldz + 16 * I + 4 * lg;
+    const size_t o = (size_t)t * (BIAS && !ldz ? S.m : ldz) + 16 * I + 4 * lg;
     if (ODT == TCQ_I32) {
         *gptr((int4v*)((int*)S.out + (KS > 1 ? (size_t)blockIdx.z * M * ldz : 0) + o)) = acc;
     } else {
@@ -659,6 +677,9 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_tcq(const typename PackOf<PL>:
         if (ODT == TCQ_F32) {
             *gptr((float4_t*)((float*)S.out + o)) = float4_t{v[0], v[1], v[2], v[3]};
         } else {
+            if (BIAS && bias)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = v[e] + bv[e];
             const u32 lo = bf16x2(v[0], v[1]);
             const u32 hi = bf16x2(v[2], v[3]);
             *gptr((u64*)((u16*)S.out + o)) = (u64)lo | ((u64)hi << 32);
@@ -772,8 +793,8 @@ static int gv_waves_per_row(const tcq_gemm_seg* segs, int nseg, int M, int nch, 
 
 template <int MODE>
 static int gemm_small(const tcq_gemm_seg* segs, int nseg, const int8_t* q, const float* s, int M, int K, int odt, int ldo,
-                      tcq_stream_t stream) {
-    if (!segs || !q || nseg <= 0 || M <= 0 || K <= 0 || ldo <= 0) return TCQ_ERR_ARG;
+                      tcq_stream_t stream, const float* const* bias = nullptr) {
+    if (!segs || !q || nseg <= 0 || M <= 0 || K <= 0 || (bias ? ldo != 0 : ldo <= 0)) return TCQ_ERR_ARG;
     const bool qb = odt & TCQ_Q_TOKEN_BLOCKS;                          // q in the token-block layout
     if ((odt & TCQ_K_PARTS2) && (odt & TCQ_K_PARTS4)) return TCQ_ERR_ARG;
     const int parts = (odt & TCQ_K_PARTS4) ? 4 : (odt & TCQ_K_PARTS2) ? 2 : 1;
@@ -798,6 +819,8 @@ static int gemm_small(const tcq_gemm_seg* segs, int nseg, const int8_t* q, const
         const size_t osz = odt == TCQ_BF16 ? 2 : 4;
         if ((uintptr_t)g.out % (4 * osz) || (g.rs && (uintptr_t)g.rs % 16)) return TCQ_ERR_ALIGN;
         P.s[i] = g;
+        if (bias && (uintptr_t)bias[i] % 16) return TCQ_ERR_ALIGN;
+        P.bias[i] = bias ? bias[i] : nullptr;
         if (g.m > max_m) max_m = g.m;
     }
     if ((size_t)M * K >= ((size_t)1 << 31)) return TCQ_ERR_SHAPE;
@@ -857,6 +880,20 @@ extern "C" int tcq_gemm_tcq(const tcq_gemm_seg* segs, int nseg, const int8_t* q,
 extern "C" int tcq_gemm_w8(const tcq_gemm_seg* segs, int nseg, const int8_t* q, const float* s, int M, int K, int out_dtype, int ldo,
                            tcq_stream_t stream) {
     return gemm_small<1>(segs, nseg, q, s, M, K, out_dtype, ldo, stream);
+}
+
+static int bias_flags_bad(int flags) { return flags & ~(TCQ_Q_TOKEN_BLOCKS | TCQ_DOT4); }
+
+extern "C" int tcq_gemm_tcq_bias(const tcq_gemm_seg* segs, int nseg, const float* const* bias, const int8_t* q, const float* s, int M,
+                                 int K, int flags, tcq_stream_t stream) {
+    if (!bias || bias_flags_bad(flags)) return TCQ_ERR_ARG;
+    return gemm_small<0>(segs, nseg, q, s, M, K, TCQ_BF16 | flags, 0, stream, bias);
+}
+
+extern "C" int tcq_gemm_w8_bias(const tcq_gemm_seg* segs, int nseg, const float* const* bias, const int8_t* q, const float* s, int M,
+                                int K, int flags, tcq_stream_t stream) {
+    if (!bias || bias_flags_bad(flags)) return TCQ_ERR_ARG;
+    return gemm_small<1>(segs, nseg, q, s, M, K, TCQ_BF16 | flags, 0, stream, bias);
 }
 
 // ------------------------------------------------------------------------------------ products with the layer prologue

@@ -1569,33 +1569,74 @@ extern "C" int tcq_quantize_rows(const void* x, int x_dtype, int ldx, int8_t* q,
     return launch_status();
 }
 
-// Epilogue of a one-sided layer (no output rotation, the GR00T "tcq" base): y[t, i] = SCALE(acc[t, col0 + i]) (+ bias[i]),
-// SCALE as in k_post. grid (ceil(N / 256), M), one element per thread.
+// Epilogue of one-sided layers (no output rotation, the GR00T "tcq" base): y[t, i] = SCALE(acc[t, col0 + i]) (+ bias[i]),
+// SCALE as in k_post. grid (ceil(max N / 1024), M, segments), four elements per thread, in 16-byte accesses where the segment is
+// aligned (vec, per segment). One launch per group and wide accesses: MI355X, q | k | v of 1536 at 50 tokens 5.6 -> 2.8 us, at 400 7.8 -> 3.2.
 template <int ADT, int YDT>
-__global__ __launch_bounds__(256) void k_post_plain(const void* acc, int lda, int col0, const float* s, const float* rs,
-                                                    const float* bias, void* y, int N) {
-    const int i = blockIdx.x * 256 + threadIdx.x, tok = blockIdx.y;
-    if (i >= N) return;
-    const size_t a = (size_t)tok * lda + col0 + i;
-    float z;
-    if constexpr (ADT == TCQ_I32) z = ((float)gptr((const int*)acc)[a] * gptr(s)[tok]) * gptr(rs)[i];
-    else if constexpr (ADT == TCQ_BF16) z = bf16_to_f32(gptr((const u16*)acc)[a]) * gptr(rs)[i];
-    else z = gptr((const float*)acc)[a];
-    if (bias) z = z + gptr(bias)[i];
-    const size_t o = (size_t)tok * N + i;
-    if constexpr (YDT == TCQ_F32) gptr((float*)y)[o] = z;
-    else if constexpr (YDT == TCQ_BF16) gptr((u16*)y)[o] = f32_to_bf16(z);
-    else gptr((u16*)y)[o] = f32_to_f16(z);
+__global__ __launch_bounds__(256) void k_post_plain(const PostPack segs, const float* s, u32 vec) {
+    const tcq_post_seg& S = segs[blockIdx.z];
+    const int i0 = blockIdx.x * 1024 + 4 * threadIdx.x, tok = blockIdx.y;
+    if (i0 >= S.N) return;
+    const size_t a = (size_t)tok * S.lda + S.col0 + i0, o = (size_t)tok * S.N + i0;
+    const float st = ADT == TCQ_I32 ? gptr(s)[tok] : 1.f;
+    auto scaled = [&](float x, float r) { return ADT == TCQ_I32 ? (x * st) * r : ADT == TCQ_BF16 ? x * r : x; };
+    if (vec >> blockIdx.z & 1) {
+        float z[4];
+        float4_t r = {1.f, 1.f, 1.f, 1.f}, b = {0.f, 0.f, 0.f, 0.f};
+        if (ADT != TCQ_F32) r = *gptr((const float4_t*)(S.rs + i0));
+        if (S.bias) b = *gptr((const float4_t*)(S.bias + i0));
+        if constexpr (ADT == TCQ_BF16) {
+            const uint2_t x = *gptr((const uint2_t*)((const u16*)S.acc + a));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) z[e] = bf16_to_f32((u16)(x[e >> 1] >> (16 * (e & 1))));
+        } else {
+            const uint4_t x = *gptr((const uint4_t*)((const u32*)S.acc + a));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) z[e] = ADT == TCQ_I32 ? (float)(int)x[e] : __uint_as_float(x[e]);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            z[e] = scaled(z[e], r[e]);
+            if (S.bias) z[e] = z[e] + b[e];
+        }
+        if constexpr (YDT == TCQ_F32) *gptr((float4_t*)((float*)S.y + o)) = float4_t{z[0], z[1], z[2], z[3]};
+        else
+            *gptr((uint2_t*)((u16*)S.y + o)) = uint2_t{f32_to_bits<YDT>(z[0]) | (f32_to_bits<YDT>(z[1]) << 16),
+                                                       f32_to_bits<YDT>(z[2]) | (f32_to_bits<YDT>(z[3]) << 16)};
+        return;
+    }
+    for (int e = 0; e < 4 && i0 + e < S.N; ++e) {
+        float z;
+        if constexpr (ADT == TCQ_I32) z = (float)gptr((const int*)S.acc)[a + e];
+        else if constexpr (ADT == TCQ_BF16) z = bf16_to_f32(gptr((const u16*)S.acc)[a + e]);
+        else z = gptr((const float*)S.acc)[a + e];
+        z = scaled(z, ADT == TCQ_F32 ? 1.f : gptr(S.rs)[i0 + e]);
+        if (S.bias) z = z + gptr(S.bias)[i0 + e];
+        if constexpr (YDT == TCQ_F32) gptr((float*)S.y)[o + e] = z;
+        else gptr((u16*)S.y)[o + e] = (u16)f32_to_bits<YDT>(z);
+    }
 }
 
-extern "C" int tcq_post(const void* acc, int acc_dtype, int lda, int col0, const float* s, const float* rs, const int8_t* sv,
-                        const float* bias, void* y, int y_dtype, int M, int N, tcq_stream_t stream) {
-    if (!acc || !y || M <= 0 || N <= 0 || col0 < 0 || lda < col0 + N) return TCQ_ERR_ARG;
-    if ((acc_dtype == TCQ_I32 && (!s || !rs)) || (acc_dtype == TCQ_BF16 && !rs)) return TCQ_ERR_ARG;
-    if (!sv) {                                                   // one-sided layer: no output rotation
-        const dim3 grid((N + 255) / 256, M);
-        hipStream_t st = (hipStream_t)stream;
-#define PLAIN_Y(AD, YD) launch_k(k_post_plain<AD, YD>, grid, dim3(256), 0, st, acc, lda, col0, s, rs, bias, y, N)
+extern "C" int tcq_post_plain_group(const tcq_post_seg* segs, int nseg, int acc_dtype, const float* s, int y_dtype, int M,
+                                    tcq_stream_t stream) {
+    if (!segs || nseg <= 0 || nseg > TCQ_MAX_SEGS || M <= 0) return TCQ_ERR_ARG;
+    if (acc_dtype == TCQ_I32 && !s) return TCQ_ERR_ARG;
+    PostPack pk = {};
+    u32 vec = 0;
+    int maxN = 0;
+    for (int i = 0; i < nseg; ++i) {
+        const tcq_post_seg& g = segs[i];
+        if (!g.acc || !g.y || g.N <= 0 || g.col0 < 0 || g.lda < g.col0 + g.N || (acc_dtype != TCQ_F32 && !g.rs)) return TCQ_ERR_ARG;
+        const size_t as = acc_dtype == TCQ_BF16 ? 8 : 16, ys = y_dtype == TCQ_F32 ? 16 : 8;
+        if (g.N % 4 == 0 && g.lda % 4 == 0 && g.col0 % 4 == 0 && (uintptr_t)g.acc % as == 0 && (uintptr_t)g.y % ys == 0 &&
+            (acc_dtype == TCQ_F32 || al16(g.rs)) && (!g.bias || al16(g.bias)))
+            vec |= 1u << i;
+        pk.s[i] = g;
+        if (g.N > maxN) maxN = g.N;
+    }
+    const dim3 grid((maxN + 1023) / 1024, M, nseg);
+    hipStream_t st = (hipStream_t)stream;
+#define PLAIN_Y(AD, YD) launch_k(k_post_plain<AD, YD>, grid, dim3(256), 0, st, pk, s, vec)
 #define PLAIN_A(AD)                                          \
     switch (y_dtype) {                                       \
         case TCQ_F32: PLAIN_Y(AD, TCQ_F32); break;           \
@@ -1603,15 +1644,24 @@ extern "C" int tcq_post(const void* acc, int acc_dtype, int lda, int col0, const
         case TCQ_F16: PLAIN_Y(AD, TCQ_F16); break;           \
         default: return TCQ_ERR_DTYPE;                       \
     }
-        switch (acc_dtype) {
-            case TCQ_I32: PLAIN_A(TCQ_I32); break;
-            case TCQ_F32: PLAIN_A(TCQ_F32); break;
-            case TCQ_BF16: PLAIN_A(TCQ_BF16); break;
-            default: return TCQ_ERR_DTYPE;
-        }
+    switch (acc_dtype) {
+        case TCQ_I32: PLAIN_A(TCQ_I32); break;
+        case TCQ_F32: PLAIN_A(TCQ_F32); break;
+        case TCQ_BF16: PLAIN_A(TCQ_BF16); break;
+        default: return TCQ_ERR_DTYPE;
+    }
 #undef PLAIN_A
 #undef PLAIN_Y
-        return launch_status();
+    return launch_status();
+}
+
+extern "C" int tcq_post(const void* acc, int acc_dtype, int lda, int col0, const float* s, const float* rs, const int8_t* sv,
+                        const float* bias, void* y, int y_dtype, int M, int N, tcq_stream_t stream) {
+    if (!acc || !y || M <= 0 || N <= 0 || col0 < 0 || lda < col0 + N) return TCQ_ERR_ARG;
+    if ((acc_dtype == TCQ_I32 && (!s || !rs)) || (acc_dtype == TCQ_BF16 && !rs)) return TCQ_ERR_ARG;
+    if (!sv) {                                                   // one-sided layer: no output rotation
+        const tcq_post_seg seg = {acc, rs, nullptr, bias, y, lda, col0, N, 0};
+        return tcq_post_plain_group(&seg, 1, acc_dtype, s, y_dtype, M, stream);
     }
     if (N > TCQ_MAX_WIDTH) return TCQ_ERR_SHAPE;
     const int asz = dsize(acc_dtype);

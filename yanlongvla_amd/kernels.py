@@ -505,6 +505,22 @@ def postg(acc, s, rs, sv, bias, ys, gelu0=False):
          ptr(ys[0]), ptr(ys[1]), ptr(y2), M, n[0], n[1], n2, acc.shape[1], int(bool(gelu0)), stream())
 
 
+def post_plain_group(segs, acc_dtype, y_dtype, s, M):
+    """post with sv None for up to MAX_SEGS segments [(acc, col0, rs, bias, y), ...] in one launch."""
+    if not 0 < len(segs) <= _lib.MAX_SEGS:
+        raise ValueError(f'post_plain_group takes 1..{_lib.MAX_SEGS} segments, got {len(segs)}')
+    arr = (_lib.PostSeg * len(segs))()
+    for i, (acc, col0, rs, bias, y) in enumerate(segs):
+        _contig(acc, rs, bias, y)
+        N = y.shape[1]
+        if col0 < 0 or col0 + N > acc.shape[1] or acc.shape[0] < M or any(t is not None and t.numel() != N for t in (rs, bias)):
+            raise ValueError(f'segment {i}: columns {col0}..{col0 + N} do not fit the accumulator / scales')
+        if y.dtype != y_dtype or acc.dtype != acc_dtype or y.shape[0] != M:
+            raise TypeError(f'segment {i}: dtypes or rows differ from the group\'s')
+        arr[i] = _lib.PostSeg(ptr(acc), ptr(rs), None, ptr(bias), ptr(y), acc.shape[1], col0, N, 0)
+    call('tcq_post_plain_group', arr, len(segs), DTYPE[acc_dtype], ptr(s), DTYPE[y_dtype], M, stream())
+
+
 def post_group(segs, acc_dtype, y_dtype, s, M, gelu_lut=None):
     """Epilogue of one layer group, at most MAX_SEGS segments [(acc, col0, rs, sv, bias, y, gelu), ...] as in post_segments,
     passed by value in the launch (reference kernels.post3 / postg as Group.posts calls them, kernels.py:618-628): every call
@@ -672,6 +688,22 @@ def gemm_tcq_segments(segs, q, s, ldo, parts=1, dot=None):
     """One-shot fused decode + product over segments (see SmallProduct)."""
     _contig(q, s)
     SmallProduct(segs, ldo)(q, s, parts, dot)
+
+
+def gemm_bias_segments(segs, q, s, resident=False):
+    """The small-M product with the epilogue of one-sided layers: segments [(w, t8, rs, bias, y), ...], y (M, m) contiguous BF16 =
+    bf16((acc * s) * rs + bias); bias (m,) FP32, 16-byte aligned, or None. q, s and resident as in SmallProduct."""
+    p = SmallProduct([(w, t8, rs, y) for w, t8, rs, _, y in segs], 0, resident)
+    _contig(q, s)
+    M, K, flags = (s.numel(), q.shape[1] * 16, Q_TOKEN_BLOCKS) if q.dim() == 4 else (*q.shape, 0)
+    if (p.K is not None and K != p.K) or s.numel() < M:
+        raise ValueError('gemm_bias_segments: activations, weights and token scales do not match')
+    for _, _, rs, bias, y in segs:
+        _contig(bias, y)
+        if y.dtype != torch.bfloat16 or y.shape != (M, rs.numel()) or (bias is not None and bias.numel() != rs.numel()):
+            raise ValueError(f'gemm_bias_segments: output {tuple(y.shape)} {y.dtype}: expected ({M}, {rs.numel()}) BF16')
+    bias = (ctypes.c_void_p * len(segs))(*[ptr(b) for _, _, _, b, _ in segs])
+    call(p.name + '_bias', p.arr, p.n, bias, ptr(q), ptr(s), M, K, flags | _dot_flag(M, None), stream())
 
 
 def gemm_w8_segments(segs, q, s, ldo, parts=1, dot=None):

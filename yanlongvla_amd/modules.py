@@ -352,11 +352,11 @@ class Group:
             ys.append(y)
         scaled = acc.dtype == torch.float32
         s_tok = b['scale'] if acc.dtype == torch.int32 else None
-        if self.one_sided:                        # no output rotation: one plain epilogue per member
+        if self.one_sided:                        # no output rotation: one plain epilogue for all members
             if gelu0:
                 raise ValueError('one-sided groups have no fused GELU epilogue')
-            for s, y in zip(self.segments, ys):
-                kernels.post(acc, s_tok, None if scaled else s.rs, None, s.bias, y, col0=s.col0)
+            kernels.post_plain_group([(acc, s.col0, None if scaled else s.rs, s.bias, y) for s, y in zip(self.segments, ys)],
+                                     acc.dtype, torch.bfloat16, s_tok, M)
         else:
             segs = [(acc, s.col0, None if scaled else s.rs, s.sv, s.bias, y, gelu0 and i == 0)
                     for i, (s, y) in enumerate(zip(self.segments, ys))]
@@ -364,13 +364,28 @@ class Group:
                                gelu_lut=kernels.gelu_table(dev) if gelu0 else None)
         return [y.reshape(*shape[:-1], s.width) for s, y in zip(self.segments, ys)]
 
+    def plain(self, b, shape):
+        """A one-sided group's outputs for few tokens: scaling, bias and BF16 rounding in the product's own epilogue, with the
+        bits of product + posts. MI355X, 50 tokens: a launch of 2.5 us less per projection."""
+        q, M = (b['q'] if b['q'] is not None else b['q4']), b['scale'].numel()
+        ys = [torch.empty(M, s.width, dtype=torch.bfloat16, device=q.device) for s in self.segments]
+        if self.W is not None:
+            segs = [(self.W[s.col0:s.col0 + s.width], None, s.rs, s.bias, y) for s, y in zip(self.segments, ys)]
+        else:
+            segs = [(L.words(), L.t8, s.rs, s.bias, y) for L, s, y in zip(self.layers, self.segments, ys)]
+        kernels.gemm_bias_segments(segs, q, b['scale'], resident=self.W is not None)
+        return [y.reshape(*shape[:-1], y.shape[1]) for y in ys]
+
     # --------------------------------------------------------------------------------------------------- runs
     def run(self, x):
         """All members' outputs for input x."""
         x2 = self.prep(x)
         if self.a8:
             b = self.quantize(x2)
-            outs = self.posts(self.product(b), b, x.shape)
+            if self.one_sided and x2.shape[0] <= SMALL_M and all(s.bias is None or s.bias.data_ptr() % 16 == 0 for s in self.segments):
+                outs = self.plain(b, x.shape)
+            else:
+                outs = self.posts(self.product(b), b, x.shape)
         else:
             outs = self.run_float(x2, x.shape)
         STATS['group_runs'] += 1
