@@ -394,6 +394,9 @@ int tcq_gemm_tcq_bias(const tcq_gemm_seg* segs, int nseg, const float* const* bi
                       int flags, tcq_stream_t stream);
 int tcq_gemm_w8_bias(const tcq_gemm_seg* segs, int nseg, const float* const* bias, const int8_t* q, const float* s, int M, int K,
                      int flags, tcq_stream_t stream);
+/* tcq_gemm_w8 at M <= 16 tokens with the stage-split FP32 output of TCQ_Z_W128T (segment rows a multiple of 128, K <= 4096; flags: 0 or
+ * TCQ_Q_TOKEN_BLOCKS). No reference counterpart. */
+int tcq_gemm_w8_w128t(const tcq_gemm_seg* segs, int nseg, const int8_t* q, const float* s, int M, int K, int flags, tcq_stream_t stream);
 /* tcq_post with sv NULL for up to TCQ_MAX_SEGS layers side by side in one launch (segs: HOST array, sv and gelu unused). */
 int tcq_post_plain_group(const tcq_post_seg* segs, int nseg, int acc_dtype, const float* s, int y_dtype, int M, tcq_stream_t stream);
 

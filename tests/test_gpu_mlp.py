@@ -232,3 +232,30 @@ def test_spread_middle_equals_mid2_and_oracle(M):
     qr, sr, _, _ = O.mlp_middle(zz[:, :N], zz[:, N:], sv.cpu().numpy()[:N], sv.cpu().numpy()[N:], su.cpu().numpy(),
                                 gelu=lambda b: lut_h[b])
     assert np.array_equal(K.rows_of_token_blocks(q2, M).cpu().numpy(), qr) and np.array_equal(s2.cpu().numpy(), sr[:, 0])
+
+
+@pytest.mark.parametrize('M', [1, 3, 16])
+@pytest.mark.parametrize('K', [16, 272, 2048, 4096])
+def test_resident_stage_split_product(M, K):
+    """gemm_w8_w128t: zt equals the resident product's z after Walsh stages h = 1 .. 64 inside 128-row blocks, block-transposed,
+    bit for bit, from rows and token blocks, at partial chunks and more chunks than are in flight at once."""
+    from yanlongvla_amd import kernels as Kn
+    g = torch.Generator(device=DEV).manual_seed(M + K)
+    i8 = lambda *s: torch.randint(-127, 128, s, generator=g, device=DEV, dtype=torch.int8)
+    q, s, widths = i8(M, K), torch.rand(M, generator=g, device=DEV) + 0.01, (384, 128)
+    pad = torch.zeros((M + 15) // 16 * 16, K, dtype=torch.int8, device=DEV)
+    pad[:M] = q
+    blocks = pad.view(-1, 16, K // 16, 16).permute(0, 2, 1, 3).contiguous()
+    ws, rss = [i8(n, K) for n in widths], [torch.rand(n, generator=g, device=DEV) + 0.01 for n in widths]
+    for act in (q, blocks):
+        zts = [torch.full((M, 128, n // 128), float('nan'), device=DEV) for n in widths]
+        Kn.gemm_w8_w128t(list(zip(ws, rss, zts)), act, s)
+        for w, rs, zt, n in zip(ws, rss, zts, widths):
+            z = torch.empty(M, n, device=DEV)
+            Kn.gemm_w8_segments([(w, None, rs, z)], q, s, n)
+            v, h = z.cpu(), 1
+            while h < 128:
+                v = v.view(M, n // (2 * h), 2, h)
+                v = torch.stack((v[:, :, 0] + v[:, :, 1], v[:, :, 0] - v[:, :, 1]), 2)
+                h *= 2
+            assert torch.equal(zt.cpu(), v.reshape(M, n // 128, 128).transpose(1, 2))

@@ -61,6 +61,7 @@ SIGNATURES = {
     'tcq_gemm_w8': [_P, _I, _P, _P, _I, _I, _I, _I, _P],
     'tcq_gemm_tcq_bias': [_P, _I, _P, _P, _P, _I, _I, _I, _P],
     'tcq_gemm_w8_bias': [_P, _I, _P, _P, _P, _I, _I, _I, _P],
+    'tcq_gemm_w8_w128t': [_P, _I, _P, _P, _I, _I, _I, _P],
     'tcq_post_plain_group': [_P, _I, _I, _P, _I, _I, _P],
     'tcq_gemm_i8': [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
     'tcq_post3': [_P, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],

@@ -429,6 +429,54 @@ __global__ __launch_bounds__(TR == 1 ? 1024 : 512) void k_gemm_small(const typen
     }
 }
 
+// The stage-split epilogue (TCQ_Z_W128T) of a workgroup that holds one 128-row block of a segment, tile row `slot` of it in a
+// wave (in: its scaled sums are valid there; acc as the MFMA leaves them): the first seven Walsh stages of the segment and the
+// transposed store zt[(t * 128 + o) * nb + blk]. zb: M rows of 128 floats. Every wave calls it (a barrier inside); M <= waves.
+__device__ __forceinline__ void w128t_store(float* zb, int4v acc, float sv, float4_t rsv, bool in, int slot, int M, float* out, int nb,
+                                        int blk) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
+    if (in) {
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = ((float)acc[e] * sv) * rsv[e];
+        float a = v[0], b = v[1];                                      // h = 1, 2: row pairs in the lane's 4 rows
+        v[0] = a + b; v[1] = a - b;
+        a = v[2]; b = v[3];
+        v[2] = a + b; v[3] = a - b;
+        a = v[0]; b = v[2];
+        v[0] = a + b; v[2] = a - b;
+        a = v[1]; b = v[3];
+        v[1] = a + b; v[3] = a - b;
+#pragma unroll
+        for (int m = 16; m <= 32; m *= 2)                              // h = 4, 8: rows 4 lg + e, lanes 16 lg + lr
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float pv = lane_xor(v[e], m, lane);
+                v[e] = (lane & m) ? pv - v[e] : v[e] + pv;
+            }
+        if (lr < M) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) zb[lr * 128 + 16 * slot + 4 * lg + e] = v[e];
+        }
+    }
+    __syncthreads();
+    if (wave < M) {                                                    // h = 16, 32, 64: token `wave`, rows l and l + 64
+        float a = zb[wave * 128 + lane], b = zb[wave * 128 + 64 + lane];
+#pragma unroll
+        for (int m = 16; m <= 32; m *= 2) {
+            const float pa = lane_xor(a, m, lane), pb = lane_xor(b, m, lane);
+            a = (lane & m) ? pa - a : a + pa;
+            b = (lane & m) ? pb - b : b + pb;
+        }
+        const float x = a;
+        a = x + b;
+        b = x - b;
+        float* zt = out + (size_t)wave * 128 * nb;
+        gptr(zt)[(size_t)lane * nb + blk] = a;
+        gptr(zt)[(size_t)(lane + 64) * nb + blk] = b;
+    }
+}
+
 // Streaming plan of the fused decode for one token block (M <= 16) and large layers (the backbone's gate/up and down
 // products at one token: 8.5 and 8.3 us on MI355X against 10.0 and 10.4 on the workgroup plan): a workgroup takes
 // RPW = NW / WPR tile rows, WPR waves per tile row, and wave p of a row takes its chunks p, p + WPR, ... (at most CMAX).
@@ -620,48 +668,7 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_tcq(const typename PackOf<PL>:
         }
     }
     if constexpr (LO) {                                                    // every wave reaches the barrier below
-        float* zb = (float*)tab + 4096;                                    // past the reduction slots: M rows of 128
-        if (part == 0) {
-            float v[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = ((float)acc[e] * sv) * rsv[e];
-            float a = v[0], b = v[1];                                      // h = 1, 2: row pairs in the lane's 4 rows
-            v[0] = a + b; v[1] = a - b;
-            a = v[2]; b = v[3];
-            v[2] = a + b; v[3] = a - b;
-            a = v[0]; b = v[2];
-            v[0] = a + b; v[2] = a - b;
-            a = v[1]; b = v[3];
-            v[1] = a + b; v[3] = a - b;
-#pragma unroll
-            for (int m = 16; m <= 32; m *= 2)                              // h = 4, 8: rows 4 lg + e, lanes 16 lg + lr
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float pv = lane_xor(v[e], m, lane);
-                    v[e] = (lane & m) ? pv - v[e] : v[e] + pv;
-                }
-            if (lr < M) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) zb[lr * 128 + 16 * slot + 4 * lg + e] = v[e];
-            }
-        }
-        __syncthreads();
-        if (wave < M) {                                                    // h = 16, 32, 64: token `wave`, rows l and l + 64
-            float a = zb[wave * 128 + lane], b = zb[wave * 128 + 64 + lane];
-#pragma unroll
-            for (int m = 16; m <= 32; m *= 2) {
-                const float pa = lane_xor(a, m, lane), pb = lane_xor(b, m, lane);
-                a = (lane & m) ? pa - a : a + pa;
-                b = (lane & m) ? pb - b : b + pb;
-            }
-            const float x = a;
-            a = x + b;
-            b = x - b;
-            const int nb = S.m >> 7, blk = I0 >> 3;
-            float* zt = (float*)S.out + (size_t)wave * 128 * nb;
-            gptr(zt)[(size_t)lane * nb + blk] = a;
-            gptr(zt)[(size_t)(lane + 64) * nb + blk] = b;
-        }
+        w128t_store((float*)tab + 4096, acc, sv, rsv, part == 0, slot, M, (float*)S.out, S.m >> 7, I0 >> 3);   // past the reduction slots
         return;
     }
     if (I0 + slot >= tiles_m) return;
@@ -685,6 +692,82 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_tcq(const typename PackOf<PL>:
             *gptr((u64*)((u16*)S.out + o)) = (u64)lo | ((u64)hi << 32);
         }
     }
+}
+
+// Resident INT8 weights with the stage-split output (TCQ_Z_W128T) for one token block: a workgroup of 16 waves takes a 128-row
+// block of a segment, two waves per tile row (chunks part, part + 2, ..), four chunks of weights in flight per wave (256 KiB
+// per workgroup at K = 2048). What bounds it is the stream of the weights; in return the rest of the gated middle runs on
+// many CUs (tcq_glu_split) where the middle of one token had one. MI355X, one token, 2 x 16384 x
+// 2048: 14.7 us, as k_gemm_small (4.9 TB/s), and 3.1 for tcq_glu_split in place of k_mid2_tw2's 16.0.
+template <bool QB>
+__global__ __launch_bounds__(1024) void k_gemv_w8t(const SegPack P, const i8* q, const float* s, int M, int K) {
+    __shared__ __attribute__((aligned(16))) int4v red[8 * 64];
+    __shared__ float zb[16 * 128];
+    extern __shared__ __attribute__((aligned(16))) char xq[];             // the activations, 256 nch bytes per token
+    const tcq_gemm_seg S = P.s[blockIdx.y];
+    const int nch = (K + 255) >> 8, I0 = blockIdx.x * 8;
+    if (I0 >= (S.m >> 4)) return;                                         // uniform
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int slot = wave >> 1, part = wave & 1, lr = lane & 15, lg = lane >> 4;
+    const rsrc_t Wr = make_rsrc(S.w, (u32)S.m * (u32)K), Q = make_rsrc(q, QB ? 16u * (u32)K : (u32)M * (u32)K);
+    const u32 wrow = (u32)(16 * (I0 + slot) + lr) * (u32)K;
+    uint4_t wa[4][4];
+    auto load = [&](int c0) {                                              // weights of chunks c0, c0 + 2, ..
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int k0 = 256 * (c0 + 2 * i) + 64 * j + 16 * lg;
+                const u32 off = k0 < K ? wrow + (u32)k0 : RSRC_OOB;
+                wa[i][j] = __builtin_bit_cast(uint4_t, __builtin_amdgcn_raw_buffer_load_b128(Wr, off, 0, 2));
+            }
+    };
+    float4_t rsv = {0.f, 0.f, 0.f, 0.f};
+    float sv = 0.f;
+    if (part == 0) {
+        rsv = gptr((const float4_t*)(S.rs + 16 * (I0 + slot) + 4 * lg))[0];
+        sv = gptr(s)[min(lr, M - 1)];
+    }
+    // activations first (loads return in order: behind the weights they would wait for all of them), 16-byte piece u of token t
+    // at slot u ^ (t & 7)
+    const int np = 16 * nch;                                               // pieces per token, whole chunks (zeros past K)
+    auto piece = [&](int t, int u) { return xq + 16 * (t * np + (u ^ (t & 7))); };
+    constexpr int XL = 4;                                                  // pieces per thread: 16 tokens x 4096 columns
+    int4v xr[XL];
+#pragma unroll
+    for (int e = 0; e < XL; ++e) {
+        const int g = threadIdx.x + 1024 * e, t = g / np, k = 16 * (g - t * np);
+        const u32 off = t < M && k < K ? (QB ? (u32)tb_offset(t, k, K) : (u32)t * (u32)K + (u32)k) : RSRC_OOB;
+        xr[e] = __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(Q, off, 0, 0));
+    }
+    load(part);
+#pragma unroll
+    for (int e = 0; e < XL; ++e) {
+        const int g = threadIdx.x + 1024 * e, t = g / np;
+        if (t < M) *(int4v*)piece(t, g - t * np) = xr[e];
+    }
+    __syncthreads();
+    int4v acc = {0, 0, 0, 0};
+    for (int c0 = part; c0 < nch; c0 += 8) {
+        if (c0 != part) load(c0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int c = c0 + 2 * i;
+            if (c >= nch) continue;                                        // uniform
+            int4v B[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                B[j] = int4v{0, 0, 0, 0};
+                if (lr < M) B[j] = *(const int4v*)piece(lr, 16 * c + 4 * j + lg);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(int4v, wa[i][j]), B[j], acc, 0, 0, 0);
+        }
+    }
+    if (part) red[slot * 64 + lane] = acc;
+    __syncthreads();
+    if (!part) acc += red[slot * 64 + lane];
+    w128t_store(zb, acc, sv, rsv, !part, slot, M, (float*)S.out, S.m >> 7, I0 >> 3);
 }
 
 // =========================================================================================================== C ABI
@@ -1040,6 +1123,29 @@ extern "C" int tcq_gemm_tcq_pro(const tcq_gemm_seg* segs, int nseg, const tcq_pr
 extern "C" int tcq_gemm_w8_pro(const tcq_gemm_seg* segs, int nseg, const tcq_prologue* pro, int K, int out_dtype, int ldo,
                                tcq_stream_t stream) {
     return gemm_small_pro<1>(segs, nseg, pro, K, out_dtype, ldo, stream);
+}
+
+extern "C" int tcq_gemm_w8_w128t(const tcq_gemm_seg* segs, int nseg, const int8_t* q, const float* s, int M, int K, int flags,
+                                 tcq_stream_t stream) {
+    if (!segs || !q || !s || nseg <= 0 || M <= 0 || K <= 0 || (flags & ~TCQ_Q_TOKEN_BLOCKS)) return TCQ_ERR_ARG;
+    if (nseg > TCQ_MAX_SEGS || M > 16 || K > 4096) return TCQ_ERR_UNSUPPORTED;
+    if (K % 16 || (size_t)M * K >= ((size_t)1 << 31)) return TCQ_ERR_SHAPE;
+    if (!pal16(q)) return TCQ_ERR_ALIGN;
+    SegPack P = {};
+    int max_m = 0;
+    for (int i = 0; i < nseg; ++i) {
+        const tcq_gemm_seg& g = segs[i];
+        if (!g.w || !g.out || !g.rs || g.m <= 0) return TCQ_ERR_ARG;
+        if (g.m % 128 || (size_t)g.m * K >= ((size_t)1 << 31)) return TCQ_ERR_SHAPE;
+        if (!pal16(g.w) || !pal16(g.out) || !pal16(g.rs)) return TCQ_ERR_ALIGN;
+        P.s[i] = g;
+        max_m = g.m > max_m ? g.m : max_m;
+    }
+    const dim3 grid(max_m / 128, nseg), block(1024);
+    const size_t lds = (size_t)M * ((K + 255) / 256) * 256;
+    if (flags & TCQ_Q_TOKEN_BLOCKS) launch_k(k_gemv_w8t<true>, grid, block, lds, (hipStream_t)stream, P, (const i8*)q, s, M, K);
+    else launch_k(k_gemv_w8t<false>, grid, block, lds, (hipStream_t)stream, P, (const i8*)q, s, M, K);
+    return launch_status();
 }
 
 // ------------------------------------------------------------------------------------------ reference-shaped helpers

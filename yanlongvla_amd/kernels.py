@@ -739,6 +739,20 @@ def gemm_tcq_w128t(segs, q, s, dot=None, pro=None):
          128, stream())
 
 
+def gemm_w8_w128t(segs, q, s):
+    """gemm_tcq_w128t on resident INT8 weights: segments [(W (m, K) int8, rs, zt), ...] (tcq_gemm_w8_w128t)."""
+    arr = (_lib.GemmSeg * len(segs))()
+    M, K = s.numel(), q.shape[1] * (16 if q.dim() == 4 else 1)
+    for i, (w, rs, zt) in enumerate(segs):
+        _contig(w, rs, zt)
+        m = rs.numel()
+        if zt.dtype != torch.float32 or tuple(zt.shape) != (M, 128, m // 128) or w.dtype != torch.int8 or w.shape != (m, K):
+            raise ValueError(f'segment {i}: weights ({m}, {K}) int8, zt ({M}, 128, {m // 128}) float32')
+        arr[i] = _lib.GemmSeg(ptr(w), None, ptr(rs), ptr(zt), m, 0)
+    _contig(q, s)
+    call('tcq_gemm_w8_w128t', arr, len(segs), ptr(q), ptr(s), M, K, Q_TOKEN_BLOCKS if q.dim() == 4 else 0, stream())
+
+
 def glu_split(zt, sv, gelu_lut, p):
     """The gated-MLP middle after gemm_tcq_w128t of gate | up: zt (2, M, 128, N / 128) float32, sv (2N,) int8 signs of
     gate | up -> p (M, N) BF16 = bf16(gelu(g) * u); kernels.pre(p, down_su, ...) then equals mid2 bit for bit. N = 16384."""

@@ -284,10 +284,20 @@ class Group:
         return z
 
     def spreads(self, M):
-        """Whether this gate | up group's middle at M tokens runs spread over many CUs (gemm_tcq_w128t + glu_split + pre):
-        the fused decode of two 16384-wide members with one table each, K <= 4096, at most 16 tokens."""
-        return (FUSE['spread'] and self.W is None and M <= 16 and self.K <= 4096 and self.N == [16384, 16384]
-                and not self.one_sided and self.col_scale is None and all(L.t8.dim() == 2 for L in self.layers))
+        """Whether this gate | up group's middle at M tokens runs spread over many CUs (gemm_*_w128t + glu_split + pre): two
+        16384-wide members, K <= 4096, decoded with one table each at most 16 tokens, resident at most 8. Resident product, middle
+        and down product of one layer on MI355X, us: one token 42.8 -> 37.0, 8 tokens 43.4 -> 39.4, 16 tokens 45.8 -> 46.4."""
+        return (FUSE['spread'] and M <= (16 if self.W is None else 8) and self.K <= 4096 and self.N == [16384, 16384]
+                and not self.one_sided and self.col_scale is None and (self.W is not None or all(L.t8.dim() == 2 for L in self.layers)))
+
+    def spread_product(self, b, zt, pro=None):
+        """The gate | up product into the stage-split zt (2, M, 128, 128) (gemm_tcq_w128t / gemm_w8_w128t)."""
+        q, s = (None, None) if pro is not None else (b['q'] if b['q'] is not None else b['q4'], b['scale'])
+        if self.W is not None:
+            kernels.gemm_w8_w128t([(self.W[g.col0:g.col0 + g.width], g.rs, zt[i]) for i, g in enumerate(self.segments)], q, s)
+        else:
+            kernels.gemm_tcq_w128t([(L.words(), L.t8, g.rs, zt[i]) for i, (L, g) in enumerate(zip(self.layers, self.segments))], q, s,
+                                   pro=pro)
 
     def gated_middle(self, b, down, b2, pro=None):
         """This gate | up group's product and the GeGLU middle (tcq_mid2's operations) into the down projection's quantized
@@ -296,11 +306,7 @@ class Group:
         M, dev = (1, self.rs.device) if pro is not None else (b['scale'].numel(), b['scale'].device)
         if self.spreads(M):
             zt = torch.empty(2, M, 128, 128, dtype=torch.float32, device=dev)
-            segs = [(L.words(), L.t8, s.rs, zt[i]) for i, (L, s) in enumerate(zip(self.layers, self.segments))]
-            if pro is not None:
-                kernels.gemm_tcq_w128t(segs, None, None, pro=pro)
-            else:
-                kernels.gemm_tcq_w128t(segs, b['q'] if b['q'] is not None else b['q4'], b['scale'])
+            self.spread_product(b, zt, pro)
             p = kernels.glu_split(zt, self.sv, kernels.gelu_table(dev), torch.empty(M, 16384, dtype=torch.bfloat16, device=dev))
             kernels.pre(p, down.su, q=b2['q'], q4=b2['q4'], scale=b2['scale'])
             STATS['spread_middles'] += 1
@@ -321,13 +327,9 @@ class Group:
         workgroup computes the INT8 row from glu_split's output); else gated_middle then down.product. pro: as in
         gated_middle."""
         M, dev = (1, self.rs.device) if pro is not None else (b['scale'].numel(), b['scale'].device)
-        if self.spreads(M) and down.pre_prologue_fits(M):
+        if self.W is None and self.spreads(M) and down.pre_prologue_fits(M):
             zt = torch.empty(2, M, 128, 128, dtype=torch.float32, device=dev)
-            segs = [(L.words(), L.t8, s.rs, zt[i]) for i, (L, s) in enumerate(zip(self.layers, self.segments))]
-            if pro is not None:
-                kernels.gemm_tcq_w128t(segs, None, None, pro=pro)
-            else:
-                kernels.gemm_tcq_w128t(segs, b['q'] if b['q'] is not None else b['q4'], b['scale'])
+            self.spread_product(b, zt, pro)
             p = kernels.glu_split(zt, self.sv, kernels.gelu_table(dev), torch.empty(M, 16384, dtype=torch.bfloat16, device=dev))
             b2 = dict(q=None, q4=None, scale=torch.empty(M, dtype=torch.float32, device=dev))
             z = down.product(None, parts, pro=kernels.prologue_pre(p, down.su, scale=b2['scale']))
@@ -598,11 +600,11 @@ class KDecoderLayer(torch.nn.Module):
     def _prologue_fits(z, og, gu):
         """Whether the o epilogue + residual + norm2 + rotate + quantize can run as the prologue of the gate | up product
         (tcq_gemm_tcq_pro): one token, int32 sums, a two-sided o projection without bias, 2048-wide rows, and a gate | up
-        group on the spread middle (256 workgroups, one per CU, so each CU runs the prologue once). Measured on MI355X at
+        group decoded on the fly to the spread middle (256 workgroups, one per CU, each running the prologue once). On MI355X at
         one token: fly 18.1 -> 17.2 us for the two launches' work; on the resident plan's 1024 workgroups the prologue
         runs four times per CU and the pair gets slower (1.50 -> 1.72 ms per decode token), so it is not used there."""
         return (FUSE['prologue'] and z.dtype == torch.int32 and z.shape[-2] == 1 and og.bias is None and not og.one_sided
-                and og.Ntot == 2048 and gu.K == 2048 and gu.a8 and gu.spreads(1))
+                and og.Ntot == 2048 and gu.K == 2048 and gu.a8 and gu.W is None and gu.spreads(1))
 
     def _attn_prologue_fits(self, M, q, og):
         """Whether the attention's merge + o rotate + quantize can run as the prologue of the o product (tcq_gemm_*_pro with
