@@ -876,3 +876,42 @@ def test_w8a8_pipeline_matches_oracle():
     y = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
     Kk.gemm_i8(qa, qw, y, sa, sw)
     assert np.array_equal(y.view(torch.int16).cpu().numpy().view(np.uint16), ref['y'])
+
+
+def _quantized(v):
+    """Per-row INT8 by definition: scale max |v| / 127 (1 for a zero row), correctly rounded FP32 quotient, half-even, clamped;
+    a NaN (which the maximum passes over) becomes -127."""
+    v = v.astype(np.float32)
+    amax = np.where(np.isnan(v), 0, np.abs(v)).max(1, keepdims=True)
+    s = np.where(amax > 0, (amax / np.float32(127)).astype(np.float32), np.float32(1)).astype(np.float32)
+    with np.errstate(all='ignore'):
+        q = np.rint((v / s).astype(np.float32))
+        return np.where(np.isnan(q), -127, np.clip(q, -127, 127)).astype(np.int8), s[:, 0]
+
+
+@pytest.mark.parametrize('K', [4, 48, 1024])
+def test_quantizer_ties_and_extremes(K):
+    """Exact ties and their FP32 neighbours, zero rows, scales whose quotient is divided (below 2^-90, above 2^90), subnormal
+    rows, infinities and NaN."""
+    from yanlongvla_amd import kernels
+    rng = np.random.default_rng(K)
+    rows = []
+    for scale in (1.0, 2.0 ** -20, 3.0e-30, 2.0 ** -100, 2.0 ** 100, 1e-38, 1e-40):
+        n = rng.integers(-126, 126, K) + 0.5
+        v = (n * scale).astype(np.float32)
+        v[::3], v[1::3] = np.nextafter(v[::3], np.float32(np.inf)), np.nextafter(v[1::3], np.float32(-np.inf))
+        v[0] = 127 * scale
+        rows.append(v)
+    rows.append(np.zeros(K))
+    v = rng.standard_normal(K)
+    v[1] = np.nan
+    rows.append(v)
+    v = rng.standard_normal(K)
+    v[2] = -np.inf
+    rows.append(v)
+    x = np.stack(rows).astype(np.float32)
+    q = torch.empty(x.shape, dtype=torch.int8, device='cuda')
+    s = torch.empty(x.shape[0], device='cuda')
+    kernels.quantize_rows(torch.from_numpy(x).cuda(), q, s)
+    qr, sr = _quantized(x)
+    assert np.array_equal(q.cpu().numpy(), qr) and np.array_equal(s.cpu().numpy(), sr)

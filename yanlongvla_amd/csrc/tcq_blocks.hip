@@ -190,7 +190,7 @@ template <int DT, class R4>
 __device__ __forceinline__ float elem4(const R4& a, int e) {
     if constexpr (DT == TCQ_F32) return __uint_as_float(a[e]);
     else if constexpr (DT == TCQ_I32) return (float)(int)a[e];
-    else if constexpr (DT == TCQ_I8) return (float)(i8)(a >> (8 * e));
+    else if constexpr (DT == TCQ_I8) return i8_f32(a, e);
     else {
         const u16 h = (u16)(a[e >> 1] >> (16 * (e & 1)));
         return DT == TCQ_BF16 ? bf16_to_f32(h) : f16_to_f32(h);
@@ -315,7 +315,8 @@ __device__ __forceinline__ void rotate_quantize_row(const Place<NW>& P, Row<FM>&
     if (threadIdx.x == 0) scale[tok] = sc;
     const QScale S = qscale(sc);
     each(P, R, [&](float(&v)[4], int i, float) {
-        const u32 w = (u32)(q8(v[0], S) & 0xff) | ((u32)(q8(v[1], S) & 0xff) << 8) | ((u32)(q8(v[2], S) & 0xff) << 16) | ((u32)(q8(v[3], S) & 0xff) << 24);
+        u32 w;
+        q8_words<1>(v, S, &w);
         if (q) *gptr((u32*)(q + (size_t)tok * P.K + i)) = w;
         if (q4) {
             if (ldq == TCQ_LDQ_TOKEN_BLOCKS) *gptr((u32*)((i8*)q4 + tb_offset(tok, i, P.K))) = w;

@@ -24,6 +24,18 @@ typedef u16 u16x2_t __attribute__((ext_vector_type(2)));
 
 // ------------------------------------------------------------------------------------------------------------ conversions
 __device__ __forceinline__ float bf16_to_f32(u16 b) { return __uint_as_float(((u32)b) << 16); }
+// signed byte e (a constant after unrolling) of w as FP32 in one instruction; from (float)(i8)(w >> 8 e) the compiler makes a
+// field extraction and a conversion (800 x 16384 BF16 rotation on MI355X 16.1 -> 15.7 us)
+__device__ __forceinline__ float i8_f32(u32 w, int e) {
+    float f;
+    switch (e) {
+        case 0: asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_0" : "=v"(f) : "v"(w)); break;
+        case 1: asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_1" : "=v"(f) : "v"(w)); break;
+        case 2: asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_2" : "=v"(f) : "v"(w)); break;
+        default: asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_3" : "=v"(f) : "v"(w)); break;
+    }
+    return f;
+}
 // FP32 -> BF16, round to nearest even, every NaN -> 0x7fc0 (reference kernels.py:20-25). gfx950's v_cvt_pk_bf16_f32
 // rounds to nearest even (subnormals kept: the kernels run with FP32 denormals on); only its NaN results differ (it keeps
 // the sign and payload), so NaN inputs are replaced after the conversion.
@@ -561,20 +573,33 @@ __device__ __forceinline__ QScale qscale(float s) {
     const bool fast = s >= 0x1p-90f && s <= 0x1p90f;
     return QScale{s, fast ? 1.f / s : 0.f, fast};
 }
-__device__ __forceinline__ int q8(float v, const QScale& S) {
-    float d;
-    if (S.fast) {
-        d = v * S.rcp;
-        float e = __builtin_fmaf(-d, S.s, v);
-        d = __builtin_fmaf(e, S.rcp, d);
-        e = __builtin_fmaf(-d, S.s, v);
-        d = __builtin_fmaf(e, S.rcp, d);
+// 4 NW values -> NW words of four INT8 (value 4 j in the low byte of word j). The rounded integer and its two's complement byte in
+// one addition: with the quotient clamped to +-127 first (rounding keeps the order, so clamping commutes with it; a NaN
+// becomes -127), adding 1.5 * 2^23 rounds it half-even to a whole number whose low byte is the byte wanted. Rotate + quantize of
+// 968 x 16384 on MI355X 19.5 -> 17.9 us, of 968 x 2048 4.9 -> 4.5.
+template <int NW>
+__device__ __forceinline__ void q8_words(const float* v, const QScale& S, u32* w) {
+    float d[4 * NW];
+    if (S.fast) {                                                          // uniform
+#pragma unroll
+        for (int k = 0; k < 4 * NW; ++k) {
+            d[k] = v[k] * S.rcp;
+            float e = __builtin_fmaf(-d[k], S.s, v[k]);
+            d[k] = __builtin_fmaf(e, S.rcp, d[k]);
+            e = __builtin_fmaf(-d[k], S.s, v[k]);
+            d[k] = __builtin_fmaf(e, S.rcp, d[k]);
+        }
     } else {
-        d = v / S.s;
+#pragma unroll
+        for (int k = 0; k < 4 * NW; ++k) d[k] = v[k] / S.s;
     }
-    float r = __builtin_rintf(d);
-    r = fminf(fmaxf(r, -127.f), 127.f);
-    return (int)r;
+#pragma unroll
+    for (int j = 0; j < NW; ++j) {
+        u32 b[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) b[k] = __float_as_uint(fminf(fmaxf(d[4 * j + k], -127.f), 127.f) + 0x1.8p23f);
+        w[j] = __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u) | __builtin_amdgcn_perm(b[3], b[2], 0x04000c0cu);
+    }
 }
 __device__ __forceinline__ float token_scale(float amax) { return amax > 0.f ? amax / 127.f : 1.f; }
 
@@ -588,8 +613,9 @@ __device__ __forceinline__ size_t tb_offset(int t, int k, int K) {
 __device__ __forceinline__ void quantize_row(const float* lds, float sc, i8* q, int* q4, int tok, int K, int ldq) {
     const QScale s = qscale(sc);
     for (int j = threadIdx.x; j < (K >> 2); j += blockDim.x) {
-        const u32 word = (u32)(q8(lds[lds_slot(4 * j)], s) & 0xff) | ((u32)(q8(lds[lds_slot(4 * j + 1)], s) & 0xff) << 8) |
-                         ((u32)(q8(lds[lds_slot(4 * j + 2)], s) & 0xff) << 16) | ((u32)(q8(lds[lds_slot(4 * j + 3)], s) & 0xff) << 24);
+        const float v[4] = {lds[lds_slot(4 * j)], lds[lds_slot(4 * j + 1)], lds[lds_slot(4 * j + 2)], lds[lds_slot(4 * j + 3)]};
+        u32 word;
+        q8_words<1>(v, s, &word);
         if (q) ((u32*)q)[j] = word;
         if (q4) {
             if (ldq == TCQ_LDQ_TOKEN_BLOCKS) *(u32*)((i8*)q4 + tb_offset(tok, 4 * j, K)) = word;
@@ -663,7 +689,7 @@ __device__ __forceinline__ Raw16<ESZ> raw16(const void* p, bool vec) {
 }
 __device__ __forceinline__ void cv16(const Raw16<1>& a, float (&v)[16]) {
 #pragma unroll
-    for (int k = 0; k < 16; ++k) v[k] = (float)(i8)(a.r[0][k >> 2] >> (8 * (k & 3)));
+    for (int k = 0; k < 16; ++k) v[k] = i8_f32(a.r[0][k >> 2], k & 3);
 }
 __device__ __forceinline__ void cv16(const Raw16<2>& a, float (&v)[16]) {
 #pragma unroll
@@ -693,10 +719,7 @@ __device__ __forceinline__ void reg_rotate_quantize(float (&v)[16], int N, float
     if (!on) return;
     const QScale S = qscale(sc);
     u32 words[4];
-#pragma unroll
-    for (int k4 = 0; k4 < 4; ++k4)
-        words[k4] = (u32)(q8(v[4 * k4], S) & 0xff) | ((u32)(q8(v[4 * k4 + 1], S) & 0xff) << 8) |
-                    ((u32)(q8(v[4 * k4 + 2], S) & 0xff) << 16) | ((u32)(q8(v[4 * k4 + 3], S) & 0xff) << 24);
+    q8_words<4>(v, S, words);
     if (q) *gptr((uint4_t*)(q + (size_t)tok * N + 16 * t)) = uint4_t{words[0], words[1], words[2], words[3]};
     if (q4 && ldq == TCQ_LDQ_TOKEN_BLOCKS) {
         *gptr((uint4_t*)((i8*)q4 + tb_offset(tok, 16 * t, N))) = uint4_t{words[0], words[1], words[2], words[3]};
@@ -736,10 +759,7 @@ __device__ __forceinline__ void tw_rotate_quantize(float (&v)[1 << LE], float* x
     if (!on) return;
     const QScale S = qscale(sc);
     u32 words[E / 4];
-#pragma unroll
-    for (int k4 = 0; k4 < E / 4; ++k4)
-        words[k4] = (u32)(q8(v[4 * k4], S) & 0xff) | ((u32)(q8(v[4 * k4 + 1], S) & 0xff) << 8) |
-                    ((u32)(q8(v[4 * k4 + 2], S) & 0xff) << 16) | ((u32)(q8(v[4 * k4 + 3], S) & 0xff) << 24);
+    q8_words<E / 4>(v, S, words);
     if constexpr (E == 8) {                                             // 8 bytes per thread: half a 16-byte group
         const u64 d = (u64)words[0] | ((u64)words[1] << 32);
         if (qs) *(u64*)(qs + 2 * t) = d;

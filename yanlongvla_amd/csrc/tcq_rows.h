@@ -39,7 +39,7 @@ __device__ __forceinline__ void c16_i8(const i8* p, bool vec, float (&v)[16]) {
     if (vec) {
         const uint4_t a = gptr((const uint4_t*)p)[0];
 #pragma unroll
-        for (int k = 0; k < 16; ++k) v[k] = (float)(i8)(a[k >> 2] >> (8 * (k & 3)));
+        for (int k = 0; k < 16; ++k) v[k] = i8_f32(a[k >> 2], k & 3);
     } else {
 #pragma unroll
         for (int k = 0; k < 16; ++k) v[k] = (float)gptr(p)[k];
@@ -166,7 +166,7 @@ struct NoMid {
 __device__ __forceinline__ void ld8_i8v(const i8* p, float (&v)[8]) {
     const u64 w = *gptr((const u64*)p);
 #pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = (float)(i8)(w >> (8 * k));
+    for (int k = 0; k < 8; ++k) v[k] = i8_f32((u32)(w >> (32 * (k >> 2))), k & 3);
 }
 __device__ __forceinline__ void ld8_bf16v(const u16* p, float (&v)[8]) {
     const uint4_t a = gptr((const uint4_t*)p)[0];
@@ -404,7 +404,7 @@ __device__ __forceinline__ void panp_waves(const PanpArgs& A, int tok, bool stor
         } else {
             const u32 x = *gptr((const u32*)p);
 #pragma unroll
-            for (int k = 0; k < 4; ++k) o[k] = (float)(i8)(x >> (8 * k));
+            for (int k = 0; k < 4; ++k) o[k] = i8_f32(x, k);
         }
     };
     auto ld_bf16 = [&](const u16* p, float (&o)[E]) {
@@ -532,10 +532,7 @@ __device__ __forceinline__ void waves_rotate_quantize(float (&v)[(1 << L) / 64 /
     }
     const QScale S = qscale(sc);
     u32 words[E / 4];
-#pragma unroll
-    for (int k4 = 0; k4 < E / 4; ++k4)
-        words[k4] = (u32)(q8(v[4 * k4], S) & 0xff) | ((u32)(q8(v[4 * k4 + 1], S) & 0xff) << 8) |
-                    ((u32)(q8(v[4 * k4 + 2], S) & 0xff) << 16) | ((u32)(q8(v[4 * k4 + 3], S) & 0xff) << 24);
+    q8_words<E / 4>(v, S, words);
     const bool tb = q4 && ldq == TCQ_LDQ_TOKEN_BLOCKS;
     if constexpr (E == 8) {
         const u64 d = (u64)words[0] | ((u64)words[1] << 32);

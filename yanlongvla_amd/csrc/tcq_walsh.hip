@@ -64,7 +64,7 @@ template <> struct Elem<TCQ_I32> {
 __device__ __forceinline__ void ld8_i8(const i8* p, int i, float (&v)[8]) {
     const u64 w = *gptr((const u64*)(p + i));
 #pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = (float)(i8)(w >> (8 * k));
+    for (int k = 0; k < 8; ++k) v[k] = i8_f32((u32)(w >> (32 * (k >> 2))), k & 3);
 }
 __device__ __forceinline__ void ld8_f32(const float* p, int i, float (&v)[8]) { Elem<TCQ_F32>::ld8(p, i, v); }
 
@@ -304,7 +304,7 @@ __global__ __launch_bounds__(64 * NWP) void k_pre_h16_wv(const void* x, const i8
     if (su) {
         const u32 sg = *gptr((const u32*)(su + 4 * t));
 #pragma unroll
-        for (int k = 0; k < 4; ++k) v[k] = v[k] * (float)(i8)(sg >> (8 * k));
+        for (int k = 0; k < 4; ++k) v[k] = v[k] * i8_f32(sg, k);
     }
     wave_walsh<2, NWP>(v, xs, [] { __syncthreads(); });
     const float c = (float)(1.0 / __builtin_sqrt((double)K));
@@ -962,7 +962,12 @@ __global__ __launch_bounds__(1 << (L - 5)) void k_postg_tw5(PostPack segs, const
             float& x = v[16 * h + k];
             x = x * sg[k];
             if (S.bias) x = x + b[k];
-            if (YDT == TCQ_BF16 && S.gelu) x = bf16_to_f32(gptr(gelu_lut)[f32_to_bf16(x)]);
+        }
+        if (YDT == TCQ_BF16 && S.gelu) {
+            u32 ix[8];
+            bf16_pack<8>(v + 16 * h, ix);
+#pragma unroll
+            for (int k = 0; k < 16; ++k) v[16 * h + k] = bf16_to_f32(gptr(gelu_lut)[k & 1 ? ix[k / 2] >> 16 : ix[k / 2] & 0xffffu]);
         }
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
@@ -1046,9 +1051,10 @@ __global__ __launch_bounds__(1 << (L - LE), 4) void k_mid2_tw(const void* acc, i
         cv16(svg[h], sg);
 #pragma unroll
         for (int k = 0; k < 16; ++k) g[16 * h + k] = g[16 * h + k] * c * sg[k];
+        u32 ix[8];
+        bf16_pack<8>(g + 16 * h, ix);
 #pragma unroll
-        for (int k = 0; k < 16; k += 2)
-            gv[8 * h + k / 2] = u16x2_t{gptr(lut)[f32_to_bf16(g[16 * h + k])], gptr(lut)[f32_to_bf16(g[16 * h + k + 1])]};
+        for (int k = 0; k < 8; ++k) gv[8 * h + k] = u16x2_t{gptr(lut)[ix[k] & 0xffffu], gptr(lut)[ix[k] >> 16]};
     }
     if constexpr (ADT != TCQ_BF16) {
         stage(ua, rs ? rs + N : nullptr);     // writes only the wave's own span: its threads have finished reading it
@@ -1062,10 +1068,14 @@ __global__ __launch_bounds__(1 << (L - LE), 4) void k_mid2_tw(const void* acc, i
         cv16(svu[h], sgu);
         cv16(sn0[h], sn);
 #pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            const float uu = bf16_to_f32(f32_to_bf16((u[16 * h + k] * c) * sgu[k]));
-            u[16 * h + k] = bf16_to_f32(f32_to_bf16(bf16_to_f32(gv[8 * h + k / 2][k & 1]) * uu)) * sn[k];
-        }
+        for (int k = 0; k < 16; ++k) u[16 * h + k] = (u[16 * h + k] * c) * sgu[k];
+        u16 b[16];
+        bf16_round<8>(u + 16 * h, b);
+#pragma unroll
+        for (int k = 0; k < 16; ++k) u[16 * h + k] = bf16_to_f32(gv[8 * h + k / 2][k & 1]) * u[16 * h + k];
+        bf16_round<8>(u + 16 * h, b);
+#pragma unroll
+        for (int k = 0; k < 16; ++k) u[16 * h + k] = u[16 * h + k] * sn[k];
     }
     tw_rotate_quantize<L, LE>(u, xs, red, q, q4, ldq, scale, tok);
 }
@@ -1109,7 +1119,7 @@ __device__ __forceinline__ void postg_wv_seg(const tcq_post_seg& S, int tok, flo
     const float c = (float)(1.0 / __builtin_sqrt((double)N));
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        v[k] = (v[k] * c) * (float)(i8)(sg >> (8 * k));
+        v[k] = (v[k] * c) * i8_f32(sg, k);
         if (S.bias) v[k] = v[k] + b[k];
         if (YDT == TCQ_BF16 && gelu) v[k] = bf16_to_f32(gptr(gelu)[f32_to_bf16(v[k])]);
     }
@@ -1184,7 +1194,7 @@ __global__ __launch_bounds__(64 * NWP) void k_mid2_wv(const void* acc, int lda, 
         } else {
             const u32 x = *gptr((const u32*)p);
 #pragma unroll
-            for (int k = 0; k < 4; ++k) o[k] = (float)(i8)(x >> (8 * k));
+            for (int k = 0; k < 4; ++k) o[k] = i8_f32(x, k);
         }
     };
     // accumulator values i0 .. i0 + E - 1 of the half at column offset h (scaled as acc_chunk scales them)
@@ -1221,12 +1231,20 @@ __global__ __launch_bounds__(64 * NWP) void k_mid2_wv(const void* acc, int lda, 
     wave_walsh2<LE, NWP>(g, u, xg, xu, bar);
     u16 gv[E];
 #pragma unroll
-    for (int k = 0; k < E; ++k) gv[k] = gptr(lut)[f32_to_bf16(g[k] * c * sg[k])];
+    for (int k = 0; k < E; ++k) g[k] = g[k] * c * sg[k];
+    u32 ix[E / 2];
+    bf16_pack<E / 2>(g, ix);
 #pragma unroll
-    for (int k = 0; k < E; ++k) {
-        const float uu = bf16_to_f32(f32_to_bf16((u[k] * c) * sgu[k]));
-        u[k] = bf16_to_f32(f32_to_bf16(bf16_to_f32(gv[k]) * uu)) * sn[k];
-    }
+    for (int k = 0; k < E; ++k) gv[k] = gptr(lut)[k & 1 ? ix[k / 2] >> 16 : ix[k / 2] & 0xffffu];
+    u16 b[E];
+#pragma unroll
+    for (int k = 0; k < E; ++k) u[k] = (u[k] * c) * sgu[k];
+    bf16_round<E / 2>(u, b);
+#pragma unroll
+    for (int k = 0; k < E; ++k) u[k] = bf16_to_f32(gv[k]) * u[k];
+    bf16_round<E / 2>(u, b);
+#pragma unroll
+    for (int k = 0; k < E; ++k) u[k] = u[k] * sn[k];
     waves_rotate_quantize<NWP, L>(u, Qr, nullptr, nullptr, q, scale, bar, tok, q4, ldq);
 }
 
