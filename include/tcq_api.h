@@ -475,6 +475,13 @@ int tcq_gemm_i8_best_parts(int M, int N, int K);
 int tcq_gemm_bf16(const void* a, const void* w, const float* sa, const float* sw, void* out, int out_dtype, int ldo, int M, int N,
                   int K, tcq_stream_t stream);
 
+/* tcq_gemm_bf16 for few output tiles over a long K: the FP32 sums of 2 or 4 K parts into part (parts * M * N floats, 16-byte aligned),
+ * then their sum * sw (NULL: factor 1) into the contiguous (M, N) out. K >= 1024. best_parts: the parts (1: tcq_gemm_bf16) with
+ * the least estimated time. No reference counterpart. */
+int tcq_gemm_bf16_parts(const void* a, const void* w, const float* sw, float* part, void* out, int out_dtype, int M, int N, int K,
+                        int parts, tcq_stream_t stream);
+int tcq_gemm_bf16_best_parts(int M, int N, int K);
+
 /* W2 float path prologue: bf16(fwht(x * su)) per token (x (M, K) of x_dtype F32 / BF16 / F16, contiguous) into h (M, K)
  * row-major and / or hT (K, ldh) with token = column (ldh >= M); either may be NULL, not both. Replaces kernels.pre_h /
  * k_preh_{bf16,f32} (deploy/tcq_kernels/kernels.py:309-317, 677-680), argument for argument. */

@@ -64,3 +64,18 @@ def test_k_parts_refused():
     for K, parts in ((2032, 2), (4096, 3)):
         with pytest.raises(_lib.TcqError):
             Kn.gemm_i8_parts(_ints(80, K, seed=7), _ints(64, K, seed=8), parts)
+
+
+@pytest.mark.parametrize('M,N,K', [(65, 64, 1024), (129, 132, 1040), (300, 1156, 4304), (968, 2048, 16384)])
+@pytest.mark.parametrize('parts', [2, 4])
+def test_bf16_parts_against_fp64(M, N, K, parts):
+    """As test_bf16_tiles_against_fp64 (any order of FP32 sums); FP32 and BF16 outputs with and without row scales agree."""
+    from yanlongvla_amd import kernels as Kn
+    g = torch.Generator(device=DEV).manual_seed(5)
+    a, w = torch.randn(M, K, generator=g, device=DEV).bfloat16(), _ints(N, K, seed=6).bfloat16()
+    want, mag = a.double() @ w.double().t(), a.double().abs() @ w.double().abs().t()
+    z = Kn.gemm_bf16_parts(a, w, torch.empty(M, N, device=DEV), parts)
+    assert bool(((z.double() - want).abs() <= K * 2.0 ** -24 * mag).all())
+    sw = torch.rand(N, device=DEV) + 0.01
+    assert torch.equal(Kn.gemm_bf16_parts(a, w, torch.empty(M, N, device=DEV), parts, sw=sw), z * sw)
+    assert torch.equal(Kn.gemm_bf16_parts(a, w, torch.empty(M, N, dtype=torch.bfloat16, device=DEV), parts), z.bfloat16())

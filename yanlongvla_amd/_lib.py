@@ -46,6 +46,8 @@ SIGNATURES = {
     'tcq_gemv_f16_post': [_P, _I, _P, _P, _I, _I, _I, _I, _P],
     'tcq_layer_f16': [_P, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P, _P, _P],
     'tcq_pre_gemv_f16': [_P, _I, _P, _P, _P, _P, _I, _I, _I, _P, _P],
+    'tcq_gemm_bf16_parts': [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
+    'tcq_gemm_bf16_best_parts': [_I, _I, _I],
     'tcq_gemm_i8_parts': [_P, _P, _P, _I, _I, _I, _I, _I, _P],
     'tcq_gemm_i8_best_parts': [_I, _I, _I],
     'tcq_gemm_bf16': [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],

@@ -248,9 +248,11 @@ __global__ __launch_bounds__(64 * WN * WM) void k_gemm_i8(const void* x_, const 
         for (; kt + NS < nfull; ++kt) step(kt, Full{});
         for (; kt < nk; ++kt) step(kt, Tail{});
     } else {
-        // FP32 sums in two levels, `flush` steps (two MFMAs each) in a row, then the sums of those: the rounding error of one
-        // chain over all of K grows with its length (relative error of the float path's layers against 64 bits, K = 16384:
-        // 4.3e-4 with two levels, as the few-token products' partial sums give; 4.6e-4 with one chain)
+        // FP32 sums in two levels, `flush` steps (two MFMAs each) in a row, then the sums of those, each with what its addition
+        // rounded away (sum - exact, by two subtractions) carried into the next chain: the error of the second level vanishes,
+        // and that of a chain grows with its length only. Relative error against 64 bits, K = 1024 / 2048 / 4096 / 16384:
+        // 4.9e-8, 5.6e-8, 6.4e-8, 8.9e-8; without the carry 6.3e-8, 7.3e-8, 8.7e-8, 1.24e-7; the few-token product's partial sums
+        // (three levels) 5.7e-8, 6.9e-8, 7.8e-8, 1.18e-7.
         acc_t sum[NB][MB];
 #pragma unroll
         for (int i = 0; i < NB; ++i)
@@ -264,8 +266,9 @@ __global__ __launch_bounds__(64 * WN * WM) void k_gemm_i8(const void* x_, const 
             for (int i = 0; i < NB; ++i)
 #pragma unroll
                 for (int j = 0; j < MB; ++j) {
-                    sum[i][j] += acc[i][j];
-                    acc[i][j] = acc_t{0, 0, 0, 0};
+                    const acc_t t = sum[i][j] + acc[i][j];
+                    acc[i][j] = acc[i][j] - (t - sum[i][j]);
+                    sum[i][j] = t;
                 }
         }
 #pragma unroll
@@ -435,4 +438,60 @@ extern "C" int tcq_gemm_bf16(const void* a, const void* w, const float* sa, cons
     if ((uintptr_t)a % 16 || (uintptr_t)w % 16 || (uintptr_t)out % 16 || (sw && (uintptr_t)sw % 16) || ldo % 4) return TCQ_ERR_ALIGN;
     launch_by_size<2>(out_dtype, (hipStream_t)stream, a, w, sa, sw, out, ldo, M, N, K, 1);
     return launch_status();
+}
+
+// FP32 K parts added in order, * sw, to FP32 or BF16: four columns per thread.
+template <int ODT>
+__global__ __launch_bounds__(256) void k_sum_parts(const float* part, const float* sw, void* out, size_t n, int N, int parts) {
+    const size_t i = 4 * ((size_t)blockIdx.x * 256 + threadIdx.x);
+    if (i >= n) return;
+    float4v v = *gptr((const float4v*)(part + i));
+    for (int p = 1; p < parts; ++p) {
+        const float4v u = *gptr((const float4v*)(part + p * n + i));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = v[e] + u[e];
+    }
+    if (sw) {
+        const float4v r = *gptr((const float4v*)(sw + i % N));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = v[e] * r[e];
+    }
+    if (ODT == TCQ_F32) *gptr((float4v*)((float*)out + i)) = v;
+    else *gptr((uint2_t*)((u16*)out + i)) = uint2_t{bf16x2(v[0], v[1]), bf16x2(v[2], v[3])};
+}
+
+extern "C" int tcq_gemm_bf16_parts(const void* a, const void* w, const float* sw, float* part, void* out, int out_dtype, int M, int N,
+                                   int K, int parts, tcq_stream_t stream) {
+    if (!a || !w || !part || !out || M <= 0 || N <= 0 || K <= 0 || (parts != 2 && parts != 4)) return TCQ_ERR_ARG;
+    if (out_dtype != TCQ_F32 && out_dtype != TCQ_BF16) return TCQ_ERR_DTYPE;
+    if (K % 16 || N % 4 || K < 64 * 16) return TCQ_ERR_SHAPE;                            // every part has steps of its own
+    if ((size_t)M * K * 2 >= ((size_t)1 << 31) || (size_t)N * K * 2 >= ((size_t)1 << 31) || (size_t)parts * M * N >= ((size_t)1 << 31))
+        return TCQ_ERR_SHAPE;
+    if ((uintptr_t)a % 16 || (uintptr_t)w % 16 || (uintptr_t)part % 16 || (uintptr_t)out % 16 || (sw && (uintptr_t)sw % 16)) return TCQ_ERR_ALIGN;
+    hipStream_t st = (hipStream_t)stream;
+    launch_by_size<2>(TCQ_F32, st, a, w, nullptr, nullptr, part, N, M, N, K, parts);
+    const int e = launch_status();
+    if (e) return e;
+    const size_t n = (size_t)M * N;
+    const dim3 grid((unsigned)((n / 4 + 255) / 256));
+    if (out_dtype == TCQ_F32) launch_k(k_sum_parts<TCQ_F32>, grid, dim3(256), 0, st, (const float*)part, sw, out, n, N, parts);
+    else launch_k(k_sum_parts<TCQ_BF16>, grid, dim3(256), 0, st, (const float*)part, sw, out, n, N, parts);
+    return launch_status();
+}
+
+// As tcq_gemm_i8_best_parts, with 2 us for the launch that adds the parts, and their write and read at 6 TB/s. MI355X, us in 1 / 2 /
+// 4 parts: 968 x 2048 x 16384 105 / 81 / 76, 256: 77 / 45 / 33; 128 x 1024 x 4096 23 / 16 / 12; 400 x 2048 x 2048 14.3 / 15.0 / 17.5.
+// Relative error against 64 bits, 968 x 2048 x 16384: 8.9e-8, 9.3e-8, 9.7e-8 (the few-token product's partial sums: 1.18e-7).
+extern "C" int tcq_gemm_bf16_best_parts(int M, int N, int K) {
+    if (M <= 64 || N <= 0 || K < 64 * 16) return 1;
+    int best = 1;
+    double bt = 0;
+    for (int parts = 1; parts <= 4; parts *= 2) {
+        long c = 0;
+        choose_tile(M, N, parts, 4, &c);
+        const int steps = (K + 63) / 64;
+        const double t = (steps + parts - 1) / parts * (c / 32.0) + (parts > 1 ? 2 + parts * 8.0 * M * N / 6e6 : 0);
+        if (parts == 1 || (t < bt && (size_t)parts * M * N < ((size_t)1 << 31))) { best = parts; bt = t; }
+    }
+    return best;
 }

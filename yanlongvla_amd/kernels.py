@@ -809,6 +809,31 @@ def gemm_bf16(a, w, out, sa=None, sw=None):
     return out
 
 
+def gemm_bf16_best(a, w, out, sw=None):
+    """gemm_bf16 into a contiguous out, in as many K parts as its size calls for (a workspace of this call holds them)."""
+    M, K = a.shape
+    N = w.shape[0]
+    parts = int(_lib.lib().tcq_gemm_bf16_best_parts(M, N, K))
+    if parts == 1:
+        return gemm_bf16(a, w, out, sw=sw)
+    return gemm_bf16_parts(a, w, out, parts, sw=sw)
+
+
+def gemm_bf16_parts(a, w, out, parts, sw=None):
+    """gemm_bf16 as the sum of 2 or 4 FP32 K parts: out (M, N) contiguous FP32 / BF16."""
+    M, K = a.shape
+    N = w.shape[0]
+    _contig(a, w, sw, out)
+    if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
+        raise TypeError('gemm_bf16_parts: BF16 operands')
+    if w.shape[1] != K or out.shape != (M, N) or (sw is not None and sw.numel() != N):
+        raise ValueError('gemm_bf16_parts: shapes do not match')
+    part = torch.empty(parts, M, N, dtype=torch.float32, device=a.device)
+    call('tcq_gemm_bf16_parts', ptr(a), ptr(w), ptr(sw), ptr(part), ptr(out), _dt(out, (0, 1), 'gemm_bf16_parts out'), M, N, K, parts,
+         stream())
+    return out
+
+
 # ------------------------------------------------------------------------------------------------------- W2 float path
 def pre_h(x, su, h=None, hT=None):
     """Rotated activations as BF16: h (M, K) row-major and / or hT (K, ldh) with token = column, bf16(fwht(x * su))

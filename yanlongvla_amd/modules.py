@@ -409,7 +409,7 @@ class Group:
                 kernels.i8_to_bf16(self.W, w)
             else:
                 self.decode(w)
-            kernels.gemm_bf16(h, w, acc, sw=self.rs if self.small else None)
+            kernels.gemm_bf16_best(h, w, acc, sw=self.rs if self.small else None)
             return self.posts(acc, None, shape)
         if self.W is not None:
             segs = [(self.W[s.col0:s.col0 + s.width], None, s.rs, acc[:, s.col0:]) for s in self.segments]
