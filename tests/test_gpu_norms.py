@@ -187,3 +187,30 @@ def test_decoder_layer_fusion_is_bitexact():
             modules.FUSE['layer'] = old
     assert torch.equal(outs[True][0], outs[False][0])
     assert torch.equal(outs[True][1], outs[False][1])
+
+
+@pytest.mark.parametrize('M,N', [(65, 2048), (419, 2048), (420, 2048), (839, 1024), (840, 1024)])
+def test_epilogues_of_more_rows_match_few(M, N):
+    """post_add_norm_pre, post and post_group around the row counts where their engine changes: each row as in calls of 40."""
+    from yanlongvla_amd import kernels as Kn
+    g = torch.Generator(device=DEV).manual_seed(M)
+    r = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    acc, x, w = r(M, N + 512), r(M, N).bfloat16(), r(N).bfloat16()
+    sv, su = (torch.where(r(N) > 0, 1, -1).to(torch.int8) for _ in range(2))
+
+    def run(a, b):
+        a_, x_, m = acc[a:b], x[a:b], b - a
+        xo, q, s = torch.empty_like(x_), torch.empty(m, N, dtype=torch.int8, device=DEV), torch.empty(m, device=DEV)
+        Kn.post_add_norm_pre(a_, None, None, sv, None, x_, xo, w, 1e-6, su, q=q, scale=s)
+        y = torch.empty_like(x_)
+        Kn.post(a_, None, None, sv, None, y)
+        ys = [torch.empty(m, n, dtype=torch.bfloat16, device=DEV) for n in (N, 256, 256)]
+        c = (0, N, N + 256)
+        Kn.post_group([(a_, c0, None, sv[:t.shape[1]], None, t, False) for c0, t in zip(c, ys)], torch.float32, torch.bfloat16, None, m)
+        one = torch.empty_like(x_)
+        Kn.post_group([(a_, 0, None, sv, None, one, False)], torch.float32, torch.bfloat16, None, m)
+        return [xo, q, s, y, one] + ys
+    whole = run(0, M)
+    parts = [run(a, min(a + 40, M)) for a in range(0, M, 40)]
+    for i, t in enumerate(whole):
+        assert torch.equal(t, torch.cat([p[i] for p in parts]))

@@ -1683,9 +1683,10 @@ extern "C" int tcq_post(const void* acc, int acc_dtype, int lda, int col0, const
     }
     if (N > TCQ_MAX_WIDTH) return TCQ_ERR_SHAPE;
     const int asz = dsize(acc_dtype);
-    if (M <= 64 && (N == 256 || N == 1024 || N == 2048) && al16(acc) && ((size_t)lda * asz) % 16 == 0 && ((size_t)col0 * asz) % 16 == 0 &&
-        al16(y) && al16(sv) && (!rs || al16(rs)) && (!bias || al16(bias))) {   // few rows: the no-transpose engine
+    if ((N == 256 || N == 1024 || N == 2048) && al16(acc) && ((size_t)lda * asz) % 16 == 0 && ((size_t)col0 * asz) % 16 == 0 &&
+        al16(y) && al16(sv) && (!rs || al16(rs)) && (!bias || al16(bias))) {   // the no-transpose engine
         hipStream_t st = (hipStream_t)stream;
+        // us on MI355X against the LDS engine: 80 x 2048 3.1 / 4.7, 968 x 2048 5.1 / 6.6, 968 x 1024 3.6 / 4.5
 #define POSTW_K(AD, YD, L, NWP) launch_k(k_post_wv<AD, YD, L, NWP>, dim3(M), dim3(64 * NWP), 0, st, acc, lda, col0, s, rs, (const i8*)sv, bias, y)
 #define POSTW_Y(AD, YD)                                                                                                    \
     if (N == 2048) POSTW_K(AD, YD, 11, 8);                                                                                 \
@@ -1740,7 +1741,7 @@ extern "C" int tcq_postg(const tcq_post_seg* segs, int nseg, int acc_dtype, cons
     if (maxN > TCQ_MAX_WIDTH) return TCQ_ERR_SHAPE;
     if (nseg > 65535) return TCQ_ERR_UNSUPPORTED;
     const bool tw = (maxN & (maxN - 1)) == 0 && maxN >= 256 && maxN <= 4096;
-    const bool wv = M <= 64 && maxN == 2048;                 // few tokens: 2048 / 256-wide segments on the no-transpose engine
+    const bool wv = M <= 384 && maxN == 2048;                // few tokens: 2048 / 256-wide segments on the no-transpose engine
     const dim3 grid(M, nseg), block(wv ? 512 : tw ? maxN / 16 : row_threads(M * nseg, maxN));
     const size_t sh = row_lds(maxN);
     hipStream_t st = (hipStream_t)stream;
@@ -1899,12 +1900,14 @@ extern "C" int tcq_post_group(const tcq_post_seg* segs, int nseg, int acc_dtype,
     // widest segment a power of two of 256 .. 4096: the register + transpose engine (16 values per thread) for the
     // power-of-two segments; measured on MI355X for q / k / v of 2048 / 256 / 256 at 50 tokens: 3.5 us against 4.1 on LDS
     const bool tw = (maxN & (maxN - 1)) == 0 && maxN >= 256 && maxN <= 4096;
-    // few tokens and segments of 256 / 2048 only, 16-byte aligned: the no-transpose engine (k_postg_wv)
+    // few tokens and segments of 256 / 2048 only, 16-byte aligned: the no-transpose engine (k_postg_wv); with more the 256-wide
+    // segments' idle waves cost it more than its fewer exchanges save (q / k / v on MI355X, us against the transpose engine: 256
+    // tokens 3.55 / 4.0, 400: 4.3 / 4.3, 968: 7.35 / 6.1), so any number of tokens only without such segments
     const int esz = dsize(acc_dtype), ysz = dsize(y_dtype);
-    bool wv = M <= 64;
+    bool wv = true;
     for (int i = 0; i < nseg; ++i) {
         const tcq_post_seg& g = segs[i];
-        wv = wv && (g.N == 256 || g.N == 2048) && al16(g.acc) && ((size_t)g.lda * esz) % 16 == 0 && ((size_t)g.col0 * esz) % 16 == 0 &&
+        wv = wv && ((g.N == 256 && M <= 384) || (g.N == 2048 && (M <= 384 || nseg == 1))) && al16(g.acc) && ((size_t)g.lda * esz) % 16 == 0 && ((size_t)g.col0 * esz) % 16 == 0 &&
              al16(g.y) && al16(g.sv) && (!g.rs || al16(g.rs)) && (!g.bias || al16(g.bias)) && ysz >= 2;
     }
     bool tw5 = maxN == 8192 || maxN == 16384;
@@ -2052,8 +2055,10 @@ extern "C" int tcq_post_add_norm_pre(const void* acc, int acc_dtype, int lda, in
     // register + transpose engine, 16 values per thread: power-of-two rows of 1024 .. 4096, aligned (measured on MI355X
     // against the register path: 50 x 1024 5.4 us against 6.9, 1 x 2048 5.7 against 7.5, 800 x 4096 13.7 against 19.5; with
     // 32 values per thread 2048-wide rows of few tokens run slower than the register path)
-    // few rows of 1024 / 2048 with the norm: the no-transpose engine, 4 values per thread on 4 / 8 waves
-    if (M <= 64 && w && !bias && (N == 1024 || N == 2048) && vec && svec && (!q || al16(q))) {
+    // few rows of 1024 / 2048 with the norm: the no-transpose engine, 4 values per thread on 4 / 8 waves, until its waves fill
+    // the chip (us on MI355X against the transpose engine: 256 x 2048 4.9 / 6.1, 400: 6.4 / 6.7, 600: 8.1 / 7.3; 600 x 1024 5.2 /
+    // 5.7, 800: 5.85 / 5.9, 968: 6.0 / 5.9)
+    if ((size_t)M * N <= 860000 && w && !bias && (N == 1024 || N == 2048) && vec && svec && (!q || al16(q))) {
 #define PANV(AD, L, NWP) launch_k(k_post_add_norm_pre_wv<AD, L, NWP>, dim3(M), dim3(64 * NWP), 0, st, acc, lda, col0, s, rs,   \
                                   (const i8*)sv, xp, (u16*)xout, wp, eps, (const i8*)su, (i8*)q, (int*)q4, ldq, scale, parts)
 #define PANVW(L, NWP)                                    \
