@@ -1135,7 +1135,7 @@ __device__ __forceinline__ void postg_wv_seg(const tcq_post_seg& S, int tok, flo
                                                    (u32)f32_to_f16(v[2]) | ((u32)f32_to_f16(v[3]) << 16)};
     }
 }
-// tcq_post of few rows 256 / 1024 / 2048 wide with 16-byte aligned operands on the no-transpose engine: one workgroup of
+// tcq_post of rows 256 / 1024 / 2048 wide with 16-byte aligned operands on the no-transpose engine: one workgroup of
 // 2^L / 256 waves per token (postg_wv_seg's steps).
 template <int ADT, int YDT, int L, int NWP>
 __global__ __launch_bounds__(64 * NWP) void k_post_wv(const void* acc, int lda, int col0, const float* s, const float* rs, const i8* sv,
