@@ -16,15 +16,18 @@
 // 37.1 us at 800 x 2048 x 16384), HBM -> LDS by buffer_load_dwordx4 ... lds without registers, into two rings: NSX steps of
 // activations, NSW of weights. Weights come from HBM and activations from the caches, so the 160 KiB of a 256 x 256 tile
 // hold three steps of weights and two of activations. A load fills 8 rows x 128 bytes; lane p writes position p, which holds
-// row p / 8 and 16-byte granule (p % 8) ^ f(row), f = the row's low three bits with bit 3 folded in, so that the rows of a
-// fragment read (consecutive, or interleaved for BF16 outputs) fall into different banks.
+// row p / 8 and 16-byte granule (p % 8) ^ turn(row). A fragment read takes 256 bytes of LDS a cycle, 16 lanes: two rows' width,
+// so the 8 even rows of a fragment, and its 8 odd ones, need 8 turns: 16 rows in a row bits 1 .. 3, the interleaved rows of BF16
+// outputs bits 1, 3 and 4, served together by bits 1, 3 and 2 ^ 4. Turns from the low three bits cost every read 4 extra
+// cycles of 8: without them a BF16 layer of 968 tokens takes 424 us against 432, INT8 at 800 x 2048 x 16384 the same 32.5.
 // A step runs in four quarters (k half x half of the wave's weight blocks); the fragment reads of the next quarter and the
 // loads of later steps are scheduled between the MFMAs of this one. The one barrier of a step stands before its last
 // quarter, whose fragments are in registers by then: it publishes the next step and frees this one, with MFMAs on both sides.
 // Rows past M / N and columns past K read zeros; waves whose tokens are all padding only load.
 // What bounds it (256 x 256, INT8, K long enough): 1.5 us per step, 2.8 POP/s; the MFMAs alone take 1.05 us, the loads and
-// fragment reads alone 0.7 (in cache) to 1.2 us (streaming): LDS cycles (fragment reads 1536 + loads 512 against 2048 MFMA
-// cycles per step) and power. One wave per SIMD with 128 x 128 each (a third fewer fragment reads) measured the same.
+// fragment reads alone 0.7 (in cache) to 1.2 us (streaming), and power: the matrix cores are busy 47 % of the cycles, at about
+// 1.8 GHz. Not the LDS: its reads are 18 % of the cycles and halving them changed nothing. One wave per SIMD with 128 x 128
+// each (a third fewer fragment reads) measured the same.
 #include "tcq_device.h"
 #include "tcq_launch.h"
 
@@ -90,17 +93,20 @@ __global__ __launch_bounds__(64 * WN * WM) void k_gemm_i8(const void* x_, const 
     const int nkall = (K + 127) >> 7, per = (nkall + parts - 1) / parts, kb = blockIdx.z * per;
     const int nk = min(per, nkall - kb), kend = min(K, 128 * (kb + nk));
 
+    // granule g of a row lies at position g ^ turn (of its row in the tile)
+    auto turn_x = [](int r) { return (r >> 1) & 7; };
+    auto turn_w = [](int r) { return ((r >> 1) & 1) | ((r >> 2) & 2) | (((r ^ (r >> 2)) & 4)); };
     // load u of a wave fills block (wave * L + u) of 8 rows: lane p writes position p, which holds row p / 8, slot p % 8
     const int prow = lane >> 3;
     u32 offw[WL], offx[XL];
 #pragma unroll
     for (int u = 0; u < WL; ++u) {
-        const int blk = wave * WL + u, row = n0 + 8 * blk + prow, g = (lane & 7) ^ prow ^ ((blk & 1) << 2);
+        const int blk = wave * WL + u, row = n0 + 8 * blk + prow, g = (lane & 7) ^ turn_w(8 * blk + prow);
         offw[u] = row < N ? (u32)row * (u32)K + 16u * g : RSRC_OOB;
     }
 #pragma unroll
     for (int u = 0; u < XL; ++u) {
-        const int blk = wave * XL + u, row = m0 + 8 * blk + prow, g = (lane & 7) ^ prow ^ ((blk & 1) << 2);
+        const int blk = wave * XL + u, row = m0 + 8 * blk + prow, g = (lane & 7) ^ turn_x(8 * blk + prow);
         offx[u] = row < M ? (u32)row * (u32)K + 16u * g : RSRC_OOB;
     }
     // loads of K step kt: the row offsets stay in registers, the step is the scalar offset; only the last, partial step of K (and
@@ -120,7 +126,7 @@ __global__ __launch_bounds__(64 * WN * WM) void k_gemm_i8(const void* x_, const 
 #pragma unroll
             for (int u = 0; u < WL; ++u) {
                 char* dst = st + u * 1024;
-                const int g = (lane & 7) ^ prow ^ (((wave * WL + u) & 1) << 2);
+                const int g = (lane & 7) ^ turn_w(8 * (wave * WL + u) + prow);
                 const u32 off = (k + 16 * g < kend) ? offw[u] + (u32)k : RSRC_OOB;
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(RW, (__attribute__((address_space(3))) void*)dst, 16, off, 0, 0, 0);
             }
@@ -140,7 +146,7 @@ __global__ __launch_bounds__(64 * WN * WM) void k_gemm_i8(const void* x_, const 
 #pragma unroll
             for (int u = 0; u < XL; ++u) {
                 char* dst = st + u * 1024;
-                const int g = (lane & 7) ^ prow ^ (((wave * XL + u) & 1) << 2);
+                const int g = (lane & 7) ^ turn_x(8 * (wave * XL + u) + prow);
                 const u32 off = (k + 16 * g < kend) ? offx[u] + (u32)k : RSRC_OOB;
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(RX, (__attribute__((address_space(3))) void*)dst, 16, off, 0, 0, 0);
             }
@@ -172,14 +178,13 @@ __global__ __launch_bounds__(64 * WN * WM) void k_gemm_i8(const void* x_, const 
     // weight row of A row r of block i: BF16 outputs pair the blocks so that a lane ends with 8 consecutive columns
     constexpr bool PAIR = ODT == TCQ_BF16;
     auto wrow = [&](int i) { return PAIR ? 32 * (i >> 1) + 8 * (lr >> 2) + 4 * (i & 1) + (lr & 3) : 16 * i + lr; };
-    auto slot = [&](int row, int g) { return row * 128 + 16 * (g ^ (row & 7) ^ (((row >> 3) & 1) << 2)); };
     // rows 32 apart share their slot pattern: two (PAIR) or one base offsets per k half, the rest constants
     int fw[2][2], fx[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-        fw[h][0] = slot(wrow(0), 4 * h + lg);
-        fw[h][1] = slot(wrow(1), 4 * h + lg);
-        fx[h] = slot(lr, 4 * h + lg);
+        fw[h][0] = wrow(0) * 128 + 16 * ((4 * h + lg) ^ turn_w(wrow(0)));
+        fw[h][1] = wrow(1) * 128 + 16 * ((4 * h + lg) ^ turn_w(wrow(1)));
+        fx[h] = lr * 128 + 16 * ((4 * h + lg) ^ turn_x(lr));
     }
     acc_t acc[NB][MB];
 #pragma unroll
