@@ -79,3 +79,30 @@ def test_bf16_parts_against_fp64(M, N, K, parts):
     sw = torch.rand(N, device=DEV) + 0.01
     assert torch.equal(Kn.gemm_bf16_parts(a, w, torch.empty(M, N, device=DEV), parts, sw=sw), z * sw)
     assert torch.equal(Kn.gemm_bf16_parts(a, w, torch.empty(M, N, dtype=torch.bfloat16, device=DEV), parts), z.bfloat16())
+
+
+@pytest.mark.parametrize('parts', [1, 2, 4])
+@pytest.mark.parametrize('M,N,K', [(65, 64, 128), (80, 68, 1024), (129, 132, 2048), (65, 64, 16384)])
+def test_bf16_infinite_operands_and_sums(M, N, K, parts):
+    """An infinite activation in each K chain's range, and products whose sums pass the largest FP32 value, give the infinities
+    (of one sign each, every weight positive) that any FP32 accumulation gives; a NaN stays one, other tokens are untouched."""
+    from yanlongvla_amd import kernels as Kn
+    if parts > 1 and K < 1024:
+        pytest.skip('K parts start at 1024 columns')
+    g = torch.Generator(device=DEV).manual_seed(K)
+    a, w = torch.randn(M, K, generator=g, device=DEV).bfloat16(), _ints(N, K, seed=9).abs().clamp(min=1).bfloat16()
+    out = torch.empty(M, N, device=DEV)
+    run = lambda: (Kn.gemm_bf16(a, w, out) if parts == 1 else Kn.gemm_bf16_parts(a, w, out, parts)).clone()
+    finite = run()
+    cols = [0, 63, 64, K // 3, K // 2, K - 65, K - 1]
+    inf = float('inf')
+    for i, c in enumerate(cols):
+        a[i, c] = inf if i % 2 == 0 else -inf
+    a[10], a[11] = 3e38, -3e38
+    a[12, K // 3] = float('nan')
+    got = run()
+    for i in range(len(cols)):
+        assert bool((got[i] == (inf if i % 2 == 0 else -inf)).all()), cols[i]
+    assert bool((got[10] == inf).all()) and bool((got[11] == -inf).all()) and bool(got[12].isnan().all())
+    others = [i for i in range(M) if not (i < len(cols) or 10 <= i <= 12)]
+    assert torch.equal(got[others], finite[others])

@@ -271,9 +271,12 @@ __global__ __launch_bounds__(64 * WN * WM) void k_gemm_i8(const void* x_, const 
             for (int i = 0; i < NB; ++i)
 #pragma unroll
                 for (int j = 0; j < MB; ++j) {
-                    const acc_t t = sum[i][j] + acc[i][j];
-                    acc[i][j] = acc[i][j] - (t - sum[i][j]);
-                    sum[i][j] = t;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float a = sum[i][j][e], b = acc[i][j][e], t = a + b, r = b - (t - a);
+                        acc[i][j][e] = fabsf(t) < __builtin_inff() ? r : 0.f;    // an infinite sum stays one (inf - inf is a NaN)
+                        sum[i][j][e] = t;
+                    }
                 }
         }
 #pragma unroll
