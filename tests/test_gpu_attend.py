@@ -107,3 +107,37 @@ def test_many_causal_tokens(M, P, H, causal):
     K.attend(q, kc, vc, kn, vn, H, causal, su=su, q8=q1, scale=s1)
     K.pre(o, su, q=q2, scale=s2)
     assert torch.equal(q1, q2) and torch.equal(s1, s2)
+
+
+def _near_ties(n):
+    """n FP32 distances d whose exp(-d) lies within a few 1e-6 of the midpoint of two BF16 values, on the other side of it than
+    2^(d log2 e) with the product rounded to FP32, and more than 2.4e-7 (two FP32 ulps) from it on both sides."""
+    d = np.random.default_rng(0).uniform(45, 80, 1 << 22).astype(np.float32)
+    right, coarse = np.exp(-d.astype(np.float64)), np.exp2((-d * np.float32(np.log2(np.e))).astype(np.float64))
+    half = np.exp2(np.floor(np.log2(right)) - 8)                               # half a BF16 ulp
+    tie = (np.floor(right / (2 * half)) + 0.5) * 2 * half
+    apart = 2.4e-7 * right
+    found = d[(np.abs(right - tie) > apart) & (np.abs(coarse - tie) > apart) & ((right > tie) != (coarse > tie))]
+    assert len(found) >= n
+    return torch.from_numpy(found[:n])
+
+
+def test_many_causal_tokens_exponentials():
+    """The probabilities of k_attn_rows are FP32 exponentials of at most one ulp, as everywhere else: with one key at the maximum
+    (value 0) and one at distance d (value 1), an output is bf16(exp(-d)), here for distances next to a rounding boundary."""
+    from yanlongvla_amd import kernels as K
+    M, H = 256, 8
+    d = _near_ties(512).repeat(4).view(M, H)
+    q, rest = torch.zeros(M, H, 256), d.clone()
+    for i in range(3):                                                         # the distance in three exact BF16 pieces
+        piece = rest.bfloat16().float()
+        q[:, :, i], rest = -16 * piece, rest - piece
+    assert not rest.any()
+    q[:, :, 3] = -65536                                                        # the call's own keys: 4096 below the maximum
+    kc, vc, kn = torch.zeros(2, 256), torch.zeros(2, 256), torch.zeros(M, 256)
+    kc[1, :3], vc[1], kn[:, 3] = 1, 1, 1
+    q, kc, vc, kn = (t.bfloat16().to(DEV) for t in (q.view(M, H * 256), kc, vc, kn))
+    o = torch.empty_like(q)
+    K.attend(q, kc, vc, kn, torch.zeros_like(kn), H, 2, o=o)
+    want = torch.exp(-d.double()).bfloat16()
+    assert torch.equal(o.view(M, H, 256).cpu(), want[:, :, None].expand(M, H, 256))

@@ -18,8 +18,9 @@ namespace {
 
 constexpr int AT = 256;          // threads of k_attn_part
 // Causal tokens from which k_attn_rows runs: where its launch of the rotate + quantize, which the combine has fused, is paid
-// back, for both kinds of call so that they round the same outputs. Outputs only, us before / after: 256 tokens 13.4 / 10.4,
-// 968: 53.2 / 33.0. Quantized: 130 tokens 11.9 / 13.6, 256: 15.0 / 14.9, 400: 20.9 / 18.5, 968: 53.9 / 37.6.
+// back, for both kinds of call so that they round the same outputs. MI355X, us on the chunks / on k_attn_rows, outputs only: 256
+// tokens 13.1 / 11.0, 400: 18.9 / 15.6, 968: 52 / 34.4. Quantized: 130 tokens 11.9 / 13.6, 256: 14.6 / 14.5, 400: 20.7 / 19.4, 968:
+// 54.3 / 39.2.
 constexpr int ATTN_ROWS_M = 256;
 
 __device__ __forceinline__ const u16* key_row(const u16* cache, const u16* fresh, int P, int j) {
@@ -492,12 +493,13 @@ __global__ __launch_bounds__(128) void k_attn_combine_reg(const float* part, int
 // fragments; values are transposed 8 x 8 in registers and pass through a wave-private LDS tile (dim row (i, dg) = dim 8 dg + i
 // at i VTI + 80 dg, 16 bytes per lane group in one of five slots turned by i: writes and reads spread over all banks), so the
 // loop has no barrier. Scores, exponentials, sums and outputs in FP32, the probabilities rounded to BF16 for the second
-// product, as in k_attn_part.
+// product, as in k_attn_part. The exponentials are expf there and here: 2^(d log2 e) on the hardware instruction, 3 % of the time
+// less (33.2 / 28.0 / 15.1 us at 968 / 800 / 400 tokens), is off by the rounded product, 2.6e-6 of a probability at d = 80.
 // What bounds it: instruction issue; a block of 32 keys is 32 MFMAs in some 500 instructions a wave (without its loads it
 // still takes four fifths of the time), so two workgroups per CU (256 registers, 80 KiB of LDS each) hide each other's
-// waits: groups of 4 tokens need all 512 registers, one workgroup per CU, and measured 33 / 29 / 20 us at 968 / 800 / 400
-// causal tokens against 33 / 26 / 14 here. k_attn_part, which writes and reads back 66 MB of chunk partials at 968 tokens,
-// took 53 / 41 / 19 with its combine. Error against 64 bits (968 tokens, normal inputs): 1.96e-3 against 1.98e-3.
+// waits: groups of 4 tokens need all 512 registers, one workgroup per CU, and took 29 / 20 us at 800 / 400 causal tokens where
+// pairs took 26 / 14 (both with the hardware exponential). Now 34.4 / 29.0 / 15.6 at 968 / 800 / 400; k_attn_part, which writes and
+// reads back 66 MB of chunk partials at 968 tokens, takes 52 / 41 / 19 with its combine. Error against 64 bits (968 tokens, normal inputs): 1.96e-3 against 1.98e-3.
 constexpr int VTI = 32 * 80, VTW = 8 * VTI;                   // bytes between dims i, i + 1 of a group; a wave's tile
 
 __global__ __launch_bounds__(256, 2) void k_attn_rows(const u16* q, const u16* kc, const u16* vc, int P, const u16* kn, const u16* vn,
@@ -563,7 +565,6 @@ __global__ __launch_bounds__(256, 2) void k_attn_rows(const u16* q, const u16* k
 #pragma unroll
     for (int tl = 0; tl < 16; ++tl) O[tl] = float4_t{0.f, 0.f, 0.f, 0.f};
     const int all_see = visible_end(t0);                             // keys below it are visible to the whole group
-    constexpr float L2E = 1.44269504088896341f;
     int j = 32 * wave;
     if (j < jend) {
         load_k(j);
@@ -613,7 +614,7 @@ __global__ __launch_bounds__(256, 2) void k_attn_rows(const u16* q, const u16* k
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            p[e] = __builtin_amdgcn_exp2f((s[e] - mz) * L2E);
+            p[e] = expf(s[e] - mz);
             l += p[e];
         }
         const uint4_t Pb = {bf16_cvt2(p[0], p[1]), bf16_cvt2(p[2], p[3]), bf16_cvt2(p[4], p[5]), bf16_cvt2(p[6], p[7])};
