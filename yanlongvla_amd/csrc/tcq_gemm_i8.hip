@@ -448,17 +448,25 @@ extern "C" int tcq_gemm_bf16(const void* a, const void* w, const float* sa, cons
     return launch_status();
 }
 
-// FP32 K parts added in order, * sw, to FP32 or BF16: four columns per thread.
+// FP32 K parts added in order, * sw, to FP32 or BF16: four columns per thread. What the additions round away is added at the end,
+// unless the sum is infinite (the launch is bound by memory): each part is rounded once more than a single sum, and with plain
+// additions four parts of K = 1024 were 3 % further from 64 bits than the few-token product's sums.
 template <int ODT>
 __global__ __launch_bounds__(256) void k_sum_parts(const float* part, const float* sw, void* out, size_t n, int N, int parts) {
     const size_t i = 4 * ((size_t)blockIdx.x * 256 + threadIdx.x);
     if (i >= n) return;
-    float4v v = *gptr((const float4v*)(part + i));
+    float4v v = *gptr((const float4v*)(part + i)), c = {0.f, 0.f, 0.f, 0.f};
     for (int p = 1; p < parts; ++p) {
         const float4v u = *gptr((const float4v*)(part + p * n + i));
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = v[e] + u[e];
+        for (int e = 0; e < 4; ++e) {
+            const float t = v[e] + u[e], b = t - v[e];
+            c[e] = c[e] + ((v[e] - (t - b)) + (u[e] - b));
+            v[e] = t;
+        }
     }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = fabsf(v[e]) < __builtin_inff() ? v[e] + c[e] : v[e];
     if (sw) {
         const float4v r = *gptr((const float4v*)(sw + i % N));
 #pragma unroll
@@ -489,7 +497,8 @@ extern "C" int tcq_gemm_bf16_parts(const void* a, const void* w, const float* sw
 
 // As tcq_gemm_i8_best_parts, with 2 us for the launch that adds the parts, and their write and read at 6 TB/s. MI355X, us in 1 / 2 /
 // 4 parts: 968 x 2048 x 16384 105 / 81 / 76, 256: 77 / 45 / 33; 128 x 1024 x 4096 23 / 16 / 12; 400 x 2048 x 2048 14.3 / 15.0 / 17.5.
-// Relative error against 64 bits, 968 x 2048 x 16384: 8.9e-8, 9.3e-8, 9.7e-8 (the few-token product's partial sums: 1.18e-7).
+// Relative error against 64 bits, 968 x 2048 x 16384: 8.9e-8, 9.3e-8, 9.2e-8 (the few-token product's partial sums: 1.18e-7); 65 x 1024 x
+// 1024: 4.9e-8, 5.5e-8, 5.0e-8 (5.7e-8).
 extern "C" int tcq_gemm_bf16_best_parts(int M, int N, int K) {
     if (M <= 64 || N <= 0 || K < 64 * 16) return 1;
     int best = 1;
