@@ -98,3 +98,34 @@ def test_epilogue_and_plain_middle(N, M, adt):
     Kn.mid1(acc.to(DEV), ds, drs, T[2], T[3], T[4], q=q, scale=sc)
     wq, ws = O.quantize_tokens(O.fwht(O.bf16_to_f32(act) * su.astype(f32)))
     assert np.array_equal(sc.cpu().numpy(), ws[:, 0]) and np.array_equal(q.cpu().numpy(), wq)
+
+
+@pytest.mark.parametrize('adt', [torch.int32, torch.float32, torch.bfloat16])
+@pytest.mark.parametrize('N,M', [(4096, 256), (4096, 257), (4096, 513), (6144, 256), (6144, 257), (4608, 256), (4608, 257), (2048, 256), (2048, 257)])
+def test_rows_around_the_lines_between_engines(N, M, adt):
+    """Widths and row counts where calls change between the wave rows and the LDS engine: each row as in calls of 40, whole
+    vectors and (columns 8 bytes off) not; epilogues alone and in a group, the plain middle, column scales."""
+    from yanlongvla_amd import kernels as Kn
+    g = torch.Generator(device=DEV).manual_seed(N + M)
+    r = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    sign = lambda n: torch.where(r(n) > 0, 1, -1).to(torch.int8)
+    acc, x, cs = (r(M, N + 8) * 1000).to(adt), r(M, N).bfloat16(), (torch.rand(N, generator=g, device=DEV) + 0.5).half()
+    sv, su, bias, rs, s = sign(N), sign(N), r(N), torch.rand(N, generator=g, device=DEV) + 0.1, torch.rand(M, generator=g, device=DEV) + 0.1
+    rs = None if adt == torch.float32 else rs
+
+    def run(a, b):
+        m, st, out = b - a, s[a:b] if adt == torch.int32 else None, []
+        for col0 in (0, 8 // acc.element_size()):
+            y = torch.empty(m, N, dtype=torch.bfloat16, device=DEV)
+            Kn.post(acc[a:b], st, rs, sv, bias, y, col0=col0)
+            ys = [torch.empty(m, N, dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+            Kn.post_group([(acc[a:b], col0, rs, sv, None, t, False) for t in ys], adt, torch.bfloat16, st, m)
+            out += [y] + ys
+        q, sc = torch.empty(m, N, dtype=torch.int8, device=DEV), torch.empty(m, device=DEV)
+        Kn.mid1(acc[a:b, :N].contiguous(), st, rs, sv, bias, su, q=q, scale=sc)
+        q2, sc2 = torch.empty_like(q), torch.empty_like(sc)
+        Kn.pre(x[a:b], su, q=q2, scale=sc2, col_scale=cs)
+        return out + [q, sc, q2, sc2]
+    whole, parts = run(0, M), [run(a, min(a + 40, M)) for a in range(0, M, 40)]
+    for i, t in enumerate(whole):
+        assert torch.equal(t, torch.cat([p[i] for p in parts]))

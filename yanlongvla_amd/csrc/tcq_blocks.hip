@@ -398,6 +398,18 @@ bool takes(int K) { return K % 4 == 0 && K >= 64 && K < 7 * 1024; }
 // Four waves per row from 2048 on (one wave of 17 groups runs 28 us through the plain middle of 768 x 4304), and from 1024 on
 // while the rows leave SIMDs idle
 bool four_waves(int M, int K) { return K >= 2048 || (M <= 256 && K >= 1024); }
+// Wide rows of one block, or of two, that the LDS engine's vectors move faster: few passes with every thread busy, against side
+// vectors read in series here. MI355X, us, LDS engine / wave rows. Epilogues: 64 x 4096 from int32 5.1 / 6.6, from FP32 5.0 / 5.9, 400:
+// 8.6 / 7.9, 968: 9.7 / 10.5; 64 x 6144 with bias from BF16 7.4 / 8.5, from FP32 7.3 / 7.7, 968 from BF16 13.6 / 14.2, from FP32 14.1 /
+// 13.4; 64 x 4608 from BF16 7.3 / 7.8, 400: 9.5 / 9.2. Plain middle: 64 x 4096 9.9 / 11.8, 64 x 2048 8.5 / 9.1, 257 x 4096 16.0 / 13.1.
+// Rotate + quantize with column scales: 64 x 4096 6.2 / 7.1, 257: 10.2 / 7.7. (Its threads per row fall from 257 rows on.)
+bool lds_post(int rows, int N, int acc_dtype) {
+    const bool scaled = acc_dtype != TCQ_F32, two = __builtin_popcount(N) == 2;
+    if (rows <= 256) return N == 4096 || N == 6144 || (N > 4096 && two && scaled);
+    return scaled && (N == 6144 || (N == 4096 && rows > 512));
+}
+bool lds_mid1(int M, int N) { return M <= 256 && (N == 2048 || N == 4096); }
+bool lds_pre(int M, int K, bool cs) { return M <= 256 && cs && K == 4096; }
 
 }  // namespace
 
@@ -417,9 +429,9 @@ bool blocks_rht(const void* x, int x_dtype, int ldx, const i8* su, void* y, int 
     return true;
 }
 
-bool blocks_pre(const void* x, int x_dtype, const i8* su, const u16* cs, i8* q, int* q4, int ldq, float* scale, int M, int K,
+bool blocks_pre(const void* x, int x_dtype, const i8* su, const u16* cs, i8* q, int* q4, int ldq, float* scale, int M, int K, bool lds,
                 hipStream_t st) {
-    if (!takes(K) || !input_type(x_dtype) || !al(x, 4 * bytes_of(x_dtype)) || (su && !al(su, 4)) || (cs && !al(cs, 8)) || (q && !al(q, 4)) ||
+    if (!takes(K) || (lds && lds_pre(M, K, cs)) || !input_type(x_dtype) || !al(x, 4 * bytes_of(x_dtype)) || (su && !al(su, 4)) || (cs && !al(cs, 8)) || (q && !al(q, 4)) ||
         (q4 && !al(q4, 4)))
         return false;
     ROWS_LAUNCH(k_pre_rows, dim3(M), M, K, x, x_dtype, su, cs, q, q4, ldq, scale, K);
@@ -427,13 +439,13 @@ bool blocks_pre(const void* x, int x_dtype, const i8* su, const u16* cs, i8* q, 
 }
 
 bool blocks_post(const tcq_post_seg* segs, int nseg, int acc_dtype, const float* s, const u16* gelu_lut, int y_dtype, int M,
-                 hipStream_t st) {
+                 bool lds, hipStream_t st) {
     if ((acc_dtype != TCQ_F32 && acc_dtype != TCQ_I32 && acc_dtype != TCQ_BF16) || !input_type(y_dtype)) return false;
     PostRows A = {};
     int most = 0;
     for (int i = 0; i < nseg; ++i) {
         const tcq_post_seg& g = segs[i];
-        if (!takes(g.N) || !al(g.acc, 4 * bytes_of(acc_dtype)) || g.lda % 4 || g.col0 % 4 || !al(g.y, 4 * bytes_of(y_dtype)) || !al(g.sv, 4) ||
+        if (!takes(g.N) || (lds && lds_post(M * nseg, g.N, acc_dtype)) || !al(g.acc, 4 * bytes_of(acc_dtype)) || g.lda % 4 || g.col0 % 4 || !al(g.y, 4 * bytes_of(y_dtype)) || !al(g.sv, 4) ||
             (acc_dtype != TCQ_F32 && !al(g.rs, 16)) || (g.bias && !al(g.bias, 16)))
             return false;
         A.s[i] = g;
@@ -446,8 +458,8 @@ bool blocks_post(const tcq_post_seg* segs, int nseg, int acc_dtype, const float*
 }
 
 bool blocks_mid1(const void* acc, int acc_dtype, int lda, const float* s, const float* rs, const i8* sv, const float* bias,
-                 const u16* lut, const i8* su, i8* q, int* q4, int ldq, float* scale, int M, int N, hipStream_t st) {
-    if ((acc_dtype != TCQ_F32 && acc_dtype != TCQ_I32 && acc_dtype != TCQ_BF16) || !takes(N) || !al(acc, 4 * bytes_of(acc_dtype)) || lda % 4 ||
+                 const u16* lut, const i8* su, i8* q, int* q4, int ldq, float* scale, int M, int N, bool lds, hipStream_t st) {
+    if ((acc_dtype != TCQ_F32 && acc_dtype != TCQ_I32 && acc_dtype != TCQ_BF16) || !takes(N) || (lds && lds_mid1(M, N)) || !al(acc, 4 * bytes_of(acc_dtype)) || lda % 4 ||
         !al(sv, 4) || !al(su, 4) || (acc_dtype != TCQ_F32 && !al(rs, 16)) || (bias && !al(bias, 16)) || (q && !al(q, 4)) || (q4 && !al(q4, 4)))
         return false;
     ROWS_LAUNCH(k_mid1_rows, dim3(M), M, N, acc, acc_dtype, lda, s, rs, sv, bias, lut, su, q, q4, ldq, scale, N);

@@ -1536,7 +1536,7 @@ extern "C" int tcq_pre_cs(const void* x, int x_dtype, const int8_t* su, const vo
         return launch_status();
     }
     // rows of several blocks, narrow ones, and column scales
-    if (blocks_pre(x, x_dtype, (const i8*)su, cs, (i8*)q, (int*)q4, ldq, scale, M, K, st)) return launch_status();
+    if (blocks_pre(x, x_dtype, (const i8*)su, cs, (i8*)q, (int*)q4, ldq, scale, M, K, vec, st)) return launch_status();
 #define PRE(XD, _) launch_k(k_pre<XD>, grid, block, sh, st, x, (const i8*)su, (i8*)q, (int*)q4, ldq, scale, K, vec, cs)
     DISPATCH_X(x_dtype, PRE, 0)
 #undef PRE
@@ -1673,6 +1673,13 @@ extern "C" int tcq_post_plain_group(const tcq_post_seg* segs, int nseg, int acc_
     return launch_status();
 }
 
+// whether the LDS engine reads and writes an epilogue segment in whole vectors
+static bool lds_vec(const tcq_post_seg& g, int acc_dtype, int y_dtype) {
+    const size_t asz = dsize(acc_dtype);
+    return g.N % 8 == 0 && al16(g.acc) && (g.lda * asz) % 16 == 0 && (g.col0 * asz) % 16 == 0 && al16(g.y) &&
+           ((size_t)g.N * dsize(y_dtype)) % 16 == 0 && al8(g.sv) && (!g.rs || al16(g.rs)) && (!g.bias || al16(g.bias));
+}
+
 extern "C" int tcq_post(const void* acc, int acc_dtype, int lda, int col0, const float* s, const float* rs, const int8_t* sv,
                         const float* bias, void* y, int y_dtype, int M, int N, tcq_stream_t stream) {
     if (!acc || !y || M <= 0 || N <= 0 || col0 < 0 || lda < col0 + N) return TCQ_ERR_ARG;
@@ -1712,11 +1719,10 @@ extern "C" int tcq_post(const void* acc, int acc_dtype, int lda, int col0, const
     }
     hipStream_t st = (hipStream_t)stream;
     const tcq_post_seg one = {acc, rs, (const i8*)sv, bias, y, lda, col0, N, 0};
-    if (blocks_post(&one, 1, acc_dtype, s, nullptr, y_dtype, M, st)) return launch_status();
+    const int vec = lds_vec(one, acc_dtype, y_dtype);
+    if (blocks_post(&one, 1, acc_dtype, s, nullptr, y_dtype, M, vec, st)) return launch_status();
     const dim3 grid(M), block(row_threads(M, N));
     const size_t sh = row_lds(N);
-    const int vec = N % 8 == 0 && al16(acc) && ((size_t)lda * asz) % 16 == 0 && ((size_t)col0 * asz) % 16 == 0 && al16(y) &&
-                    ((size_t)N * dsize(y_dtype)) % 16 == 0 && al8(sv) && (!rs || al16(rs)) && (!bias || al16(bias));
 #define POST_Y(AD, YD) launch_k(k_post<AD, YD>, grid, block, sh, st, acc, lda, col0, s, rs, (const i8*)sv, bias, y, N, vec)
 #define POST_A(AD)                                           \
     switch (y_dtype) {                                       \
@@ -1858,7 +1864,7 @@ extern "C" int tcq_mid1(const void* acc, int acc_dtype, int lda, const float* s,
     const int svec = al16(sv) && al16(su) && (!bias || al16(bias));
     hipStream_t st = (hipStream_t)stream;
     const i8 *svp = (const i8*)sv, *sup = (const i8*)su;
-    if (blocks_mid1(acc, acc_dtype, lda, s, rs, svp, bias, (const u16*)gelu_lut, sup, (i8*)q, (int*)q4, ldq, scale, M, N, st)) return launch_status();
+    if (blocks_mid1(acc, acc_dtype, lda, s, rs, svp, bias, (const u16*)gelu_lut, sup, (i8*)q, (int*)q4, ldq, scale, M, N, vec && svec, st)) return launch_status();
     switch (acc_dtype) {
         case TCQ_I32: launch_k(k_mid1<TCQ_I32>, grid, block, sh, st, acc, lda, s, rs, svp, bias, gelu_lut, sup, (i8*)q, (int*)q4, ldq, scale, N, vec, svec); break;
         case TCQ_F32: launch_k(k_mid1<TCQ_F32>, grid, block, sh, st, acc, lda, s, rs, svp, bias, gelu_lut, sup, (i8*)q, (int*)q4, ldq, scale, N, vec, svec); break;
@@ -1940,7 +1946,9 @@ extern "C" int tcq_post_group(const tcq_post_seg* segs, int nseg, int acc_dtype,
         return launch_status();
     }
     // segments of several blocks: rows in the registers of a wave or four
-    if (!wv && !tw && blocks_post(segs, nseg, acc_dtype, s, (const u16*)gelu_lut, y_dtype, M, (hipStream_t)stream)) return launch_status();
+    bool lds = true;
+    for (int i = 0; i < nseg; ++i) lds = lds && lds_vec(segs[i], acc_dtype, y_dtype);
+    if (!wv && !tw && blocks_post(segs, nseg, acc_dtype, s, (const u16*)gelu_lut, y_dtype, M, lds, (hipStream_t)stream)) return launch_status();
     const dim3 grid(M, nseg), block(wv ? 512 : tw ? maxN / 16 : row_threads(M * nseg, maxN));
     // no dynamic LDS for k_postg_wv here: its own checks equal the ones above, so it never takes its LDS fallback
     const size_t sh = wv ? 0 : row_lds(maxN);
