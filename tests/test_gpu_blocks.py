@@ -129,3 +129,32 @@ def test_rows_around_the_lines_between_engines(N, M, adt):
     whole, parts = run(0, M), [run(a, min(a + 40, M)) for a in range(0, M, 40)]
     for i, t in enumerate(whole):
         assert torch.equal(t, torch.cat([p[i] for p in parts]))
+
+
+@pytest.mark.parametrize('widths', [(2048, 1024, 1024), (2048, 256, 256), (2048, 2048), (2048,), (8192, 8192), (16384,)])
+@pytest.mark.parametrize('M', [64, 65, 256, 257, 384, 385, 512, 513])
+def test_group_epilogues_around_the_lines(widths, M):
+    """Epilogue groups where row counts, widths and types change the engine, segments in the launch and in device memory: the
+    rows of tcq_post in calls of 40."""
+    from yanlongvla_amd import kernels as Kn
+    g = torch.Generator(device=DEV).manual_seed(M + sum(widths))
+    r = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    s = torch.rand(M, generator=g, device=DEV) + 0.1
+    for adt in (torch.int32, torch.float32, torch.bfloat16):
+        acc = (r(M, sum(widths)) * 1000).to(adt)
+        st = s if adt == torch.int32 else None
+        for ydt in (torch.bfloat16, torch.float32):
+            segs, want, c = [], [], 0
+            for n in widths:
+                sv, rs = torch.where(r(n) > 0, 1, -1).to(torch.int8), None if adt == torch.float32 else torch.rand(n, generator=g, device=DEV)
+                segs.append((acc, c, rs, sv, None, torch.empty(M, n, dtype=ydt, device=DEV), False))
+                want.append(torch.empty(M, n, dtype=ydt, device=DEV))
+                for a in range(0, M, 40):
+                    Kn.post(acc[a:a + 40], None if st is None else st[a:a + 40], rs, sv, None, want[-1][a:a + 40], col0=c)
+                c += n
+            Kn.post_group(segs, adt, ydt, st, M)
+            assert all(torch.equal(t[5], w) for t, w in zip(segs, want))
+            for t in segs:
+                t[5].zero_()
+            Kn.post_batched(Kn.post_segments(segs, DEV), len(segs), adt, ydt, st, M, max(widths))
+            assert all(torch.equal(t[5], w) for t, w in zip(segs, want))

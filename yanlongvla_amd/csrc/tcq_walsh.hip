@@ -1747,7 +1747,9 @@ extern "C" int tcq_postg(const tcq_post_seg* segs, int nseg, int acc_dtype, cons
     if (maxN > TCQ_MAX_WIDTH) return TCQ_ERR_SHAPE;
     if (nseg > 65535) return TCQ_ERR_UNSUPPORTED;
     const bool tw = (maxN & (maxN - 1)) == 0 && maxN >= 256 && maxN <= 4096;
-    const bool wv = M <= 384 && maxN == 2048;                // few tokens: 2048 / 256-wide segments on the no-transpose engine
+    // few tokens: 2048 / 256-wide segments on the no-transpose engine. No more tokens than 64: the descriptors are in device memory,
+    // and segments of other widths go through the LDS inside that kernel (2048 | 1024 | 1024 at 300 tokens 8.8 us against 4.5)
+    const bool wv = M <= 64 && maxN == 2048;
     const dim3 grid(M, nseg), block(wv ? 512 : tw ? maxN / 16 : row_threads(M * nseg, maxN));
     const size_t sh = row_lds(maxN);
     hipStream_t st = (hipStream_t)stream;
