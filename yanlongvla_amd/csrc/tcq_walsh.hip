@@ -934,18 +934,17 @@ __global__ void k_postg_tw(SEGS segs, const float* s, const u16* gelu_lut, int m
     store_post_row<YDT>(lds, S.y, (size_t)tok * N, S.sv, S.bias, gl, N, vec);
 }
 
-// The same for groups of segments 2^L wide only (8192, 16384; 32 values per thread, 16-byte aligned, checked by the host).
-// Two BF16 rows of 16384 at 968 tokens: 59 us through the LDS engine.
+// The same for groups of segments 2^L wide only (8192, 16384; 32 values per thread, 16-byte aligned, FP32 or BF16 sums, 16-bit
+// outputs, checked by the host).
 template <int ADT, int YDT, int L>
-__global__ __launch_bounds__(1 << (L - 5)) void k_postg_tw5(PostPack segs, const float* s, const u16* gelu_lut) {
+__global__ __launch_bounds__(1 << (L - 5)) void k_postg_tw5(PostPack segs, const u16* gelu_lut) {
     extern __shared__ float lds[];
     const tcq_post_seg S = segs[blockIdx.y];
     const int tok = blockIdx.x, i0 = 32 * threadIdx.x;
-    const float st = ADT == TCQ_I32 ? s[tok] : 1.f;
     float v[32];
 #pragma unroll
     for (int h = 0; h < 2; ++h)
-        acc_chunk<ADT>(S.acc, (size_t)tok * S.lda + S.col0 + i0 + 16 * h, st, S.rs ? S.rs + i0 + 16 * h : nullptr, part16(v, h));
+        acc_chunk<ADT>(S.acc, (size_t)tok * S.lda + S.col0 + i0 + 16 * h, 1.f, S.rs ? S.rs + i0 + 16 * h : nullptr, part16(v, h));
     const Raw16<1> sv[2] = {raw16<1>(S.sv + i0, true), raw16<1>(S.sv + i0 + 16, true)};
     tw_walsh<L, 5>(v, lds);
     const float c = (float)(1.0 / __builtin_sqrt((double)(1 << L)));
@@ -1908,17 +1907,22 @@ extern "C" int tcq_post_group(const tcq_post_seg* segs, int nseg, int acc_dtype,
     // widest segment a power of two of 256 .. 4096: the register + transpose engine (16 values per thread) for the
     // power-of-two segments; measured on MI355X for q / k / v of 2048 / 256 / 256 at 50 tokens: 3.5 us against 4.1 on LDS
     const bool tw = (maxN & (maxN - 1)) == 0 && maxN >= 256 && maxN <= 4096;
-    // few tokens and segments of 256 / 2048 only, 16-byte aligned: the no-transpose engine (k_postg_wv); with more the 256-wide
-    // segments' idle waves cost it more than its fewer exchanges save (q / k / v on MI355X, us against the transpose engine: 256
-    // tokens 3.55 / 4.0, 400: 4.3 / 4.3, 968: 7.35 / 6.1), so any number of tokens only without such segments
+    // few tokens and segments of 256 / 2048 only, 16-byte aligned: the no-transpose engine (k_postg_wv), up to 512 rows of 2048 and
+    // 384 tokens with 256-wide segments. With more, eight waves a row (most of them idle for a 256-wide one) cost it more than its
+    // fewer exchanges save. MI355X, us against the transpose engine: q / k / v 256 tokens 3.55 / 4.0, 400: 4.3 / 4.3, 968: 7.35 /
+    // 6.1; one segment of 2048 from FP32, 600 rows 4.6 / 4.45, 800: 5.3 / 4.7; three of them, 200 tokens 4.55 / 4.4, 350: 6.0 / 5.1
     const int esz = dsize(acc_dtype), ysz = dsize(y_dtype);
-    bool wv = true;
+    int rows = 0;
+    for (int i = 0; i < nseg; ++i) rows += segs[i].N == 2048 ? M : 0;
+    bool wv = rows <= 512;
     for (int i = 0; i < nseg; ++i) {
         const tcq_post_seg& g = segs[i];
-        wv = wv && ((g.N == 256 && M <= 384) || (g.N == 2048 && (M <= 384 || nseg == 1))) && al16(g.acc) && ((size_t)g.lda * esz) % 16 == 0 && ((size_t)g.col0 * esz) % 16 == 0 &&
+        wv = wv && ((g.N == 256 && M <= 384) || g.N == 2048) && al16(g.acc) && ((size_t)g.lda * esz) % 16 == 0 && ((size_t)g.col0 * esz) % 16 == 0 &&
              al16(g.y) && al16(g.sv) && (!g.rs || al16(g.rs)) && (!g.bias || al16(g.bias)) && ysz >= 2;
     }
-    bool tw5 = maxN == 8192 || maxN == 16384;
+    // 8192 or 16384 alone, unscaled or BF16 sums to 16-bit outputs: the transpose engine with 32 values per thread (us against the LDS
+    // engine: 968 x 2 x 16384 from FP32 41 / 50.6, from BF16 41 / 47.9; int32 sums 55.5 / 52.4, FP32 outputs 60.4 / 56.6)
+    bool tw5 = (maxN == 8192 || maxN == 16384) && acc_dtype != TCQ_I32 && y_dtype != TCQ_F32;
     for (int i = 0; i < nseg; ++i) {
         const tcq_post_seg& g = segs[i];
         tw5 = tw5 && g.N == maxN && al16(g.acc) && ((size_t)g.lda * esz) % 16 == 0 && ((size_t)g.col0 * esz) % 16 == 0 && al16(g.y) &&
@@ -1928,17 +1932,15 @@ extern "C" int tcq_post_group(const tcq_post_seg* segs, int nseg, int acc_dtype,
         const dim3 g5(M, nseg);
         const hipStream_t st5 = (hipStream_t)stream;
 #define POST5_Y(AD, YD)                                                                                                    \
-    if (maxN == 8192) launch_k(k_postg_tw5<AD, YD, 13>, g5, dim3(256), row_lds(8192), st5, pk, s, (const u16*)gelu_lut);   \
-    else launch_k(k_postg_tw5<AD, YD, 14>, g5, dim3(512), row_lds(16384), st5, pk, s, (const u16*)gelu_lut)
+    if (maxN == 8192) launch_k(k_postg_tw5<AD, YD, 13>, g5, dim3(256), row_lds(8192), st5, pk, (const u16*)gelu_lut);      \
+    else launch_k(k_postg_tw5<AD, YD, 14>, g5, dim3(512), row_lds(16384), st5, pk, (const u16*)gelu_lut)
 #define POST5_A(AD)                                          \
     switch (y_dtype) {                                       \
-        case TCQ_F32: POST5_Y(AD, TCQ_F32); break;           \
         case TCQ_BF16: POST5_Y(AD, TCQ_BF16); break;         \
         case TCQ_F16: POST5_Y(AD, TCQ_F16); break;           \
         default: return TCQ_ERR_DTYPE;                       \
     }
         switch (acc_dtype) {
-            case TCQ_I32: POST5_A(TCQ_I32); break;
             case TCQ_F32: POST5_A(TCQ_F32); break;
             case TCQ_BF16: POST5_A(TCQ_BF16); break;
             default: return TCQ_ERR_DTYPE;
