@@ -126,8 +126,8 @@ def test_many_causal_tokens_exponentials():
     """The probabilities of k_attn_rows are FP32 exponentials of at most one ulp, as everywhere else: with one key at the maximum
     (value 0) and one at distance d (value 1), an output is bf16(exp(-d)), here for distances next to a rounding boundary."""
     from yanlongvla_amd import kernels as K
-    M, H = 256, 8
-    d = _near_ties(512).repeat(4).view(M, H)
+    M, H = 288, 8
+    d = _near_ties(512).repeat(5)[:M * H].view(M, H)
     q, rest = torch.zeros(M, H, 256), d.clone()
     for i in range(3):                                                         # the distance in three exact BF16 pieces
         piece = rest.bfloat16().float()
@@ -141,3 +141,10 @@ def test_many_causal_tokens_exponentials():
     K.attend(q, kc, vc, kn, torch.zeros_like(kn), H, 2, o=o)
     want = torch.exp(-d.double()).bfloat16()
     assert torch.equal(o.view(M, H, 256).cpu(), want[:, :, None].expand(M, H, 256))
+
+
+@pytest.mark.parametrize('M,P,H,causal', [(287, 31, 8, 31), (289, 31, 5, 31), (290, 64, 8, 3), (291, 1, 8, 400), (288, 33, 7, 33), (511, 0, 4, 0),
+                                          (513, 40, 3, 40), (967, 5, 2, 5), (969, 31, 2, 31), (970, 0, 1, 0)])
+def test_many_causal_tokens_by_heads_and_cache(M, P, H, causal):
+    """test_many_causal_tokens around the counts that fewer heads and a cache move the kernels' line to."""
+    test_many_causal_tokens(M, P, H, causal)

@@ -17,11 +17,14 @@
 namespace {
 
 constexpr int AT = 256;          // threads of k_attn_part
-// Causal tokens from which k_attn_rows runs: where its launch of the rotate + quantize, which the combine has fused, is paid
-// back, for both kinds of call so that they round the same outputs. MI355X, us on the chunks / on k_attn_rows, outputs only: 256
-// tokens 13.1 / 11.0, 400: 18.9 / 15.6, 968: 52 / 34.4. Quantized: 130 tokens 11.9 / 13.6, 256: 14.6 / 14.5, 400: 20.7 / 19.4, 968:
-// 54.3 / 39.2.
-constexpr int ATTN_ROWS_M = 256;
+// Whether k_attn_rows runs M causal tokens behind a cache of P: one rule for calls that want outputs and for calls that want them
+// quantized (a launch of its own there, which the chunks' combine has fused), so that both round the same outputs. It computes 8
+// query rows per token whatever H is, while the chunks' partials shrink with H; at 256 tokens a cache gives its waves uneven
+// blocks. MI355X, us on the chunks / on k_attn_rows. Outputs only, H = 8: 256 tokens 13.1 / 11.0, 400: 18.9 / 15.6, 968: 52 / 34.4.
+// Quantized, H = 8: 130 tokens 11.9 / 13.6, 256: 14.9 / 14.7, 256 behind 200 20.1 / 23.8, 288 behind 200 24.6 / 24.3, 968: 54.5 / 39.2;
+// H = 5: 288: 18.9 / 17.2; H = 4: 400: 17.1 / 18.5, 512: 23.0 / 19.7; H = 2: 800 behind 200 41.5 / 42.1, 968: 42.1 / 36.9. One head stays on
+// the chunks: 512 behind 200 24.2 / 29.9, 1200 behind 2000 172 / 182.
+bool attn_rows_fits(int M, int P, int H) { return M >= (H >= 5 ? (P ? 288 : 256) : H >= 3 ? 512 : 968) && H > 1; }
 
 __device__ __forceinline__ const u16* key_row(const u16* cache, const u16* fresh, int P, int j) {
     return j < P ? cache + (size_t)j * AD : fresh + (size_t)(j - P) * AD;
@@ -686,7 +689,7 @@ extern "C" int tcq_attend_q4(const void* q, const void* k_cache, const void* v_c
     hipStream_t st = (hipStream_t)stream;
     // many causal tokens: no partials; the BF16 rows (into the workspace when the caller wants only their quantized form), then
     // the rotate + quantize of the row kernels
-    if (M >= ATTN_ROWS_M && causal_offset >= 0 && (!o || (uintptr_t)o % 8 == 0)) {
+    if (attn_rows_fits(M, P, H) && causal_offset >= 0 && (!o || (uintptr_t)o % 8 == 0)) {
         u16* rows = o ? (u16*)o : (u16*)part;
         launch_k(k_attn_rows, dim3((M + 1) / 2), dim3(256), (size_t)4 * VTW, st, (const u16*)q, (const u16*)k_cache,
                  (const u16*)v_cache, P, (const u16*)k_new, (const u16*)v_new, M, H, causal_offset, rows);
