@@ -360,18 +360,22 @@ static void launch_gemm(int odt, hipStream_t st, const void* x, const void* w, c
 // costs, c2 a step of two rounds (the tiles up to 128 x 128 fit two workgroups on a CU, which share its LDS and matrix
 // cores), later rounds as pairs. In units of 1/16 us per 128-byte step, fitted to INT8 runs over M = 80 .. 968 and N = 1024
 // .. 32768 on MI355X (us, K = 2048): 64 x 64 8.0 (256 workgroups) / 10.1 (512), 128 x 64 9.9 / 15.4, 128 x 128 13.4 / 24.6,
-// 256 x 128 19.4 / 44, 256 x 256 33 / 73. The best tile was the chosen one or within 8 % of it at every size measured:
-// 968 x 2560: 13.3 on 128 x 128 against 15.0 and 15.4; 968 x 2048: 10.6 on 64 x 64 against 12.8 on 128 x 128; 768 x 1152 x
-// 4304: 13.5 on 64 x 64 against 25.2 on 128 x 128.
+// 256 x 128 19.4 / 44, 256 x 256 33 / 73. Of equal estimates the one whose rounds are fullest, and of those the larger tile, which
+// reads less: 300 x 32768 33.4 us on 256 x 256 against 39.5 on 128 x 128 and 49.5 on 128 x 64, all with full rounds; 700 x 12288 FP32 37.8,
+// 31.7 and 35.4 (144 workgroups of 256, 576 of 768, 1056 of 1280). Over 684 runs (19 weight shapes of K = 1024 .. 16384, M = 65 .. 968, int32
+// and FP32 out) the chosen tile was 2.4 % above the best of the five on average and more than 8 % above it in 74, most where a
+// last round is partly filled: 400 x 2560 x 2048 takes 128 x 64 at 9.5 us where 64 x 64 needs 8.3, 900 x 4608 x 1536 256 x 128 at 17.3 where
+// 128 x 128 needs 14.4. A short K pays the longer ramp of these tiles: with int32 out 700 .. 968 tokens x 2560 or 3072 x 1024 take 9.2 us,
+// 8.1 .. 8.8 with 64-byte steps and 32 x 32 blocks; from K = 1536 on that form is slower nearly everywhere, by up to a third.
 struct TileCost { int tn, tm, c1, c2; };
 constexpr TileCost TILES[5] = {{64, 64, 4, 7}, {128, 64, 6, 12}, {128, 128, 9, 20}, {256, 128, 16, 38}, {256, 256, 30, 68}};
 static int choose_tile(int M, int N, int parts, int tiles, long* cost = nullptr) {
     int best = 0;
-    long bc = 0;
+    long bc = 0, bw = 0, br = 1;
     for (int i = 0; i < tiles; ++i) {
         const long w = (long)((N + TILES[i].tn - 1) / TILES[i].tn) * ((M + TILES[i].tm - 1) / TILES[i].tm) * parts, r = (w + 255) / 256;
         const long c = r == 1 ? 2 * TILES[i].c1 : r * TILES[i].c2;
-        if (i == 0 || c < bc) { best = i; bc = c; }
+        if (i == 0 || c < bc || (c == bc && w * br >= bw * r)) { best = i; bc = c; bw = w; br = r; }
     }
     if (cost) *cost = bc;                               // a step's time in units of 1/32 us
     return best;
