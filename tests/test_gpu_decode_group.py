@@ -72,3 +72,25 @@ def test_float_group_across_the_token_bound(M, part):
         ref = O.bf16_to_f32(O.w2_linear(x.float().cpu().numpy(), ol, small=part == 'expert'))
         got = outs[0][i].float().cpu().numpy()
         assert np.linalg.norm(got - ref) <= 2e-3 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize('part', ['llm', 'expert'])
+@pytest.mark.parametrize('widths,K,M', [((2048, 1024), 1152, 226), ((2048, 1024), 1152, 227), ((512,), 16384, 190), ((512,), 16384, 191), ((2048,), 16384, 65)])
+def test_float_group_across_the_dense_line(widths, K, M, part):
+    """As test_float_group_across_the_token_bound on both sides of the line between the fused products and dense weights (226 / 227
+    tokens of 3072 x 1152, 190 / 191 of 512 x 16384) and where 65 tokens are past it."""
+    from yanlongvla_amd import modules
+    layers = [layer(m, K, 70 + i) for i, m in enumerate(widths)]
+    for L in layers[1:]:
+        L.su = layers[0].su
+    x = torch.randn(M, K, device=DEV, generator=torch.Generator(device=DEV).manual_seed(M)).bfloat16()
+    groups = [modules.Group(layers, part, mode, a8=False) for mode in ('fly', 'resident')]
+    assert all(G.dense_float(M) == (M in (227, 191, 65)) for G in groups)
+    outs = [G.run(x) for G in groups]
+    for i, L in enumerate(layers):
+        assert torch.equal(outs[0][i], outs[1][i])
+        ol = O.Layer(L.name, dict(bits=L.bits.cpu().numpy(), tlut=L.tlut.cpu().numpy(), row_scale=L.row_scale.cpu().numpy(),
+                                  su=L.su.cpu().numpy(), sv=L.sv.cpu().numpy()))
+        ref = O.bf16_to_f32(O.w2_linear(x.float().cpu().numpy(), ol, small=part == 'expert'))
+        got = outs[0][i].float().cpu().numpy()
+        assert np.linalg.norm(got - ref) <= 2e-3 * np.linalg.norm(ref)

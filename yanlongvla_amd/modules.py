@@ -393,17 +393,27 @@ class Group:
         STATS['group_runs'] += 1
         return outs
 
+    def dense_float(self, M):
+        """Whether M tokens of the float path run on dense weights. The fused products decode every weight again per 64 tokens
+        (backbone gate | up at 968 tokens: 1252 us against 30 for the weights and 149 for the GEMM), but a small layer's decode
+        hides in a launch that is waiting anyway, and dense weights cost a launch or two: the line lies at 8e8 multiply-adds in
+        more workgroups than CUs, or at 1.6e9. One group's whole run on MI355X, us fused / dense: 8192 x 1024 80 tokens 26 / 27,
+        128: 30 / 27; 1024 x 2048 256: 20 / 23, 400: 30 / 26; 1024 x 4096 256: 28 / 29, 400: 47 / 31; 3456 x 1152 128: 25 / 29, 256:
+        39 / 32; 2560 x 2048 128: 29 / 31, 160: 34 / 29; 2048 x 16384 65: 71 / 53. (The GEMM takes weights below 2 GiB.)"""
+        work = M * self.Ntot * self.K
+        full = self.Ntot // 16 * ((M + 63) // 64) > 256                                 # the fused products' workgroups
+        return M > SMALL_M and self.Ntot * self.K < 1 << 30 and (work >= 16e8 or (full and work >= 8e8))
+
     def run_float(self, x2, shape):
         """W2: BF16 rotated activations (kernels.rht = the reference's pre_h), the INT8 table values as BF16 weights, FP32
         sums. Few tokens on the fused products (kernels.gemmf_segments: the packed words decoded on the fly, or the resident
-        INT8 weights); many tokens on the BF16 MFMA GEMM over dense BF16 weights made for the call, as the reference's
-        prefill does (modules.py:117-130): the fused products decode every weight again per 64 tokens (backbone gate | up at
-        968 tokens: 1252 us against 30 for the weights and 125 for the GEMM). Expert: z = acc * rs in FP32; prefill: the
+        INT8 weights); many tokens on the BF16 MFMA GEMM over dense BF16 weights made for the call (2 Ntot K bytes), as the
+        reference's prefill does (modules.py:117-130): dense_float. Expert: z = acc * rs in FP32; prefill: the
         product rounded to BF16, scaled by rs in the epilogue (modules.py:117-144)."""
         M, dev = x2.shape[0], x2.device
         h = kernels.rht(x2, self.su, torch.empty(M, self.K, dtype=torch.bfloat16, device=dev))
         acc = torch.empty(M, self.Ntot, dtype=torch.float32 if self.small else torch.bfloat16, device=dev)
-        if M > SMALL_M and self.Ntot * self.K < 1 << 30:             # (the GEMM takes weights below 2 GiB)
+        if self.dense_float(M):
             w = torch.empty(self.Ntot, self.K, dtype=torch.bfloat16, device=dev)
             if self.W is not None:
                 kernels.i8_to_bf16(self.W, w)
