@@ -62,7 +62,7 @@ __device__ __forceinline__ int4v dot_to_mfma_layout(int v, int lane) {
 
 }  // namespace
 
-// bias: FP32 bias of each segment's rows or NULL (BF16 outputs)
+// bias: FP32 bias of each segment's rows or NULL (the BIAS forms of the kernels)
 struct SegPack {
     tcq_gemm_seg s[TCQ_MAX_SEGS];
     const float* bias[TCQ_MAX_SEGS];
@@ -145,7 +145,9 @@ enum { QL_ROWS = 0, QL_BLOCKS = 1, QL_WORDS = 2 };
 // grid (tile-row groups of the largest segment, segments), NW = blockDim.x / 64 waves; a workgroup takes TR consecutive tile
 // rows (the activation fragments of its chunks, the bulk of the loads, then serve TR rows). MODE 0: decode from tcq_repack
 // words (RB: from the reference word layout, 64 bytes per tile, tiles row-major); MODE 1: resident INT8 weights. ODT: output
-// dtype (F32 scaled; BF16 scaled, plus the segment's bias, with rows ldz apart or, for ldz 0, contiguous; I32 accumulators). QL: activation layout (ldq only for QL_WORDS).
+// dtype (F32 scaled; BF16 scaled; I32 accumulators). QL: activation layout (ldq only for QL_WORDS).
+// BIAS (BF16): plus the segment's bias where it has one, output rows contiguous. A form of its own, as its registers cost the plain one
+// its sixth wave per SIMD: resident 1 x 2 x 16384 x 2048 13.3 us, 14.0 with them.
 // KS > 1 (I32 only): K parts, blockIdx.z = part p takes chunks [p * ceil(nch / KS), ...) and writes at out + p * M * ldz.
 // DOT (M == 1): the product on v_dot4c_i32_i8 (dot_product) instead of the MFMA; the epilogues are shared.
 // PL > 0 (M == 1, K = 2^PL): the activations come from the prologue run by every workgroup (run_prologue, ProShape)
@@ -154,9 +156,10 @@ enum { QL_ROWS = 0, QL_BLOCKS = 1, QL_WORDS = 2 };
 // while waves 8 .. NW - 1 fill the table and decode the weight fragments of their chunks (chunk c0 + wave - 8) into
 // registers, meeting the prologue's barriers; after the row is in LDS they multiply, and their partial sums add in chunk
 // order as without OVS (the same sums and outputs).
-template <int MODE, int NB, int ODT, int TR, int QL, bool RB = false, int KS = 1, bool DOT = false, int PL = 0, bool OVS = false>
+template <int MODE, int NB, int ODT, int TR, int QL, bool RB = false, int KS = 1, bool DOT = false, int PL = 0, bool OVS = false, bool BIAS = false>
 __global__ __launch_bounds__(TR == 1 ? 1024 : 512) void k_gemm_small(const typename PackOf<PL>::type P, const i8* q, const float* s,
                                                                     int M, int K, int ldz, int ldq) {
+    static_assert(!BIAS || (ODT == TCQ_BF16 && !PL), "bias");
     static_assert(!OVS || ((PL == PRO_LAYER || PL == PRO_ATTN) && MODE == 0 && TR == 1 && !RB), "overlapped prologue");
     static_assert(KS == 1 || ODT == TCQ_I32, "K parts are int32 sums");
     static_assert(!DOT || (NB == 1 && QL != QL_WORDS), "dot products: one token, q rows or token blocks");
@@ -258,10 +261,9 @@ __global__ __launch_bounds__(TR == 1 ? 1024 : 512) void k_gemm_small(const typen
     if (!PL && c0 + wave < nch) load(c0 + wave);
     if (OVS && pw >= 0 && c0 + pw < nch) load(c0 + pw);
     // epilogue scales, loaded with the operands (wave 0 stores; OVS: wave 8)
-    constexpr bool BIAS = ODT == TCQ_BF16 && !PL;
     const float* bias = nullptr;
     if constexpr (BIAS) bias = P.bias[blockIdx.y];
-    const int ld = BIAS && !ldz ? S.m : ldz;
+    const int ld = BIAS ? S.m : ldz;
     float4_t rsv[TR], bv[BIAS ? TR : 1];
     float sv[NB];
 #pragma unroll
@@ -491,13 +493,13 @@ constexpr int GV_NW = 16;              // waves per workgroup (one 64 KiB table 
 // stages of the block Walsh of the whole segment (h = 1 .. 64, which stay inside such a block) run here, in the reference's
 // stage order, and the block is stored transposed: zt[(t * 128 + o) * (m / 128) + blk] for row 128 blk + o of token t.
 // DOT (M == 1): the product on v_dot4c_i32_i8 (dot_product) instead of the MFMA; the epilogues are shared.
-// PL > 0: activations from the prologue, as k_gemm_small.
+// BIAS, PL > 0 (activations from the prologue): as k_gemm_small.
 // OV (the layer prologue of a 2048-wide row): the prologue runs on waves 0 .. 3 from entry (panp_waves,
 // waves_rotate_quantize, at a raised issue priority) while the other waves fill the table and then decode the weight
 // fragments of their chunks into registers, one chunk after each of the prologue's WAVES_SYNCS barriers (the first of
 // which is also the table's); one more barrier hands the row to every wave for its products. The same row, sums and
 // outputs as without OV.
-template <int ODT, bool QB, int WPR, int NW, int KS = 1, bool LO = false, bool DOT = false, int PL = 0, bool OV = false>
+template <int ODT, bool QB, int WPR, int NW, int KS = 1, bool LO = false, bool DOT = false, int PL = 0, bool OV = false, bool BIAS = false>
 __global__ __launch_bounds__(64 * NW) void k_gemv_tcq(const typename PackOf<PL>::type P, const i8* q, const float* s, int M, int K,
                                                       int ldz) {
     static_assert(KS == 1 || ODT == TCQ_I32, "K parts are int32 sums");
@@ -556,7 +558,6 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_tcq(const typename PackOf<PL>:
     };
     int4v Bf[2][4];                                                        // activation fragments, two chunks in turn
     if constexpr (!PL) loadB(c0 + part, Bf[0]);
-    constexpr bool BIAS = ODT == TCQ_BF16 && !PL;
     const float* bias = nullptr;
     if constexpr (BIAS) bias = P.bias[blockIdx.y];
     float4_t rsv = float4_t{0.f, 0.f, 0.f, 0.f}, bv = rsv;
@@ -674,7 +675,7 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_tcq(const typename PackOf<PL>:
     if (I0 + slot >= tiles_m) return;
     const int t = lr;
     if (t >= M) return;
-    const size_t o = (size_t)t * (BIAS && !ldz ? S.m : ldz) + 16 * I + 4 * lg;
+    const size_t o = (size_t)t * (BIAS ? S.m : ldz) + 16 * I + 4 * lg;
     if (ODT == TCQ_I32) {
         *gptr((int4v*)((int*)S.out + (KS > 1 ? (size_t)blockIdx.z * M * ldz : 0) + o)) = acc;
     } else {
@@ -771,12 +772,20 @@ __global__ __launch_bounds__(1024) void k_gemv_w8t(const SegPack P, const i8* q,
 }
 
 // =========================================================================================================== C ABI
+// odt BF16 with ldo 0: the bias form
 template <int MODE, int NB, int TR, int QL, bool RB, bool DOT = false>
 static void launch_small_nb(dim3 grid, dim3 block, hipStream_t st, const SegPack& P, const i8* q, const float* s, int M, int K,
                             int ldo, int ldq, int odt) {
     switch (odt) {
         case TCQ_F32: launch_k(k_gemm_small<MODE, NB, TCQ_F32, TR, QL, RB, 1, DOT>, grid, block, 0, st, P, q, s, M, K, ldo, ldq); break;
-        case TCQ_BF16: launch_k(k_gemm_small<MODE, NB, TCQ_BF16, TR, QL, RB, 1, DOT>, grid, block, 0, st, P, q, s, M, K, ldo, ldq); break;
+        case TCQ_BF16:
+            if constexpr (QL != QL_WORDS)
+                if (!ldo) {
+                    launch_k(k_gemm_small<MODE, NB, TCQ_BF16, TR, QL, RB, 1, DOT, 0, false, true>, grid, block, 0, st, P, q, s, M, K, ldo, ldq);
+                    break;
+                }
+            launch_k(k_gemm_small<MODE, NB, TCQ_BF16, TR, QL, RB, 1, DOT>, grid, block, 0, st, P, q, s, M, K, ldo, ldq);
+            break;
         default: launch_k(k_gemm_small<MODE, NB, TCQ_I32, TR, QL, RB, 1, DOT>, grid, block, 0, st, P, q, s, M, K, ldo, ldq); break;
     }
 }
@@ -796,17 +805,17 @@ static void launch_small_tr(dim3 grid, dim3 block, hipStream_t st, const SegPack
     else launch_small_qb<MODE, TR, QL_ROWS>(grid, block, st, P, q, s, M, K, ldo, 0, odt);
 }
 
-template <int ODT, bool QB, bool DOT>
+template <int ODT, bool QB, bool DOT, bool BIAS>
 static void launch_gv(int wpr, int rows, int nseg, hipStream_t st, const SegPack& P, const i8* q, const float* s, int M, int K,
                       int ldo) {
     const int rpw = GV_NW / wpr;
     const dim3 grid((rows + rpw - 1) / rpw, nseg), block(64 * GV_NW);
     switch (wpr) {
-        case 1: launch_k(k_gemv_tcq<ODT, QB, 1, GV_NW, 1, false, DOT>, grid, block, 0, st, P, q, s, M, K, ldo); break;
-        case 2: launch_k(k_gemv_tcq<ODT, QB, 2, GV_NW, 1, false, DOT>, grid, block, 0, st, P, q, s, M, K, ldo); break;
-        case 4: launch_k(k_gemv_tcq<ODT, QB, 4, GV_NW, 1, false, DOT>, grid, block, 0, st, P, q, s, M, K, ldo); break;
-        case 8: launch_k(k_gemv_tcq<ODT, QB, 8, GV_NW, 1, false, DOT>, grid, block, 0, st, P, q, s, M, K, ldo); break;
-        default: launch_k(k_gemv_tcq<ODT, QB, 16, GV_NW, 1, false, DOT>, grid, block, 0, st, P, q, s, M, K, ldo); break;
+        case 1: launch_k(k_gemv_tcq<ODT, QB, 1, GV_NW, 1, false, DOT, 0, false, BIAS>, grid, block, 0, st, P, q, s, M, K, ldo); break;
+        case 2: launch_k(k_gemv_tcq<ODT, QB, 2, GV_NW, 1, false, DOT, 0, false, BIAS>, grid, block, 0, st, P, q, s, M, K, ldo); break;
+        case 4: launch_k(k_gemv_tcq<ODT, QB, 4, GV_NW, 1, false, DOT, 0, false, BIAS>, grid, block, 0, st, P, q, s, M, K, ldo); break;
+        case 8: launch_k(k_gemv_tcq<ODT, QB, 8, GV_NW, 1, false, DOT, 0, false, BIAS>, grid, block, 0, st, P, q, s, M, K, ldo); break;
+        default: launch_k(k_gemv_tcq<ODT, QB, 16, GV_NW, 1, false, DOT, 0, false, BIAS>, grid, block, 0, st, P, q, s, M, K, ldo); break;
     }
 }
 
@@ -854,9 +863,12 @@ template <bool QB, bool DOT>
 static void launch_gv_odt(int odt, int wpr, int rows, int nseg, hipStream_t st, const SegPack& P, const i8* q, const float* s,
                           int M, int K, int ldo) {
     switch (odt) {
-        case TCQ_F32: launch_gv<TCQ_F32, QB, DOT>(wpr, rows, nseg, st, P, q, s, M, K, ldo); break;
-        case TCQ_BF16: launch_gv<TCQ_BF16, QB, DOT>(wpr, rows, nseg, st, P, q, s, M, K, ldo); break;
-        default: launch_gv<TCQ_I32, QB, DOT>(wpr, rows, nseg, st, P, q, s, M, K, ldo); break;
+        case TCQ_F32: launch_gv<TCQ_F32, QB, DOT, false>(wpr, rows, nseg, st, P, q, s, M, K, ldo); break;
+        case TCQ_BF16:
+            if (!ldo) launch_gv<TCQ_BF16, QB, DOT, true>(wpr, rows, nseg, st, P, q, s, M, K, ldo);
+            else launch_gv<TCQ_BF16, QB, DOT, false>(wpr, rows, nseg, st, P, q, s, M, K, ldo);
+            break;
+        default: launch_gv<TCQ_I32, QB, DOT, false>(wpr, rows, nseg, st, P, q, s, M, K, ldo); break;
     }
 }
 
