@@ -162,11 +162,12 @@ struct NoMid {
     __device__ void operator()() const {}
 };
 // BIAS = false: A.bias is ignored (callers that have none save its registers).
-// 8-element pieces (the eight-values-per-thread engine): loads of 8 consecutive values as FP32.
+// 8-element pieces (the eight-values-per-thread engine): loads of 8 consecutive values as FP32. Plain conversions, which the compiler
+// spreads better than i8_f32's in these short rows (residual without norm, 50 x 2048: 3.27 against 3.39 us).
 __device__ __forceinline__ void ld8_i8v(const i8* p, float (&v)[8]) {
     const u64 w = *gptr((const u64*)p);
 #pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = i8_f32((u32)(w >> (32 * (k >> 2))), k & 3);
+    for (int k = 0; k < 8; ++k) v[k] = (float)(i8)(w >> (8 * k));
 }
 __device__ __forceinline__ void ld8_bf16v(const u16* p, float (&v)[8]) {
     const uint4_t a = gptr((const uint4_t*)p)[0];
@@ -394,6 +395,9 @@ template <int ADT, int NWP, int L = 11, class F, class SY>
 __device__ __forceinline__ void panp_waves(const PanpArgs& A, int tok, bool store, float (&v)[(1 << L) / 64 / NWP], WavesLds& Q,
                                            F&& mid, SY&& sync) {
     constexpr int N = 1 << L, E = N / 64 / NWP, LE = E == 8 ? 3 : 2, LPC = 16 / E;
+    // i8_f32 in launches of their own (50 x 1024: 3.86 -> 3.81 us); as a product's prologue its fixed instructions cost the product
+    // registers, five waves per SIMD instead of six (resident 2 x 16384 x 2048 behind it 19.7 us, 17.8 with plain conversions)
+    constexpr bool ALONE = std::is_same_v<F, NoMid>;
     static_assert((L == 10 || L == 11) && (E == 4 || E == 8), "rows of 1024 or 2048, 4 or 8 values per thread");
     const int t = threadIdx.x, i0 = E * t, lane = t & 63, w = t >> 6;
     const size_t row = (size_t)tok * N, base = (size_t)tok * A.lda + A.col0 + i0;
@@ -404,7 +408,7 @@ __device__ __forceinline__ void panp_waves(const PanpArgs& A, int tok, bool stor
         } else {
             const u32 x = *gptr((const u32*)p);
 #pragma unroll
-            for (int k = 0; k < 4; ++k) o[k] = i8_f32(x, k);
+            for (int k = 0; k < 4; ++k) o[k] = ALONE ? i8_f32(x, k) : (float)(i8)(x >> (8 * k));
         }
     };
     auto ld_bf16 = [&](const u16* p, float (&o)[E]) {
