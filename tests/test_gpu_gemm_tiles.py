@@ -131,3 +131,26 @@ def test_tiles_of_equal_estimates(M, N, K):
     """Sizes whose estimate several tiles share: full rounds (the larger tile) and partly filled ones (the fullest)."""
     test_int8_tiles_bitexact(M, N, K)
     test_bf16_tiles_against_fp64(M, N, K)
+
+
+@pytest.mark.parametrize('M,N,K', [(65, 68, 1024), (130, 132, 2048), (300, 2052, 2048), (129, 8200, 528)])
+def test_bf16_scaled_infinities(M, N, K):
+    """Scaled FP32 and BF16 outputs of every tile width around infinite sums: (z sa) sw of the unscaled FP32 output z, its BF16
+    rounding, infinities where z is checked to have them."""
+    from yanlongvla_amd import kernels as Kn
+    g = torch.Generator(device=DEV).manual_seed(N)
+    a, w = torch.randn(M, K, generator=g, device=DEV).bfloat16(), _ints(N, K, seed=9).abs().clamp(min=1).bfloat16()
+    a[5, 3], a[M - 1, K - 1], a[40, 64] = float('inf'), float('-inf'), float('nan')
+    w[N - 2, 100] = float('inf')                                               # both signs of activations: infinities of both
+    sa, sw = torch.rand(M, generator=g, device=DEV) + 0.1, torch.rand(N, generator=g, device=DEV) + 0.1
+    z = Kn.gemm_bf16(a, w, torch.empty(M, N, device=DEV))
+    col = torch.sign(a[:, 100].float()) * float('inf')
+    rows = [m for m in range(M) if m not in (5, 40, M - 1)]
+    assert torch.equal(z[rows, N - 2], col[rows]) and bool(z[40].isnan().all())
+    rest = [n for n in range(N) if n != N - 2]
+    assert bool((z[5, rest] == float('inf')).all()) and bool((z[M - 1, rest] == float('-inf')).all())
+    want = (z * sa[:, None]) * sw
+    got = Kn.gemm_bf16(a, w, torch.empty(M, N, device=DEV), sa=sa, sw=sw)
+    assert torch.equal(got.nan_to_num(nan=7.0, posinf=8.0, neginf=9.0), want.nan_to_num(nan=7.0, posinf=8.0, neginf=9.0))
+    b = Kn.gemm_bf16(a, w, torch.empty(M, N, dtype=torch.bfloat16, device=DEV), sa=sa, sw=sw)
+    assert torch.equal(b.nan_to_num(nan=7.0, posinf=8.0, neginf=9.0), want.bfloat16().nan_to_num(nan=7.0, posinf=8.0, neginf=9.0))

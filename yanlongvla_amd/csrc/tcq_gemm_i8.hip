@@ -254,8 +254,9 @@ __global__ __launch_bounds__(64 * WN * WM) void k_gemm_i8(const void* x_, const 
         for (; kt < nk; ++kt) step(kt, Tail{});
     } else {
         // FP32 sums in two levels, `flush` steps (two MFMAs each) in a row, then the sums of those, each with what its addition
-        // rounded away (sum - exact, by two subtractions) carried into the next chain: the error of the second level vanishes,
-        // and that of a chain grows with its length only. Relative error against 64 bits, K = 1024 / 2048 / 4096 / 16384:
+        // rounded away (exact - sum, by two subtractions: exact while the running sum is the larger of the two, close to it
+        // otherwise) carried into the next chain; what the last one rounded away is less than half an ulp. Most of the second level's
+        // error goes, and that of a chain grows with its length only. Relative error against 64 bits, K = 1024 / 2048 / 4096 / 16384:
         // 4.9e-8, 5.6e-8, 6.4e-8, 8.9e-8; without the carry 6.3e-8, 7.3e-8, 8.7e-8, 1.24e-7; the few-token product's partial sums
         // (three levels) 5.7e-8, 6.9e-8, 7.8e-8, 1.18e-7.
         acc_t sum[NB][MB];
@@ -271,18 +272,35 @@ __global__ __launch_bounds__(64 * WN * WM) void k_gemm_i8(const void* x_, const 
             for (int i = 0; i < NB; ++i)
 #pragma unroll
                 for (int j = 0; j < MB; ++j) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float a = sum[i][j][e], b = acc[i][j][e], t = a + b, r = b - (t - a);
-                        acc[i][j][e] = fabsf(t) < __builtin_inff() ? r : 0.f;    // an infinite sum stays one (inf - inf is a NaN)
-                        sum[i][j][e] = t;
-                    }
+                    const acc_t t = sum[i][j] + acc[i][j];
+                    acc[i][j] = acc[i][j] - (t - sum[i][j]);
+                    sum[i][j] = t;
                 }
         }
 #pragma unroll
         for (int i = 0; i < NB; ++i)
 #pragma unroll
             for (int j = 0; j < MB; ++j) acc[i][j] = sum[i][j];
+    }
+    // BF16: an infinite sum's carry is inf - inf, so a NaN here may stand for an infinity. Such outputs are summed again in one
+    // plain chain at the end (a test of every carry, so that none becomes a NaN, cost 2 to 7 %: 968 x 32768 x 2048 147.2 us, 152.7 with it
+    // and 148.9 so, 800 x 8192 x 1024 23.5, 25.1, 23.6, 65 x 1152 x 1152 9.6, 9.9, 9.6)
+    u64 nans = 0;                                   // bit 4 (i MB + j) + e
+    if constexpr (ESZ == 2) {
+        static_assert(4 * NB * MB <= 64, "a bit per value");
+        bool any = false;
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int j = 0; j < MB; ++j)
+                any |= __builtin_isunordered(acc[i][j][0], acc[i][j][1]) | __builtin_isunordered(acc[i][j][2], acc[i][j][3]);
+        if (__builtin_amdgcn_ballot_w64(any))
+#pragma unroll
+            for (int i = 0; i < NB; ++i)
+#pragma unroll
+                for (int j = 0; j < MB; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) nans |= (u64)__builtin_isnan(acc[i][j][e]) << (4 * (i * MB + j) + e);
     }
     wait_cnt<0, 0>();                               // no load into the LDS outlives the workgroup
     // D: register e of lane (g, c) = weight row 4 g + e of the A block, token c of the B block
@@ -339,6 +357,27 @@ __global__ __launch_bounds__(64 * WN * WM) void k_gemm_i8(const void* x_, const 
                     *gptr((float4v*)((float*)out + ((size_t)z * M + m) * ldo + n)) = v;
                 }
             }
+        }
+    }
+    if constexpr (ESZ == 2) {
+        while (nans) {
+            const int b = __builtin_ctzll(nans), e = b & 3, j = (b >> 2) % MB, i = (b >> 2) / MB;
+            nans &= nans - 1;
+            const int m = m0 + (wm * MB + j) * 16 + lr, n = n0 + wn * NB * 16 + (PAIR ? 32 * (i >> 1) + 8 * lg + 4 * (i & 1) : 16 * i + 4 * lg) + e;
+            if (m >= M || n >= N) continue;
+            const u16 *xr = (const u16*)x_ + (size_t)m * K_, *wr = (const u16*)w_ + (size_t)n * K_;
+            float v = 0.f;
+            for (int k = 64 * kb; k < kend / 2 && !__builtin_isnan(v); k += 8) {
+                const uint4_t a = *gptr((const uint4_t*)(xr + k)), c = *gptr((const uint4_t*)(wr + k));
+#pragma unroll
+                for (int h = 0; h < 8; ++h)
+                    v = __builtin_fmaf(bf16_to_f32((u16)(a[h >> 1] >> (16 * (h & 1)))), bf16_to_f32((u16)(c[h >> 1] >> (16 * (h & 1)))), v);
+            }
+            if (sa) v = v * gptr(sa)[m];
+            if (sw) v = v * gptr(sw)[n];
+            const size_t o = ((size_t)z * M + m) * ldo + n;
+            if (PAIR) gptr((u16*)out)[o] = f32_to_bf16(v);
+            else gptr((float*)out)[o] = v;
         }
     }
 }
