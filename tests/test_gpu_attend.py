@@ -148,3 +148,32 @@ def test_many_causal_tokens_exponentials():
 def test_many_causal_tokens_by_heads_and_cache(M, P, H, causal):
     """test_many_causal_tokens around the counts that fewer heads and a cache move the kernels' line to."""
     test_many_causal_tokens(M, P, H, causal)
+
+
+@pytest.mark.parametrize('P,causal', [(0, 0), (40, 40)])
+@pytest.mark.parametrize('M', [255, 290])
+def test_infinite_and_nan_keys_and_values(M, P, causal):
+    """On either kernel (255 tokens on the chunks, 290 on k_attn_rows): a NaN key or a key of infinite score makes every row that
+    sees it NaN, an infinite value gives that infinity in its column and nothing else; rows of token pairs before it keep their
+    bits (a pair shares its products, so the token just before may not)."""
+    from yanlongvla_amd import kernels as K
+    q, kc, vc, kn, vn = inputs(M, P, 8, 3 * M + P)
+
+    def run(kn, vn):
+        o = torch.empty(M, 2048, dtype=torch.bfloat16, device=DEV)
+        K.attend(q, kc, vc, kn, vn, 8, causal, o=o)
+        return o.view(M, 8, 256)
+    clean = run(kn, vn)
+    j = 100                                                                    # even: the first of its pair
+    for bad in (float('nan'), float('inf')):
+        k2 = kn.clone()
+        k2[j] = bad
+        o = run(k2, vn)
+        assert torch.equal(o[:j], clean[:j]) and bool(o[j:].isnan().all())     # (inf x both signs of q: NaN too)
+    for bad in (float('inf'), float('-inf')):
+        v2 = vn.clone()
+        v2[j, 7] = bad
+        o = run(kn, v2)
+        assert torch.equal(o[:j], clean[:j]) and bool((o[j:, :, 7] == bad).all())
+        o[j:, :, 7] = clean[j:, :, 7]
+        assert torch.equal(o, clean)
