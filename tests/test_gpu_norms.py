@@ -214,3 +214,49 @@ def test_epilogues_of_more_rows_match_few(M, N):
     parts = [run(a, min(a + 40, M)) for a in range(0, M, 40)]
     for i, t in enumerate(whole):
         assert torch.equal(t, torch.cat([p[i] for p in parts]))
+
+
+@pytest.mark.parametrize('parts', [2, 4])
+@pytest.mark.parametrize('M,N', [(65, 2048), (419, 2048), (420, 2048), (839, 1024), (840, 1024), (130, 4096)])
+def test_k_parts_of_more_rows(M, N, parts):
+    """post_add_norm_pre without a bias over the int32 K parts that a product of more than 64 tokens hands it, on both sides of the
+    row counts where its engine changes: the outputs of their sum in one accumulator, and of calls of 40 rows."""
+    from yanlongvla_amd import kernels as Kn
+    g = torch.Generator(device=DEV).manual_seed(M + parts)
+    r = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    acc, x, w = (r(parts, M, N) * 1e4).int(), r(M, N).bfloat16(), r(N).bfloat16()
+    s, rs = (torch.rand(n, generator=g, device=DEV) * 1e-2 + 1e-4 for n in (M, N))
+    sv, su = (torch.where(r(N) > 0, 1, -1).to(torch.int8) for _ in range(2))
+
+    def run(acc, a, b):
+        x_, m = x[a:b], b - a
+        xo, q, sc = torch.empty_like(x_), torch.empty(m, N, dtype=torch.int8, device=DEV), torch.empty(m, device=DEV)
+        Kn.post_add_norm_pre(acc[..., a:b, :].contiguous(), s[a:b], rs, sv, None, x_, xo, w, 1e-6, su, q=q, scale=sc)
+        return xo, q, sc
+    whole, one = run(acc, 0, M), run(acc.sum(0).int(), 0, M)
+    pieces = [run(acc, a, min(a + 40, M)) for a in range(0, M, 40)]
+    for i, t in enumerate(whole):
+        assert torch.equal(t, one[i]) and torch.equal(t, torch.cat([p[i] for p in pieces]))
+
+
+@pytest.mark.parametrize('runtime', ['fly', 'resident'])
+@pytest.mark.parametrize('M', [65, 200, 450])
+def test_decoder_layers_with_and_without_k_parts(M, runtime):
+    """A backbone prefill whose o and down products run in K parts (more than one at these counts) gives the outputs of one part,
+    bit for bit, chained prologues included."""
+    from yanlongvla_amd import gemma, modules
+    model = gemma.make_policy(gemma.BackbonePolicy, DEV, seed=5, layers=2, vocab=512)
+    modules.install(model, runtime=runtime, layers=gemma.synthetic_layers(model, 16, DEV))
+    down = [G for G in model._tcq_groups if G.K == 16384]
+    assert len(down) == 2 and all(G.epilogue_parts(M) > 1 for G in down)
+    x = torch.randn(M, 2048, generator=torch.Generator(device=DEV).manual_seed(M), device=DEV).bfloat16()
+    outs = {}
+    for parts in (False, True):
+        modules.FUSE['k_parts'] = parts
+        try:
+            h, ks, vs = model.prefill(x)
+            outs[parts] = [h, *ks, *vs]
+        finally:
+            modules.FUSE['k_parts'] = True
+    for a, b in zip(outs[False], outs[True]):
+        assert torch.equal(a, b)

@@ -192,3 +192,33 @@ def test_k_parts_rule():
         assert parts(2048, 16384, 1) == 1
     finally:
         modules.FUSE['k_parts'] = old
+
+
+def test_many_token_k_parts_rule():
+    """The parts of a product of more than 64 tokens: one below, for a short K, for widths the epilogue takes no parts of, for
+    unaligned side vectors and when off; two and four where few tiles meet a long K (the sizes the rule's comments time)."""
+    from yanlongvla_amd import kernels
+    best = kernels.gemm_i8_best_parts
+    assert [best(m, 2048, 16384) for m in (1, 64)] == [1, 1] and best(200, 2048, 1024) == 1
+    assert [best(m, 2048, 16384) for m in (200, 800, 968)] == [4, 2, 2]
+    assert [best(*s) for s in ((400, 1024, 4096), (968, 1024, 4096), (968, 2048, 2048), (968, 32768, 2048))] == [2, 1, 1, 1]
+    bf16 = kernels._lib.lib().tcq_gemm_bf16_best_parts
+    assert [bf16(*s) for s in ((64, 2048, 16384), (200, 2048, 512), (256, 2048, 16384), (968, 2048, 16384))] == [1, 1, 4, 4]
+    assert [bf16(*s) for s in ((400, 2048, 2048), (968, 32768, 2048))] == [1, 1]
+
+    class G:
+        k_parts = modules.Group.k_parts
+
+    def parts(m, *vectors, width=2048):
+        g = G()
+        g.Ntot, g.K, g.rs, g.sv, g.bias = width, 16384, torch.ones(width), torch.ones(width, dtype=torch.int8), None
+        return modules.Group.epilogue_parts(g, m, *vectors)
+    assert parts(1) == parts(modules.SMALL_M) == 2 and parts(200) == 4           # up to 64 tokens: those of k_parts
+    assert parts(200, None, torch.ones(2048)) == 4 and parts(200, torch.ones(2052)[1:2049]) == 1
+    assert parts(200, width=1536) == 1 and parts(200, width=512) == 1
+    old = modules.FUSE['k_parts']
+    modules.FUSE['k_parts'] = False
+    try:
+        assert parts(200) == 1
+    finally:
+        modules.FUSE['k_parts'] = old
