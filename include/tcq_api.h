@@ -471,8 +471,8 @@ int tcq_gemm_i8_best_parts(int M, int N, int K);
  * the INT8 table values as BF16 from tcq_decode_f16 with the BF16 table); out = (acc * sa[m]) * sw[n] as FP32 or BF16
  * (sa / sw may be NULL: factor 1). K % 16 == 0, N % 4 == 0; a, w, out 16-byte aligned. Replaces the prefill product of the
  * reference's Group.run_float, `h @ W.t()` on BF16 weights decoded by kernels.decode_bf16 (deploy/tcq_kernels/modules.py:
- * 120-126); the module layer decodes such weights for calls of more than 64 tokens and runs tcq_gemmf_* for fewer. FP32 sums in
- * two levels whose second carries what its additions round away. */
+ * 120-126); the module layer decodes such weights for calls of more than 64 tokens with enough work and runs tcq_gemmf_* for the
+ * others. FP32 sums in two levels; the second carries what its additions round away. */
 int tcq_gemm_bf16(const void* a, const void* w, const float* sa, const float* sw, void* out, int out_dtype, int ldo, int M, int N,
                   int K, tcq_stream_t stream);
 

@@ -494,7 +494,8 @@ __global__ __launch_bounds__(128) void k_attn_combine_reg(const float* part, int
 // layout (lane (g, c): keys 4 g .. 4 g + 3 of query c) is the B operand of O^T = V^T P^T once the keys of a 32-key block
 // take the order "4 g .. 4 g + 3 of both 16-key tiles" in lane group g. Keys go from memory straight into the A
 // fragments; values are transposed 8 x 8 in registers and pass through a wave-private LDS tile (dim row (i, dg) = dim 8 dg + i
-// at i VTI + 80 dg, 16 bytes per lane group in one of five slots turned by i: writes and reads spread over all banks), so the
+// at i VTI + 80 dg, 16 bytes per lane group in one of five slots turned by i: writes spread over all banks; a read's 16 lanes
+// take the slots of eight dims, 0 1 2 3 4 0 1 2 and, for the next dim group, 5 .. 9 5 6 7, so six of them wait for another), so the
 // loop has no barrier. Scores, exponentials, sums and outputs in FP32, the probabilities rounded to BF16 for the second
 // product, as in k_attn_part. The exponentials are expf there and here: 2^(d log2 e) on the hardware instruction, 3 % of the time
 // less (33.2 / 28.0 / 15.1 us at 968 / 800 / 400 tokens), is off by the rounded product, 2.6e-6 of a probability at d = 80.

@@ -202,7 +202,7 @@ __device__ __forceinline__ void st4(void* p, size_t i, int dt, const float (&v)[
     else *gptr((uint2_t*)((u16*)p + i)) = uint2_t{(u32)f32_to_f16(v[0]) | ((u32)f32_to_f16(v[1]) << 16), (u32)f32_to_f16(v[2]) | ((u32)f32_to_f16(v[3]) << 16)};
 }
 
-// the row of type DT into R: every load issued before the first use, then use(values, index) with load's words of each group
+// the row of type DT into R: every load issued before the first use
 template <int DT, int NW, int FM>
 __device__ __forceinline__ void load_row4(const Place<NW>& P, Row<FM>& R, const void* row) {
     constexpr int SZ = DT == TCQ_F32 || DT == TCQ_I32 ? 4 : 2;

@@ -262,7 +262,7 @@ class Group:
         if parts > 1:
             if M > SMALL_M:
                 if parts != self.epilogue_parts(M):
-                    raise ValueError(f'{parts} K parts are for at most {SMALL_M} tokens')
+                    raise ValueError(f'{M} tokens take {self.epilogue_parts(M)} K parts (epilogue_parts), got {parts}')
                 return kernels.gemm_i8_parts(q, self.dense(), parts)
             acc = torch.empty(parts, M, self.Ntot, dtype=torch.int32, device=dev)
             if self.W is not None:
@@ -323,9 +323,9 @@ class Group:
     def gated_down(self, b, down, parts=1, pro=None):
         """This gate | up group's product, the GeGLU middle and the down projection's product: (z, b2) with z as
         down.product(b2, parts) returns it and b2 the down input's buffers (its token scale for the epilogue). On the
-        spread middle at one token the down projection's rotate + quantize runs inside its product's launch (every
-        workgroup computes the INT8 row from glu_split's output); else gated_middle then down.product. pro: as in
-        gated_middle."""
+        spread middle at one token, weights decoded on the fly, the down projection's rotate + quantize runs inside its
+        product's launch (every workgroup computes the INT8 row from glu_split's output); else gated_middle then
+        down.product. pro: as in gated_middle."""
         M, dev = (1, self.rs.device) if pro is not None else (b['scale'].numel(), b['scale'].device)
         if self.W is None and self.spreads(M) and down.pre_prologue_fits(M):
             zt = torch.empty(2, M, 128, 128, dtype=torch.float32, device=dev)
@@ -611,8 +611,8 @@ class KDecoderLayer(torch.nn.Module):
         """Whether the o epilogue + residual + norm2 + rotate + quantize can run as the prologue of the gate | up product
         (tcq_gemm_tcq_pro): one token, int32 sums, a two-sided o projection without bias, 2048-wide rows, and a gate | up
         group decoded on the fly to the spread middle (256 workgroups, one per CU, each running the prologue once). On MI355X at
-        one token: fly 18.1 -> 17.2 us for the two launches' work; on the resident plan's 1024 workgroups the prologue
-        runs four times per CU and the pair gets slower (1.50 -> 1.72 ms per decode token), so it is not used there."""
+        one token: fly 18.1 -> 17.2 us for the two launches' work. Resident groups' tcq_gemm_w8_w128t takes no prologue; on
+        tcq_gemm_w8_pro, whose 1024 workgroups run it four times per CU, a decoded token took 1.72 ms instead of 1.50."""
         return (FUSE['prologue'] and z.dtype == torch.int32 and z.shape[-2] == 1 and og.bias is None and not og.one_sided
                 and og.Ntot == 2048 and gu.K == 2048 and gu.a8 and gu.W is None and gu.spreads(1))
 
