@@ -128,7 +128,7 @@ def test_bf16_sums_as_close_to_fp64_as_the_few_token_product(M, N, K):
 
 @pytest.mark.parametrize('M,N,K', [(300, 32768, 144), (330, 32768, 272), (960, 12288, 256)])
 def test_tiles_of_equal_estimates(M, N, K):
-    """Sizes whose estimate several tiles share: full rounds (the larger tile) and partly filled ones (the fullest)."""
+    """Sizes whose tiles lie close together: full rounds of several, and partly filled ones."""
     test_int8_tiles_bitexact(M, N, K)
     test_bf16_tiles_against_fp64(M, N, K)
 

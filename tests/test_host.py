@@ -200,8 +200,8 @@ def test_many_token_k_parts_rule():
     from yanlongvla_amd import kernels
     best = kernels.gemm_i8_best_parts
     assert [best(m, 2048, 16384) for m in (1, 64)] == [1, 1] and best(200, 2048, 1024) == 1
-    assert [best(m, 2048, 16384) for m in (200, 800, 968)] == [4, 2, 2]
-    assert [best(*s) for s in ((400, 1024, 4096), (968, 1024, 4096), (968, 2048, 2048), (968, 32768, 2048))] == [2, 1, 1, 1]
+    assert [best(m, 2048, 16384) for m in (200, 968)] == [4, 2] and best(65, 1024, 4096) == 4
+    assert [best(*s) for s in ((400, 1024, 4096), (968, 2048, 2048), (968, 32768, 2048))] == [2, 1, 1]
     bf16 = kernels._lib.lib().tcq_gemm_bf16_best_parts
     assert [bf16(*s) for s in ((64, 2048, 16384), (200, 2048, 512), (256, 2048, 16384), (968, 2048, 16384))] == [1, 1, 4, 4]
     assert [bf16(*s) for s in ((400, 2048, 2048), (968, 32768, 2048))] == [1, 1]

@@ -395,35 +395,41 @@ static void launch_gemm(int odt, hipStream_t st, const void* x, const void* w, c
     else launch_k(k_gemm_i8<ESZ, TN, TM, WN, WM, NSW, NSX, TCQ_BF16>, grid, block, lds, st, x, w, sa, sw, out, ldo, M, N, K, parts, flush);
 }
 
-// The tile with the least estimated time. Workgroups run in rounds of 256 (one per CU); c1 is what a step of one round
-// costs, c2 a step of two rounds (the tiles up to 128 x 128 fit two workgroups on a CU, which share its LDS and matrix
-// cores), later rounds as pairs. In units of 1/16 us per 128-byte step, fitted to INT8 runs over M = 80 .. 968 and N = 1024
-// .. 32768 on MI355X (us, K = 2048): 64 x 64 8.0 (256 workgroups) / 10.1 (512), 128 x 64 9.9 / 15.4, 128 x 128 13.4 / 24.6,
-// 256 x 128 19.4 / 44, 256 x 256 33 / 73. Of equal estimates the one whose rounds are fullest, and of those the larger tile, which
-// reads less: 300 x 32768 33.4 us on 256 x 256 against 39.5 on 128 x 128 and 49.5 on 128 x 64, all with full rounds; 700 x 12288 FP32 37.8,
-// 31.7 and 35.4 (144 workgroups of 256, 576 of 768, 1056 of 1280). Over 684 runs (19 weight shapes of K = 1024 .. 16384, M = 65 .. 968, int32
-// and FP32 out) the chosen tile was 2.4 % above the best of the five on average and more than 8 % above it in 74, most where a
-// last round is partly filled: 400 x 2560 x 2048 takes 128 x 64 at 9.5 us where 64 x 64 needs 8.3, 900 x 4608 x 1536 256 x 128 at 17.3 where
-// 128 x 128 needs 14.4. A short K pays the longer ramp of these tiles: with int32 out 700 .. 968 tokens x 2560 or 3072 x 1024 take 9.2 us,
-// 8.1 .. 8.8 with 64-byte steps and 32 x 32 blocks; from K = 1536 on that form is slower nearly everywhere, by up to a third.
-struct TileCost { int tn, tm, c1, c2; };
-constexpr TileCost TILES[5] = {{64, 64, 4, 7}, {128, 64, 6, 12}, {128, 128, 9, 20}, {256, 128, 16, 38}, {256, 256, 30, 68}};
-static int choose_tile(int M, int N, int parts, int tiles, long* cost = nullptr) {
+// The tile with the least estimated time. Workgroups run in rounds of 256 (one per CU; the tiles up to 128 x 128 fit two on a CU, so
+// several rounds overlap): a single round takes ramp + one x its 128-byte steps, each of several ramp + more x steps, in ns. The
+// constants are fitted to which tile was the fastest, and to the times, in 1304 INT8 and 1574 BF16 runs of every tile on MI355X (M = 65 ..
+// 2400, N = 256 .. 32768, K = 1024 .. 16384; int32 and FP32 out; BF16 in 1, 2 and 4 K parts). Over 954 and 1215 runs of other random
+// sizes the chosen tile was 0.6 % (INT8) and 0.9 % (BF16) above the best on average and more than 8 % above it in 23 and 51; one cost
+// per step whatever the K, from INT8 runs alone, was 2.6 % and 2.0 % above, more than 8 % in 65 and 88. us, that rule's tile / this one:
+// INT8 to FP32 400 x 2560 x 2048 11.1 / 9.4, 900 x 4608 x 1536 21.2 / 15.8, 700 x 12288 x 2048 37.2 / 32.0; BF16 600 x 16384 x 2048 60.0 / 52.3,
+// 1300 x 32768 x 2048 248 / 210. Most of what is left is a partly filled last round: BF16 800 x 32768 x 2048 takes 128 x 128 at 147 where
+// 256 x 128 in three rounds and a half needs 133. A short K pays the longer ramp of 128-byte steps: with int32 out 700 .. 968 tokens x 2560 or
+// 3072 x 1024 take 9.2 us, 8.1 .. 8.8 with 64-byte steps and 32 x 32 blocks; from K = 1536 on that form is slower nearly everywhere, by up
+// to a third. BF16 of 16384 columns and more pays its second level: one chain on 256 x 256 tiles took 968 x 32768 x 2048 in 136 us
+// where this takes 150, at 1.54e-7 from 64 bits instead of 5.6e-8.
+struct Tile { int tn, tm; double one, more, ramp; };
+constexpr Tile TILES_I8[] = {{64, 64, 389, 247, 1386}, {128, 64, 455, 409, 3420}, {128, 128, 623, 447, 2469}, {256, 128, 820, 722, 6128},
+                             {256, 256, 1113, 717, 12191}};
+constexpr Tile TILES_BF16[] = {{64, 64, 359, 223, 3642}, {128, 64, 402, 369, 5058}, {128, 128, 538, 489, 4597}, {256, 128, 591, 666, 15412}};
+template <int ESZ>
+static int choose_tile(int M, int N, int K, int parts, double* ns = nullptr) {
+    const Tile* T = ESZ == 1 ? TILES_I8 : TILES_BF16;           // BF16 keeps two levels of sums: no registers for 256 x 256
+    const int nk = (int)(((long)K * ESZ + 127) / 128), steps = (nk + parts - 1) / parts;
     int best = 0;
-    long bc = 0, bw = 0, br = 1;
-    for (int i = 0; i < tiles; ++i) {
-        const long w = (long)((N + TILES[i].tn - 1) / TILES[i].tn) * ((M + TILES[i].tm - 1) / TILES[i].tm) * parts, r = (w + 255) / 256;
-        const long c = r == 1 ? 2 * TILES[i].c1 : r * TILES[i].c2;
-        if (i == 0 || c < bc || (c == bc && w * br >= bw * r)) { best = i; bc = c; bw = w; br = r; }
+    double bt = 0;
+    for (int i = 0; i < (ESZ == 1 ? 5 : 4); ++i) {
+        const long w = (long)((N + T[i].tn - 1) / T[i].tn) * ((M + T[i].tm - 1) / T[i].tm) * parts, r = (w + 255) / 256;
+        const double t = r == 1 ? T[i].ramp + T[i].one * steps : r * (T[i].ramp + T[i].more * steps);
+        if (i == 0 || t < bt) { best = i; bt = t; }
     }
-    if (cost) *cost = bc;                               // a step's time in units of 1/32 us
+    if (ns) *ns = bt;
     return best;
 }
 
 template <int ESZ>
 static void launch_by_size(int odt, hipStream_t st, const void* x, const void* w, const float* sa, const float* sw, void* out, int ldo,
                            int M, int N, int K, int parts) {
-    switch (choose_tile(M, N, parts, ESZ == 1 ? 5 : 4)) {       // BF16 keeps two levels of sums: no registers for 256 x 256
+    switch (choose_tile<ESZ>(M, N, K, parts)) {
         case 0: launch_gemm<ESZ, 64, 64, 2, 2, 4, 4>(odt, st, x, w, sa, sw, out, ldo, M, N, K, parts); break;
         case 1: launch_gemm<ESZ, 128, 64, 4, 2, 3, 3>(odt, st, x, w, sa, sw, out, ldo, M, N, K, parts); break;
         case 2: launch_gemm<ESZ, 128, 128, 2, 4, 3, 2>(odt, st, x, w, sa, sw, out, ldo, M, N, K, parts); break;
@@ -460,21 +466,19 @@ extern "C" int tcq_gemm_i8_parts(const int8_t* a, const int8_t* w, int32_t* out,
     return launch_status();
 }
 
-// The K parts with the least estimated time: steps at choose_tile's cost, and for each part past the first its write and the
-// epilogue's read at 3 TB/s. A long K over few tiles leaves the large tiles too few workgroups and the small ones bound by
-// their loads into LDS; parts give the larger tiles the whole chip. MI355X, us with the epilogue in 1 / 2 / 4 parts, the
-// chosen one first: 968 x 2048 x 16384 49 (2) against 61 / 48.7, 800: 45.7 (2) against 56 / 44.4, 200: 23.5 (4) against 40 / 26;
-// 400 x 1024 x 4096 14.5 (2) against 17.5 / 15.8, 968 x 1024 x 4096 19.3 (1) against 18.8 / 20.9; 968 x 2048 x 2048 22.4 (1)
-// against 24.5 / 26.6.
+// The K parts with the least estimated time: choose_tile's, and for each part past the first its write and the epilogue's read
+// at 3 TB/s. A long K over few tiles leaves the large tiles too few workgroups and the small ones bound by their loads into
+// LDS; parts give the larger tiles the whole chip. MI355X, us with the epilogue in 1 / 2 / 4 parts: 968 x 2048 x 16384 65.4 / 53.1 /
+// 53.0 (2 taken), 200: 37.3 / 25.9 / 23.3 (4); 400 x 1024 x 4096 16.4 / 13.7 / 14.7 (2), 968: 19.6 / 19.4 / 21.3 (2); 968 x 2048 x 2048 23.4 /
+// 25.8 / 27.8 (1). Over 160 sizes (N = 1024 .. 8192, M = 65 .. 2000) the parts taken are 0.2 % above the best on average, 5 % at most.
 extern "C" int tcq_gemm_i8_best_parts(int M, int N, int K) {
     if (M <= 64 || N <= 0 || K < 128 * 16) return 1;
     int best = 1;
     double bt = 0;
     for (int parts = 1; parts <= 4; parts *= 2) {
-        long c = 0;
-        choose_tile(M, N, parts, 5, &c);
-        const int steps = (K + 127) / 128;
-        const double t = (steps + parts - 1) / parts * (c / 32.0) + (parts - 1) * (8.0 * M * N) / 3e6;
+        double t = 0;
+        choose_tile<1>(M, N, K, parts, &t);
+        t += (parts - 1) * (8.0 * M * N) / 3e3;
         if (parts == 1 || (t < bt && (size_t)parts * M * N < ((size_t)1 << 31))) { best = parts; bt = t; }
     }
     return best;
@@ -538,8 +542,8 @@ extern "C" int tcq_gemm_bf16_parts(const void* a, const void* w, const float* sw
     return launch_status();
 }
 
-// As tcq_gemm_i8_best_parts, with 2 us for the launch that adds the parts, and their write and read at 6 TB/s. MI355X, us in 1 / 2 /
-// 4 parts: 968 x 2048 x 16384 105 / 81 / 76, 256: 77 / 45 / 33; 128 x 1024 x 4096 23 / 16 / 12; 400 x 2048 x 2048 14.3 / 15.0 / 17.5.
+// As tcq_gemm_i8_best_parts, with 2 us for the launch that adds the parts, and their write and read at 4 TB/s (1.0 % above the best
+// parts and tile on average over 471 sizes). MI355X, us in 1 / 2 / 4 parts: 968 x 2048 x 16384 105 / 81 / 76, 256: 77 / 45 / 33; 128 x 1024 x 4096 23 / 16 / 12; 400 x 2048 x 2048 14.3 / 15.0 / 17.5.
 // Relative error against 64 bits, 968 x 2048 x 16384: 8.9e-8, 9.3e-8, 9.2e-8 (the few-token product's partial sums: 1.18e-7); 65 x 1024 x
 // 1024: 4.9e-8, 5.5e-8, 5.0e-8 (5.7e-8).
 extern "C" int tcq_gemm_bf16_best_parts(int M, int N, int K) {
@@ -547,10 +551,9 @@ extern "C" int tcq_gemm_bf16_best_parts(int M, int N, int K) {
     int best = 1;
     double bt = 0;
     for (int parts = 1; parts <= 4; parts *= 2) {
-        long c = 0;
-        choose_tile(M, N, parts, 4, &c);
-        const int steps = (K + 63) / 64;
-        const double t = (steps + parts - 1) / parts * (c / 32.0) + (parts > 1 ? 2 + parts * 8.0 * M * N / 6e6 : 0);
+        double t = 0;
+        choose_tile<2>(M, N, K, parts, &t);
+        t += parts > 1 ? 2e3 + parts * 8.0 * M * N / 4e3 : 0;
         if (parts == 1 || (t < bt && (size_t)parts * M * N < ((size_t)1 << 31))) { best = parts; bt = t; }
     }
     return best;
